@@ -1460,22 +1460,11 @@ static int transition_topk_forward_impl(const float* sender_strength, const floa
              "workspace too small: need %zu bytes, got %zu", s.bytes, workspace_bytes);
   const int B = (int)batch, Ns = (int)src_nodes, Nd = (int)dst_nodes, r = (int)rank;
 
-  // 1. projections P_s = src . Ws^T, P_t = dst . Wt^T  (modules.py:435-437), side by side
+  // 1. projections P_s = src . Ws^T, P_t = dst . Wt^T  (modules.py:435-437)
   const SideStream* side = side_stream_for(st, batch * src_nodes * k);
-  if (side) {
-    rc = fork_to(side, st);
-    if (rc) return rc;
-  }
-  rc = gemm_project(dst_val, dst_dim, target_weight, target_weight, r, dst_dim, dst_proj, r, B * Nd, r, (int)dst_dim,
-                    side ? side->stream : st, bf16);
+  rc = gemm_project_two(src_val, source_weight, src_proj, B * Ns, (int)src_dim, dst_val, target_weight, dst_proj,
+                        B * Nd, (int)dst_dim, r, st, side, bf16);
   if (rc) return rc;
-  rc = gemm_project(src_val, src_dim, source_weight, source_weight, r, src_dim, src_proj, r, B * Ns, r, (int)src_dim,
-                    st, bf16);
-  if (rc) return rc;
-  if (side) {
-    rc = join_from(side, st);
-    if (rc) return rc;
-  }
 
   // 2. per-source edge list: logits ((P_s * w) . P_t + b) / T, top-k over destinations
   if (k < dst_nodes) {
@@ -2336,11 +2325,8 @@ static int transition_dense_forward_impl(const float* sender_strength, const flo
   const int B = (int)batch, Ns = (int)src_nodes, Nd = (int)dst_nodes, r = (int)rank, Dv = (int)val_dim;
 
   // 1. projections P_s = src . Ws^T, P_t = dst . Wt^T  (modules.py:435-437)
-  rc = gemm_project(src_val, src_dim, source_weight, source_weight, r, src_dim, src_proj, r, B * Ns, r, (int)src_dim,
-                    st, bf16);
-  if (rc) return rc;
-  rc = gemm_project(dst_val, dst_dim, target_weight, target_weight, r, dst_dim, dst_proj, r, B * Nd, r, (int)dst_dim,
-                    st, bf16);
+  rc = gemm_project_two(src_val, source_weight, src_proj, B * Ns, (int)src_dim, dst_val, target_weight, dst_proj,
+                        B * Nd, (int)dst_dim, r, st, nullptr, bf16);
   if (rc) return rc;
   // 2. raw logits L_b = (P_s diag(w)) P_t^T; with heads, max_h of each head's
   //    logits plus its bias (one GEMM per head, folded in the epilogue)

@@ -376,6 +376,20 @@ __device__ __forceinline__ void store_pack(T* p, const Pack<W>& x) {
   }
 }
 
+// The exact three-term bf16 split of an fp32 value: x = h + m + l, each a bf16
+// value in the high half of its word (truncations, and the last remainder).
+__device__ __forceinline__ void x3_split(uint32_t u, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = u & 0xFFFF0000u;
+  const float r = __uint_as_float(u) - __uint_as_float(h);
+  m = __float_as_uint(r) & 0xFFFF0000u;
+  l = __float_as_uint(r - __uint_as_float(m));
+}
+
+// the bf16 values in the high halves of two words as one bf16x2 word (first in the low half)
+__device__ __forceinline__ uint32_t x3_pair(uint32_t first, uint32_t second) {
+  return __builtin_amdgcn_perm(second, first, 0x07060302u);  // bytes 2, 3 of first, then of second
+}
+
 // Streaming accesses (data read or written once): non-temporal, so they do
 // not displace data that is reused (gathered rows, GEMM operands) from L2.
 typedef unsigned int u32x4_nt __attribute__((ext_vector_type(4)));

@@ -1290,18 +1290,6 @@ constexpr int kX3K = 32;                 // K per slice
 constexpr int kX3S = kX3K + 8;           // LDS row stride in bf16 elements (80 bytes: conflict-free fragments)
 constexpr int kX3Plane = kBfT * kX3S;    // one plane of one operand
 
-__device__ __forceinline__ void x3_split(uint32_t u, uint32_t& h, uint32_t& m, uint32_t& l) {
-  h = u & 0xFFFF0000u;
-  const float r = __uint_as_float(u) - __uint_as_float(h);
-  m = __float_as_uint(r) & 0xFFFF0000u;
-  l = __float_as_uint(r - __uint_as_float(m));
-}
-
-// the bf16 values in the high halves of two words as one bf16x2 word (first in the low half)
-__device__ __forceinline__ uint32_t x3_pair(uint32_t first, uint32_t second) {
-  return __builtin_amdgcn_perm(second, first, 0x07060302u);  // bytes 2, 3 of first, then of second
-}
-
 // Operand loader of one slice: 128 rows (m or n) x 32 k of fp32 into the three
 // LDS planes [row][k].  KC: rows with k contiguous (row stride ld); else k rows
 // of stride ld.  `base` addresses the slice's (row 0, k 0).
@@ -1597,6 +1585,29 @@ static bool fast_path_ok(const GemmArgs& g, bool a_kc, bool b_kc) {
   return f4_aligned(g.A) && f4_aligned(g.B0) && f4_aligned(g.B1) && f4_aligned(g.a_kscale);
 }
 
+// 128 x 128 tiles halve the operand traffic per flop; 64 x 64 when an extent
+// is too small to fill them or the grid would be too small.  (The 128 x 128
+// kernel applies the k scale of a scaled use unconditionally.)
+static bool fast_choice(const GemmArgs& g, GemmUse use, int64_t zdim, int forced) {
+  const GemmUseInfo& info = kGemmUses[use];
+  const int64_t tiles128 = (int64_t)((g.M + kFT - 1) / kFT) * ((g.N + kFT - 1) / kFT) * zdim;
+  const bool big = forced ? forced == kFT : (g.M >= kFT && g.N >= kFT && tiles128 >= 256);
+  return big && tiles128 < (1LL << 31) && fast_path_ok(g, info.a_kc, info.b_kc) &&
+         (!info.a_kscale || g.a_kscale != nullptr);
+}
+
+// The rows kernel's form of a projection (use kGemmProject or
+// kGemmProjectBf16) when it takes it: its arithmetic is that of the kernel
+// chosen otherwise, so it must not stand in for gemm_f32_fast_kernel (`fast`).
+static bool rows_form(const GemmArgs& g, int use, bool fast, RowsGemm& r) {
+  const bool bf = use == kGemmProjectBf16;
+  r = RowsGemm{g.A, g.lda, g.B0, g.B1, g.b_split, g.ldb, g.C, g.ldc, g.M, g.N, g.K, 0};
+  if (bf ? bf16_path_ok(g, use, 1) : x3_path_ok(g, use, 1)) r.arith = bf ? kRowsBf : kRowsX3;
+  else if (!fast) r.arith = bf ? kRowsC4Bf : kRowsC4;
+  else return false;
+  return gemm_rows_fits(r);
+}
+
 int launch_gemm(const GemmArgs& g, GemmUse use, int splits, hipStream_t stream) {
   JN_REQUIRE(g.M >= 0 && g.N >= 0 && g.K >= 0, kInvalidArgument, "negative GEMM extent");
   if (g.M == 0 || g.N == 0) return kOk;
@@ -1609,19 +1620,17 @@ int launch_gemm(const GemmArgs& g, GemmUse use, int splits, hipStream_t stream) 
              "GEMM use %s takes one B buffer", info.name);
   const int64_t zdim = g.batch > 1 ? g.batch : splits;
   JN_REQUIRE((g.M + kGBM - 1) / kGBM < 65536, kUnsupported, "GEMM M extent too large");
-  // 128 x 128 tiles halve the operand traffic per flop; 64 x 64 when an
-  // extent is too small to fill them or the grid would be too small
-  const int64_t tiles128 = (int64_t)((g.M + kFT - 1) / kFT) * ((g.N + kFT - 1) / kFT) * zdim;
   const int forced = g_gemm_tile.load(std::memory_order_relaxed);
-  const bool big = forced ? forced == kFT : (g.M >= kFT && g.N >= kFT && tiles128 >= 256);
-  // (the 128 x 128 kernel applies the k scale of a scaled use unconditionally)
-  const bool fast = big && tiles128 < (1LL << 31) && fast_path_ok(g, info.a_kc, info.b_kc) &&
-                    (!info.a_kscale || g.a_kscale != nullptr);
+  const bool fast = fast_choice(g, use, zdim, forced);
   // 32 x 32 tiles for the projection uses when a 64 x 64 grid would not reach
   // one workgroup per CU
   const int64_t tiles64 = (int64_t)((g.M + kGBM - 1) / kGBM) * ((g.N + kGBM - 1) / kGBM) * zdim;
   const bool small = !fast && gemm_use_small_tile(use) && (g.M + 31) / 32 < 65536 &&
                      (forced ? forced == 32 : tiles64 < 256);
+  if ((use == kGemmProject || use == kGemmProjectBf16) && forced == 0) {
+    RowsGemm r;
+    if (rows_form(g, use, fast, r)) return launch_gemm_rows(&r, 1, stream);
+  }
   if (gemm_use_dense_bf16(use)) {
     JN_REQUIRE(bf16_path_ok(g, use, splits), kUnsupported,
                "%s needs M, N >= 128, N and the strides multiples of 8 and 16-byte aligned operands", info.name);
@@ -1782,17 +1791,41 @@ int gemm_batched(const BatchedGemm& m, GemmUse use, hipStream_t stream) {
   return launch_gemm(g, use, 1, stream);
 }
 
-// C[M][N] = X[M][K] . [W0;W1]^T with W0 rows [0, split) and W1 rows [split, N).
-// x_bf16: X holds bf16 elements.
-int gemm_project(const float* X, int64_t ldx, const float* W0, const float* W1, int split, int64_t ldw, float* C,
-                 int64_t ldc, int M, int N, int K, hipStream_t stream, bool x_bf16) {
+static GemmArgs project_args(const float* X, int64_t ldx, const float* W0, const float* W1, int split, int64_t ldw,
+                             float* C, int64_t ldc, int M, int N, int K) {
   GemmArgs g{};
   g.A = X; g.lda = ldx;
   g.B0 = W0; g.B1 = W1; g.ldb = ldw; g.b_split = split;
   g.C = C; g.ldc = ldc;
   g.M = M; g.N = N; g.K = K;
   g.k_chunk = K; g.c_split_stride = 0;
-  return launch_gemm(g, x_bf16 ? kGemmProjectBf16 : kGemmProject, 1, stream);
+  return g;
+}
+
+// C[M][N] = X[M][K] . [W0;W1]^T with W0 rows [0, split) and W1 rows [split, N).
+// x_bf16: X holds bf16 elements.
+int gemm_project(const float* X, int64_t ldx, const float* W0, const float* W1, int split, int64_t ldw, float* C,
+                 int64_t ldc, int M, int N, int K, hipStream_t stream, bool x_bf16) {
+  return launch_gemm(project_args(X, ldx, W0, W1, split, ldw, C, ldc, M, N, K),
+                     x_bf16 ? kGemmProjectBf16 : kGemmProject, 1, stream);
+}
+
+int gemm_project_two(const float* X0, const float* W0, float* C0, int M0, int K0, const float* X1, const float* W1,
+                     float* C1, int M1, int K1, int r, hipStream_t stream, const SideStream* side,
+                     bool x_bf16) {
+  const GemmUse use = x_bf16 ? kGemmProjectBf16 : kGemmProject;
+  const GemmArgs g[2] = {project_args(X0, K0, W0, W0, r, K0, C0, r, M0, r, K0),
+                         project_args(X1, K1, W1, W1, r, K1, C1, r, M1, r, K1)};
+  RowsGemm p[2];
+  if (g_gemm_tile.load(std::memory_order_relaxed) == 0 && rows_form(g[0], use, fast_choice(g[0], use, 1, 0), p[0]) &&
+      rows_form(g[1], use, fast_choice(g[1], use, 1, 0), p[1]) && p[0].arith == p[1].arith)
+    return launch_gemm_rows(p, 2, stream);
+  int rc;
+  if (side && (rc = fork_to(side, stream))) return rc;
+  rc = launch_gemm(g[1], use, 1, side ? side->stream : stream);
+  if (!rc) rc = launch_gemm(g[0], use, 1, stream);
+  if (rc) return rc;
+  return side ? join_from(side, stream) : kOk;
 }
 
 // dX[M][N] = dP[M][K] . [W0;W1] (+ addend), W0 rows [0, split) of K.

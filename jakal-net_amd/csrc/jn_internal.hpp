@@ -83,9 +83,36 @@ constexpr int kRegRank = 128;
 constexpr int kMaxRank = 1024;
 
 // ---- fp32 MFMA GEMMs (jn_gemm.hip) ----------------------------------------
+// Projections of few rows (jn_gemm_rows.hip): C[M][N] = X[M][K] . [W0; W1]^T,
+// W0 holding weight rows [0, split).
+struct RowsGemm {
+  const void* X;
+  int64_t ldx;
+  const float* W0;
+  const float* W1;
+  int split;
+  int64_t ldw;
+  float* C;
+  int64_t ldc;
+  int M, N, K;
+  int arith;  // kRows*: the tile kernel whose arithmetic it follows
+};
+constexpr int kRowsX3 = 0, kRowsC4 = 1, kRowsBf = 2, kRowsC4Bf = 3;
+constexpr int kRowsMaxM = 32768, kRowsMaxN = 1024;
+bool gemm_rows_fits(const RowsGemm& g);
+// One launch over one or two products (of one arithmetic).
+int launch_gemm_rows(const RowsGemm* p, int n, hipStream_t stream);
+
 // x_bf16: the layer operand X (and dX with its addend) holds bf16 elements.
 int gemm_project(const float* X, int64_t ldx, const float* W0, const float* W1, int split, int64_t ldw, float* C,
                  int64_t ldc, int M, int N, int K, hipStream_t stream, bool x_bf16 = false);
+// Two projections of their own weights, rank r each: in one launch where both
+// run on the rows kernel in one arithmetic, else side by side (side: a second
+// stream, or null) or one after the other.
+struct SideStream;
+int gemm_project_two(const float* X0, const float* W0, float* C0, int M0, int K0, const float* X1, const float* W1,
+                     float* C1, int M1, int K1, int r, hipStream_t stream, const SideStream* side,
+                     bool x_bf16 = false);
 int gemm_grad_input(const float* dP, int64_t ldp, const float* W0, const float* W1, int split, int64_t ldw,
                     const float* addend, int64_t ld_add, float* dX, int64_t ldx, int M, int N, int K,
                     hipStream_t stream, bool x_bf16 = false);

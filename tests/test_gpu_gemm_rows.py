@@ -1,0 +1,74 @@
+"""The few-rows projection kernel on its edges: partial row and column tiles,
+partial K slices, weight rows split over two buffers off every tile, and each
+tile choice (by row count), fp32 and bf16.
+
+Bound: a projection is one fp32 sum of K products (exact for bf16 operands, one
+rounding each for fp32) in partial sums, so an element is off from float64 by
+at most (K + 8) 2^-24 sum |x w|.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _project(dev, M, r, K, bf16):
+    """projections [M, 2r] of a window forward (one node per batch element) with its operands."""
+    import jakal_net_native as jn
+
+    g = torch.Generator().manual_seed(M * 131 + r * 17 + K)
+    X = torch.randn(M, 1, K, generator=g).to(dev, torch.bfloat16 if bf16 else torch.float32)
+    U, V = (torch.randn(r, K, generator=g).to(dev) for _ in range(2))
+    ps, w = torch.randn(M, 1, generator=g).to(dev), torch.ones(r, device=dev)
+    ds, proj = torch.empty(M, 1, device=dev), torch.full((M, 2 * r), float("nan"), device=dev)
+    dv, idx = torch.empty_like(X), torch.empty(M, 1, 1, device=dev, dtype=torch.int32)
+    score = torch.empty(M, 1, 1, device=dev)
+    fn = jn._LIB.jn_propagation_window_forward_bf16 if bf16 else jn._LIB.jn_propagation_window_forward
+    p = jn._ptr
+    jn._check(fn(p(X), p(ps), p(X), p(U), p(V), p(w), None, M, 1, K, K, r, 0, 0, p(ds), p(dv), p(proj), p(idx),
+                 p(score), jn._stream(dev)))
+    torch.cuda.synchronize()
+    return X[:, 0].double(), U, V, proj
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("M,r,K", [
+    (1, 1, 8), (16, 8, 32), (17, 9, 40), (33, 32, 520), (1500, 33, 64), (1537, 64, 72), (3100, 24, 200),
+    (4111, 64, 96), (8209, 64, 136), (8209, 20, 24), (16384, 64, 64), (16385, 64, 64), (32768, 16, 32),
+    (40, 130, 264),
+])
+def test_projection_edges(M, r, K, bf16):
+    dev = torch.device("cuda:0")
+    X, U, V, proj = _project(dev, M, r, K, bf16)
+    W = torch.cat([U, V])
+    W = (W.bfloat16() if bf16 else W).double()
+    want, scale = X @ W.t(), X.abs() @ W.abs().t()
+    assert ((proj.double() - want).abs() <= (K + 8) * 2.0 ** -24 * scale).all()
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("Ns,Nd,r", [(100, 37, 24), (37, 300, 64), (520, 16, 8)])
+def test_two_projections_in_one_launch(Ns, Nd, r, bf16):
+    """A transition's source and destination projections, of unequal rows and widths, against torch."""
+    import jakal_net as J
+
+    dev, B, Ds, Dd = torch.device("cuda:0"), 3, 72, 136
+    g = torch.Generator().manual_seed(Ns + Nd)
+    route = J.LowRankBilinearRoute(Ds, Dd, rank=r).to(dev)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    a, b = (torch.randn(B, n, d, generator=g).to(dev, dt) for n, d in ((Ns, Ds), (Nd, Dd)))
+    val_proj = lambda v: v[..., :1].expand(*v.shape[:-1], Dd)  # noqa: E731
+    op = J.SparseTransition(route, topk=Nd, val_proj_fn=val_proj, implementation="native")
+    src = J.Layer(Ds, Ns, torch.randn(B, Ns, generator=g).to(dev, dt), a)
+    dst = J.Layer(Dd, Nd, torch.zeros(B, Nd, device=dev, dtype=dt), b)
+    with torch.no_grad():
+        got = op.compute_delta(src, dst)
+        if bf16:
+            for p in (route.source_proj.weight, route.target_proj.weight):
+                p.copy_(p.bfloat16())
+        f = lambda layer: J.Layer(layer.dim, layer.num_nodes, layer.state.double(), layer.val.double())  # noqa: E731
+        op.double().implementation = "reference"
+        want = op.compute_delta(f(src), f(dst))
+    tol = 2e-2 if bf16 else 1e-5
+    assert (got.delta_val.double() - want.delta_val).norm() <= tol * want.delta_val.norm()
