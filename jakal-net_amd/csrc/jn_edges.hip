@@ -916,6 +916,151 @@ __global__ __launch_bounds__(256) void csr_fill_kernel(CsrArgs a, int tile_rows,
   if (t == 0 && tid == 0) seg[a.Nk] = carry;
 }
 
+// ---- the grouping of small edge lists in one launch ---------------------------
+// A workgroup of 16 waves owns `kg` (at most 64) consecutive keys of one batch
+// element and reads all of the element's edge index, each wave a consecutive
+// part of it held in registers (EPT loads per lane, all in flight together).
+// It counts its keys' edges per wave (LDS counters) and the edges into lower
+// keys, which gives its segment starts without any other workgroup's counts;
+// then each wave lists its edges in order and takes them 64 at a time: the
+// lanes that hold one key (six ballots, whatever the keys: top-k lists have
+// hubs that many rows choose) take consecutive slots at the key's cursor.
+// Same segments and records as the three launches above.
+//
+// Bound: latency (one read of the index, two barriers).  It replaces three
+// dependent launches whose work is a few microseconds each: with the events'
+// own 5 us per launch 6.3 + 6.2 + 11.5 -> 7.2 us at 16 x 256 rows of 16 edges,
+// 7.7 + 6.4 + 12.6 -> 8.4 at 8 x 1024 (256) rows of 16.  The index is read
+// ceil(Nk / kg) times per element, from L2, and a workgroup with hubs (keys
+// that many rows choose) takes them in one wave's steps, so it serves lists of
+// up to kCsrGroupEdges edges per element (20,000 edges on 1531 keys: 21.6 us
+// against 27 in three launches, 17 against 12 without the events).  k_inv: ceil(2^32 / k), so that the high
+// word of e * k_inv is e / k (exact while e k < 2^32; k > 1).
+constexpr int kCsrGroupWaves = 16;
+constexpr int kCsrGroupEdges = 16 * 64 * kCsrGroupWaves;  // 16 edges per lane at most
+
+template <int EPT>
+__global__ __launch_bounds__(64 * kCsrGroupWaves) void csr_group_kernel(CsrArgs a, int kg, uint32_t k_inv) {
+  __shared__ int cnt[kCsrGroupWaves][kWave];  // a wave's edges per key, then the prefix over the waves
+  __shared__ int below[kCsrGroupWaves];       // its edges into lower keys
+  __shared__ int start[kWave];
+  constexpr int BATCH = EPT < 8 ? EPT : 8;
+  __shared__ uint32_t list[kCsrGroupWaves][BATCH * kWave];  // a part's edges: offset in the wave's part, key
+  const int lane = lane_id(), wave = wave_id();
+  const int b = blockIdx.y, j0 = blockIdx.x * kg, ng = min(kg, a.Nk - j0);
+  const int E = a.Nq * a.k, per = EPT * kWave;
+  const int64_t batch_base = (int64_t)b * E;
+  const int32_t* idx = a.idx + batch_base;
+
+  int rel[EPT];  // key - j0, or a value outside [0, ng)
+  const int e0 = wave * per + lane;
+#pragma unroll
+  for (int u = 0; u < EPT; ++u) rel[u] = e0 + u * kWave < E ? idx[e0 + u * kWave] : -1;
+  cnt[wave][lane] = 0;
+  wave_lds_sync();
+  int lower = 0;
+#pragma unroll
+  for (int u = 0; u < EPT; ++u) {
+    const int j = rel[u];
+    if (j >= 0 && j < j0) ++lower;
+    rel[u] = j >= j0 && j < j0 + ng ? j - j0 : -1;
+    if (rel[u] >= 0) atomicAdd(&cnt[wave][rel[u]], 1);
+  }
+  lower = wave_reduce_i(lower, [](int x, int y) { return x + y; });
+  if (lane == 0) below[wave] = lower;
+  __syncthreads();
+  if (wave == 0) {
+    int deg = 0, first = 0;
+#pragma unroll
+    for (int w = 0; w < kCsrGroupWaves; ++w) {
+      const int c = cnt[w][lane];
+      cnt[w][lane] = deg;
+      deg += c;
+      first += below[w];
+    }
+    int incl = deg;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int y = __builtin_amdgcn_ds_bpermute(((lane - o) & 63) << 2, incl);
+      if (lane >= o) incl += y;
+    }
+    int32_t* seg = a.seg_start + (int64_t)b * (a.Nk + 1);
+    start[lane] = first + incl - deg;
+    if (lane < ng) seg[j0 + lane] = first + incl - deg;
+    if (j0 + ng == a.Nk && lane == ng - 1) seg[a.Nk] = first + incl;
+  }
+  __syncthreads();
+  int* cursor = cnt[wave];  // of this wave: the next slot of each key
+  cursor[lane] += start[lane];
+  uint32_t* mine = list[wave];
+  const uint64_t lower_lanes = (1ULL << lane) - 1;
+#pragma unroll
+  for (int u0 = 0; u0 < EPT; u0 += BATCH) {
+    // this part's edges of the group, in order
+    int n = 0;
+#pragma unroll
+    for (int u = u0; u < u0 + BATCH; ++u) {
+      const uint64_t m = __ballot(rel[u] >= 0);
+      if (rel[u] >= 0) mine[n + __popcll(m & lower_lanes)] = (uint32_t)((u * kWave + lane) << 6 | rel[u]);
+      n += __popcll(m);
+    }
+    wave_lds_sync();
+    for (int c = 0; c < n; c += kWave) {
+      const bool in = c + lane < n;
+      const uint32_t x = in ? mine[c + lane] : 0u;
+      const int key = (int)(x & 63u);
+      const int e = wave * per + (int)(x >> 6);
+      const int row = a.k > 1 ? (int)__umulhi((uint32_t)e, k_inv) : e;
+      const int64_t eid = batch_base + e;
+      float cf = 0.f, gs = 0.f, gd = 0.f;
+      int hd = 0;
+      if (in) {
+        cf = a.coef ? a.coef[eid] : (a.score ? a.score[eid] : 0.f);
+        if (a.rec_eid) gs = __int_as_float((int)eid);
+        else if (a.g_score) gs = a.g_score[eid];
+        if (a.gds) gd = a.gds[(int64_t)b * a.Nq + row];
+        if (a.ehead) hd = (int)a.ehead[eid];
+      }
+      // the lanes of the same key: agreement in every bit of it
+      uint64_t same = __ballot(in);
+#pragma unroll
+      for (int bit = 0; bit < 6; ++bit) {
+        const uint64_t set = __ballot((key >> bit) & 1);
+        same &= (key >> bit) & 1 ? set : ~set;
+      }
+      int pos = 0;
+      if (in) pos = cursor[key] + __popcll(same & lower_lanes);
+      wave_lds_sync();
+      if (in && (same & lower_lanes) == 0) cursor[key] += __popcll(same);
+      wave_lds_sync();
+      if (in) {
+        if (!a.coef && a.score) cf = softsign_f(cf);
+        a.rec[batch_base + pos] = make_float4(__int_as_float((b * a.Nq + row) | (hd << kRecHeadShift)), cf, gs,
+                                              a.gds ? cf * gd : 0.f);
+        if (a.pos) a.pos[eid] = (int32_t)(batch_base + pos);
+      }
+    }
+    wave_lds_sync();  // the list is read before the next part replaces it
+  }
+}
+
+static bool csr_group_fits(const CsrArgs& a) { return (int64_t)a.Nq * a.k <= kCsrGroupEdges && a.B < 65536; }
+
+static int launch_csr_group(const CsrArgs& a, hipStream_t stream) {
+  // about a workgroup per CU, 4 to 64 keys each
+  const int kg = (int)std::min<int64_t>(kWave, std::max<int64_t>(4, ((int64_t)a.B * a.Nk + 255) / 256));
+  const dim3 grid((a.Nk + kg - 1) / kg, a.B), block(64 * kCsrGroupWaves);
+  const int ept = (a.Nq * a.k + 64 * kCsrGroupWaves - 1) / (64 * kCsrGroupWaves);
+  const uint32_t k_inv = (uint32_t)(((1ULL << 32) + a.k - 1) / a.k);
+  JN_PROFILE("csr_group_kernel", stream);
+  if (ept <= 2) hipLaunchKernelGGL(csr_group_kernel<2>, grid, block, 0, stream, a, kg, k_inv);
+  else if (ept <= 4) hipLaunchKernelGGL(csr_group_kernel<4>, grid, block, 0, stream, a, kg, k_inv);
+  else if (ept <= 8) hipLaunchKernelGGL(csr_group_kernel<8>, grid, block, 0, stream, a, kg, k_inv);
+  else hipLaunchKernelGGL(csr_group_kernel<16>, grid, block, 0, stream, a, kg, k_inv);
+  JN_LAUNCH_CHECK();
+  return kOk;
+}
+
 int launch_csr(const CsrArgs& a, hipStream_t stream) {
   int rc = launch_csr_layout(a, stream);
   if (rc) return rc;
@@ -929,6 +1074,7 @@ int launch_csr_layout(const CsrArgs& a, hipStream_t stream) {
   JN_REQUIRE(csr_table_fits(a.B, a.Nq, a.Nk), kUnsupported,
              "edge grouping table of %lld tiles x %d keys exceeds %lld entries", (long long)a.B * csr_tiles(a),
              a.Nk, (long long)kCsrMaxTableEntries);
+  if (csr_group_fits(a)) return kOk;  // launch_csr_fill groups the edges by itself
   dim3 g2(csr_tiles(a), a.B);
   {
     JN_PROFILE("csr_count_kernel", stream);
@@ -947,6 +1093,7 @@ int launch_csr_fill(const CsrArgs& a, hipStream_t stream) {
   JN_REQUIRE(!a.score || a.compress == 0, kInvalidArgument, "records take inline coefficients for softsign only");
   JN_REQUIRE(a.k >= 1 && a.k <= 256 * kCsrFillEpt, kUnsupported, "edge grouping takes up to %d edges per row",
              256 * kCsrFillEpt);
+  if (csr_group_fits(a)) return launch_csr_group(a, stream);
   const int chunk_rows = std::max(1, std::min(kCsrChunkRows, 256 * kCsrFillEpt / a.k));
   dim3 g2(csr_tiles(a), a.B);
   const size_t lds = (size_t)min(a.Nk, kCsrFillSlice) * 3 * sizeof(uint32_t);

@@ -151,3 +151,52 @@ def test_edge_layout_is_the_stable_key_sort(dev, B, N, k):
         want_pos = np.empty(N * k, np.int64)
         want_pos[order] = base + np.arange(N * k)
         assert (pos[base: base + N * k] == want_pos).all()
+
+
+@pytest.mark.parametrize("B,N,k,heads", [
+    (1, 2, 1, 1), (2, 70, 7, 1), (17, 64, 4, 2), (3, 500, 32, 1), (1, 4000, 4, 1), (5, 129, 64, 1), (2, 5, 3, 1),
+    (2, 1024, 16, 1),   # 16,384 edges per element: the largest grouped in one launch
+    (2, 1025, 16, 1),   # above: count, prefix and fill
+])
+def test_grouping_is_a_stable_sort(dev, B, N, k, heads):
+    """Segments, records and record indices of the layout against a stable sort of each element's edges by key."""
+    import numpy as np
+    import jakal_net_native as jn
+
+    g = torch.Generator().manual_seed(N * 7 + k)
+    D, r = 16, 8
+    X = torch.randn(B, N, D, generator=g).to(dev).requires_grad_(True)
+    shape = (heads, r, D) if heads > 1 else (r, D)
+    U, V = (torch.randn(shape, generator=g).to(dev) for _ in range(2))
+    w = torch.ones(shape[:-1], device=dev) / r ** 0.5
+    kind = "multihead_max_low_rank_bilinear" if heads > 1 else "low_rank_bilinear"
+    out = jn.propagation_topk_selection(kind, w, None, V, None, U, None, "softsign", X,
+                                        torch.randn(B, N, generator=g).to(dev), X, k, 128, 128)
+    fn = out[1].grad_fn
+    while not hasattr(fn, "edge_layout"):
+        fn = fn.next_functions[0][0]
+    torch.cuda.synchronize()
+    raw = fn.edge_layout.cpu().numpy().tobytes()
+    head = fn.saved_tensors[9] if heads > 1 else None
+    head = head.cpu().numpy().reshape(B, -1) if heads > 1 else np.zeros((B, N * k), np.int64)
+    idx, score = out[2].cpu().numpy().reshape(B, -1), out[3].detach().cpu().numpy().reshape(B, -1)
+    at = 0
+
+    def take(count, dtype):
+        nonlocal at
+        a = np.frombuffer(raw, dtype, count, at)
+        at += (a.nbytes + 255) // 256 * 256
+        return a
+
+    seg = take(B * (N + 1), np.int32).reshape(B, N + 1)
+    rec = take(B * N * k * 4, np.int32).reshape(B, N * k, 4)
+    pos = take(B * N * k, np.int32).reshape(B, -1)
+    for b in range(B):
+        order = np.argsort(idx[b], kind="stable")
+        np.testing.assert_array_equal(seg[b], np.searchsorted(idx[b][order], np.arange(N + 1)))
+        np.testing.assert_array_equal(rec[b, :, 0] & ((1 << 27) - 1), b * N + order // k)
+        np.testing.assert_array_equal(rec[b, :, 0] >> 27, head[b][order])
+        np.testing.assert_array_equal(rec[b, :, 2], b * N * k + order)
+        s = score[b][order]
+        np.testing.assert_allclose(rec[b, :, 1].copy().view(np.float32), s / (1 + np.abs(s)), rtol=1e-6)
+        np.testing.assert_array_equal(pos[b][order], b * N * k + np.arange(N * k))
