@@ -34,7 +34,7 @@ def _node_axes(state: Tensor, val: Tensor, owner: str) -> tuple[int, int]:
         raise ValueError(f"{owner}: the state tensor has no node axis (a 0-d tensor was given).")
     if val.dim() < 2:
         raise ValueError(f"{owner}: the value tensor needs [..., nodes, dim] axes, got shape {tuple(val.shape)}.")
-    if tuple(val.shape[:-1]) != tuple(state.shape):
+    if val.shape[:-1] != state.shape:
         raise ValueError(
             f"{owner}: a value tensor of shape {tuple(val.shape)} does not pair with a state tensor of shape "
             f"{tuple(state.shape)} (values add one trailing axis to the state's shape)."
@@ -137,7 +137,7 @@ def finish_layer(layer: Layer, layer_fn: Callable[[Layer], Layer] | None) -> Lay
 
 def expect_shape(tensor: Tensor, shape: tuple[int, ...] | torch.Size, produced_by: str) -> None:
     """ValueError naming the callable that produced ``tensor`` when its shape is not ``shape``."""
-    if tuple(tensor.shape) != tuple(shape):
+    if tensor.shape != shape and tuple(tensor.shape) != tuple(shape):
         raise ValueError(f"{produced_by} produced a tensor of shape {tuple(tensor.shape)}; expected {tuple(shape)}.")
 
 

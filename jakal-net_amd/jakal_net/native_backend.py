@@ -28,7 +28,6 @@ from jakal_net.core import LayerDelta
 from jakal_net.kernel_common import (
     pairwise_kernel_spec,
     pairwise_route_kernel_spec,
-    supports_pairwise_kernel,
     supports_pairwise_route_kernel,
 )
 
@@ -101,12 +100,12 @@ class _NativeLoader:
         )
 
     def load(self, force_reload: bool = False) -> NativeStatus:
-        name = _module_name()
         if native_disabled_by_env():  # the switch wins over a module already loaded
             self.module = None
-            self.status = NativeStatus(False, name, None, (), (),
+            self.status = NativeStatus(False, _module_name(), None, (), (),
                                        f"native backend switched off by {DISABLE_NATIVE_ENV}")
         elif self.status is None or force_reload:
+            name = _module_name()
             try:
                 module = self._locate(name)
             except Exception as exc:  # noqa: BLE001
@@ -136,6 +135,12 @@ def native_supports(op_name: str) -> bool:
 def native_supports_device(device_type: str) -> bool:
     status = native_status()
     return status.available and device_type in status.supported_devices
+
+
+def native_runs(op_name: str, device_type: str) -> bool:
+    """Whether the native module takes this op on this device type."""
+    status = native_status()
+    return status.available and op_name in status.supported_ops and device_type in status.supported_devices
 
 
 def require_native_for_device(op_name: str, device_type: str) -> None:
@@ -170,6 +175,16 @@ def _as_layer_delta(result: Any) -> LayerDelta:
                     f"(delta_state, delta_val) pair")
 
 
+def _pairwise_spec(pairwise_fn: object, module: Any) -> Any:
+    """The kernel arguments of a score module; the core weight goes to a module
+    with a raw_scale (or unit_scale) op as it is, for the op to normalise."""
+    scale = getattr(module, "raw_scale", None) or getattr(module, "unit_scale", None)
+    try:
+        return pairwise_kernel_spec(pairwise_fn, unit_scale=scale)
+    except TypeError:
+        raise TypeError("Unsupported pairwise_fn for native propagation.") from None
+
+
 # ---------------------------------------------------------------------------
 # Hot-path wrappers (argument lists of the reference's pybind ops).
 # ---------------------------------------------------------------------------
@@ -184,11 +199,10 @@ def propagation_topk_native(
     target_block_size: int,
     source_block_size: int,
 ) -> LayerDelta:
-    if not supports_pairwise_kernel(pairwise_fn):
-        raise TypeError("Unsupported pairwise_fn for native propagation.")
-    spec = pairwise_kernel_spec(pairwise_fn, unit_scale=getattr(_native_module(), "unit_scale", None))
+    module = _native_module()
+    spec = _pairwise_spec(pairwise_fn, module)
     return _as_layer_delta(
-        _native_module().propagation_topk(
+        module.propagation_topk(
             spec.kind, spec.weight, spec.bias, spec.in_weight, spec.in_bias, spec.out_weight, spec.out_bias,
             edge_compress_name, layer_val, projected_state, projected_val, topk, target_block_size,
             source_block_size,
@@ -207,11 +221,10 @@ def propagation_window_native(
     target_block_size: int,
     source_block_size: int,
 ) -> LayerDelta:
-    if not supports_pairwise_kernel(pairwise_fn):
-        raise TypeError("Unsupported pairwise_fn for native propagation.")
-    spec = pairwise_kernel_spec(pairwise_fn, unit_scale=getattr(_native_module(), "unit_scale", None))
+    module = _native_module()
+    spec = _pairwise_spec(pairwise_fn, module)
     return _as_layer_delta(
-        _native_module().propagation_window(
+        module.propagation_window(
             spec.kind, spec.weight, spec.bias, spec.in_weight, spec.in_bias, spec.out_weight, spec.out_bias,
             edge_compress_name, layer_val, projected_state, projected_val, window, target_block_size,
             source_block_size,
@@ -230,11 +243,10 @@ def propagation_dense_native(
     target_block_size: int,
     source_block_size: int,
 ) -> LayerDelta:
-    if not supports_pairwise_kernel(pairwise_fn):
-        raise TypeError("Unsupported pairwise_fn for native propagation.")
-    spec = pairwise_kernel_spec(pairwise_fn, unit_scale=getattr(_native_module(), "unit_scale", None))
+    module = _native_module()
+    spec = _pairwise_spec(pairwise_fn, module)
     return _as_layer_delta(
-        _native_module().propagation_dense(
+        module.propagation_dense(
             spec.kind, spec.weight, spec.bias, spec.in_weight, spec.in_bias, spec.out_weight, spec.out_bias,
             edge_compress_name, layer_val, projected_state, projected_val, source_state, target_block_size,
             source_block_size,

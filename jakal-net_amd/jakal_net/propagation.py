@@ -47,8 +47,7 @@ from jakal_net.core import (
 from jakal_net.kernel_common import supports_pairwise_kernel
 from jakal_net.native_backend import (
     native_disabled_by_env,
-    native_supports,
-    native_supports_device,
+    native_runs,
     propagation_dense_native,
     propagation_topk_native,
     propagation_window_native,
@@ -174,7 +173,7 @@ class Propagation(nn.Module):
         if compress is None or native_disabled_by_env():
             return None
         op, device_type = self._native_op_name(), layer.val.device.type
-        if not (native_supports(op) and native_supports_device(device_type)):
+        if not native_runs(op, device_type):
             if strict:
                 require_native_for_device(op, device_type)
             return None

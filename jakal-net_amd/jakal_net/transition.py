@@ -45,8 +45,7 @@ from jakal_net.core import (
 from jakal_net.kernel_common import supports_pairwise_route_kernel
 from jakal_net.native_backend import (
     native_disabled_by_env,
-    native_supports,
-    native_supports_device,
+    native_runs,
     require_native_for_device,
     transition_pairwise_dense_native,
     transition_pairwise_topk_native,
@@ -208,7 +207,7 @@ class Transition(nn.Module):
         if not self._on_native_path() or native_disabled_by_env():
             return None
         op, device_type = self._native_op_name(), src_layer.val.device.type
-        if not (native_supports(op) and native_supports_device(device_type)):
+        if not native_runs(op, device_type):
             if strict:
                 require_native_for_device(op, device_type)
             return None

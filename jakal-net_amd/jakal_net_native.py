@@ -19,12 +19,14 @@ loaded; nothing here computes on the CPU.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from pathlib import Path
 
 import torch
 from torch import Tensor
+from torch.autograd import forward_ad
 
 LIB_ENV = "JAKAL_NET_HIP_LIB"
 _HERE = Path(__file__).resolve().parent
@@ -335,11 +337,56 @@ def _check(rc: int) -> None:
 
 
 def _ptr(t: Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if _raw_stream is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """A context that makes `device` the current one (nothing to do when it is)."""
+    return _SAME_DEVICE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+
+
+def _records(*tensors: Tensor | None) -> bool:
+    """Whether a call on these tensors has to go through its autograd function:
+    a backward may follow, or a transform (forward mode, torch.func, tracing)
+    looks at it.  Otherwise the forward runs by itself and keeps nothing."""
+    if torch.is_grad_enabled():
+        for t in tensors:
+            if t is not None and t.requires_grad:
+                return True
+    return (forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
+            or torch._C._are_functorch_transforms_active())
+
+
+class _NoContext:
+    """Stands for an autograd function's context in a forward that keeps nothing."""
+
+    def __init__(self, inputs: int) -> None:
+        self.needs_input_grad = (False,) * inputs
+
+    def save_for_backward(self, *tensors) -> None:
+        pass
+
+    def set_materialize_grads(self, value: bool) -> None:
+        pass
+
+
+def _run(function, *args):
+    """function.apply(*args), or its forward alone where nothing records it."""
+    if _records(*(a for a in args if isinstance(a, Tensor))):
+        return function.apply(*args)
+    return function.forward(_NoContext(len(args)), *args)
 
 
 def _require_gpu(*tensors: Tensor | None) -> torch.device:
@@ -347,18 +394,33 @@ def _require_gpu(*tensors: Tensor | None) -> torch.device:
     for t in tensors:
         if t is None:
             continue
+        if device is not None and t.device == device:
+            continue
         if t.device.type != "cuda":
             raise RuntimeError(f"jakal_net_native ops need GPU tensors, got a tensor on {t.device}.")
-        if device is None:
-            device = t.device
-        elif t.device != device:
+        if device is not None:
             raise RuntimeError("jakal_net_native ops need all tensors on one device.")
+        device = t.device
     assert device is not None
     return device
 
 
 def _f32(t: Tensor | None) -> Tensor | None:
-    return None if t is None else t.float().contiguous()
+    if t is None or (t.dtype is torch.float32 and t.is_contiguous()):
+        return t
+    return t.float().contiguous()
+
+
+def _rows(t: Tensor, *shape: int) -> Tensor:
+    """t [..., *shape] with its batch axes flattened to one."""
+    return t if t.shape[1:] == shape else t.reshape(-1, *shape)
+
+
+def _like(t: Tensor, batch_shape: tuple, dtype: torch.dtype) -> Tensor:
+    """An op's [B, ...] output with the caller's batch axes and dtype."""
+    if len(batch_shape) != 1:
+        t = t.reshape(*batch_shape, *t.shape[1:])
+    return t if t.dtype is dtype else t.to(dtype)
 
 
 def _same_storage_view(a: Tensor, b: Tensor) -> bool:
@@ -391,6 +453,70 @@ def _edges_per_row(mode: str, param: int, N: int) -> int:
     return param if mode == "topk" else min(param + 1, N)
 
 
+def _pad64(n: int) -> int:
+    """n elements of 4 bytes up to whole 256 bytes: the next buffer of one allocation starts there."""
+    return (n + 63) // 64 * 64
+
+
+def _edges_forward(X, ps, pv_t, V, U, w, bias, mode: str, param: int, compress: int, heads: int, bf16: bool,  # noqa: N803
+                   raw: int, keep_edges: bool, layout_bytes: int):
+    """The forward of an edge-list propagation (see _PropagationEdges).
+
+    Returns (delta_state, delta_val, proj, idx, score, head, layout): proj
+    holds the score scale (when raw) and then the projections; with keep_edges
+    idx and score are the [B, N, k] edge list, otherwise idx is one flat
+    buffer of both and score is None."""
+    B, N, Din = X.shape
+    Dout = pv_t.shape[-1]
+    r = U.shape[0]
+    mh = heads > 1
+    rank_arg = (r // heads, heads) if mh else (r,)
+    k = _edges_per_row(mode, param, N)
+    dev = X.device
+    M = B * N
+    fwd = getattr(_LIB, _EDGE_OPS[mode, "bf16" if bf16 else mh][0])
+    with _on(dev):
+        stream = _stream(dev)
+        ds = torch.empty(B, N, device=dev, dtype=torch.float32)
+        dv = torch.empty(B, N, Dout, device=dev, dtype=torch.bfloat16 if bf16 else torch.float32)
+        scale_n = _pad64(r) if raw else 0
+        proj = torch.empty(scale_n + M * 2 * r, device=dev, dtype=torch.float32)
+        w_ptr = w.data_ptr()
+        if raw:
+            _check(_LIB.jn_unit_scale_forward(w_ptr, raw, r // raw, UNIT_SCALE_EPS, proj.data_ptr(), stream))
+            w_ptr = proj.data_ptr()
+        if keep_edges:
+            idx = torch.empty(B, N, k, device=dev, dtype=torch.int32)
+            score = torch.empty(B, N, k, device=dev, dtype=torch.float32)
+            score_ptr = score.data_ptr()
+        else:
+            idx = torch.empty(2 * _pad64(M * k), device=dev, dtype=torch.int32)
+            score = None
+            score_ptr = idx.data_ptr() + 4 * _pad64(M * k)
+        head = torch.empty(B, N, k, device=dev, dtype=torch.uint8) if mh else None
+        args = [
+            X.data_ptr(), ps.data_ptr(), pv_t.data_ptr(), U.data_ptr(), V.data_ptr(), w_ptr, _ptr(bias),
+            B, N, Din, Dout, *rank_arg, param, compress,
+            ds.data_ptr(), dv.data_ptr(), proj.data_ptr() + 4 * scale_n, idx.data_ptr(), score_ptr,
+        ]
+        if mh:
+            args.append(head.data_ptr())
+        layout = None
+        if mode == "topk":
+            if layout_bytes:
+                layout = torch.empty(layout_bytes, device=dev, dtype=torch.uint8)
+                args += [layout.data_ptr(), layout_bytes]
+            else:
+                args += [None, 0]
+            # the select's scratch
+            ws_bytes = int(_LIB.jn_propagation_topk_forward_multihead_workspace_bytes(B, N, *rank_arg) if mh
+                           else _LIB.jn_propagation_topk_forward_workspace_bytes(B, N, r))
+            ws = torch.empty(max(ws_bytes, 1), device=dev, dtype=torch.uint8)
+            args += [ws.data_ptr(), ws_bytes]
+        _check(fwd(*args, stream))
+    return ds, dv, proj, idx, score, head, layout
+
+
 class _PropagationEdges(torch.autograd.Function):
     """Differentiable low-rank propagation over an edge list on the HIP library.
 
@@ -398,98 +524,83 @@ class _PropagationEdges(torch.autograd.Function):
     (param = window) takes the causal band j in [i - window, i].  Inputs (all
     fp32, contiguous): layer_val X [B,N,Din], projected_state [B,N],
     projected_val [B,N,Dout] or None when it is X itself, V and U [r,Din],
-    w_hat [r], bias [] or None.  With heads > 1 the r ranks are `heads`
-    equal head slices (max-aggregated scores) and bias is [heads].  With
-    bf16, X and pv are bf16 (one head) and delta_val comes back in bf16."""
+    w [r], bias [] or None.  With heads > 1 the r ranks are `heads` equal head
+    slices (max-aggregated scores) and bias is [heads].  With bf16, X and pv
+    are bf16 (one head) and delta_val comes back in bf16.  raw = 0: w is the
+    score scale w_hat; raw = rows: w holds that many rows of raw weights, which
+    the op scales to unit norm itself (jn_unit_scale_*).  The edge list is an
+    output only with keep_edges."""
 
     @staticmethod
-    def forward(ctx, X, ps, pv, V, U, w_hat, bias, mode: str, param: int, compress: int, heads: int = 1,  # noqa: N803
-                bf16: bool = False):
-        B, N, Din = X.shape
-        pv_is_x = pv is None
-        pv_t = X if pv_is_x else pv
-        Dout = pv_t.shape[-1]
-        r = U.shape[0]
-        mh = heads > 1
-        rank_arg = [r // heads, heads] if mh else [r]
-        k = _edges_per_row(mode, param, N)
-        dev = X.device
-        variant = "bf16" if bf16 else mh
-        fwd = getattr(_LIB, _EDGE_OPS[mode, variant][0])
-        with torch.cuda.device(dev):
-            ds = torch.empty(B, N, device=dev, dtype=torch.float32)
-            dv = torch.empty(B, N, Dout, device=dev, dtype=torch.bfloat16 if bf16 else torch.float32)
-            proj = torch.empty(B * N, 2 * r, device=dev, dtype=torch.float32)
-            idx = torch.empty(B, N, k, device=dev, dtype=torch.int32)
-            score = torch.empty(B, N, k, device=dev, dtype=torch.float32)
-            head = torch.empty(B, N, k, device=dev, dtype=torch.uint8) if mh else None
-            args = [
-                _ptr(X), _ptr(ps), _ptr(pv_t), _ptr(U), _ptr(V), _ptr(w_hat), _ptr(bias),
-                B, N, Din, Dout, *rank_arg, param, compress,
-                _ptr(ds), _ptr(dv), _ptr(proj), _ptr(idx), _ptr(score),
-            ]
-            if mh:
-                args.append(_ptr(head))
-            layout = None
-            if mode == "topk":
-                # the edges grouped by key for the backward, built beside the
-                # forward's row pass when a backward will follow
-                if EDGE_LAYOUT and any(ctx.needs_input_grad[:7]):
-                    layout_bytes = int(_LIB.jn_propagation_topk_layout_bytes(B, N, k))
-                    layout = torch.empty(layout_bytes, device=dev, dtype=torch.uint8)
-                    args += [_ptr(layout), layout_bytes]
-                else:
-                    args += [None, 0]
-                # the select's scratch
-                ws_bytes = int(_LIB.jn_propagation_topk_forward_multihead_workspace_bytes(B, N, *rank_arg) if mh
-                               else _LIB.jn_propagation_topk_forward_workspace_bytes(B, N, r))
-                ws = torch.empty(max(ws_bytes, 1), device=dev, dtype=torch.uint8)
-                args += [_ptr(ws), ws_bytes]
-            _check(fwd(*args, _stream(dev)))
-        ctx.save_for_backward(X, ps, pv_t, V, U, w_hat, proj, idx, score, head)
+    def forward(ctx, X, ps, pv, V, U, w, bias, mode: str, param: int, compress: int, heads: int = 1,  # noqa: N803
+                bf16: bool = False, raw: int = 0, keep_edges: bool = True):
+        pv_t = X if pv is None else pv
+        # the edges grouped by key for the backward, built beside the forward's
+        # row pass when a backward will follow
+        layout_bytes = 0
+        if mode == "topk" and EDGE_LAYOUT and any(ctx.needs_input_grad[:7]):
+            layout_bytes = int(_LIB.jn_propagation_topk_layout_bytes(X.shape[0], X.shape[1], param))
+        ds, dv, proj, idx, score, head, layout = _edges_forward(X, ps, pv_t, V, U, w, bias, mode, param, compress,
+                                                                heads, bf16, raw, keep_edges, layout_bytes)
+        ctx.save_for_backward(X, ps, pv_t, V, U, w, proj, idx, score, head)
         ctx.edge_layout = layout
-        ctx.meta = (mode, param, compress, pv_is_x, bias is not None, heads, bf16)
+        ctx.meta = (mode, param, compress, pv is None, bias is not None, heads, bf16, raw)
+        ctx.set_materialize_grads(False)  # no zero-filled gradients for unused outputs
+        if not keep_edges:
+            return ds, dv
         ctx.mark_non_differentiable(idx, score)
-        ctx.set_materialize_grads(False)  # no zero-filled gradients for the edge-list outputs
         return ds, dv, idx, score
 
     @staticmethod
     def backward(ctx, g_ds, g_dv, _g_idx=None, _g_score=None):
-        X, ps, pv, V, U, w_hat, proj, idx, score, head = ctx.saved_tensors
-        mode, param, compress, pv_is_x, has_bias, heads, bf16 = ctx.meta
+        X, ps, pv, V, U, w, proj, idx, score, head = ctx.saved_tensors
+        mode, param, compress, pv_is_x, has_bias, heads, bf16, raw = ctx.meta
         mh = heads > 1
         _, ws_name, bwd_name = _EDGE_OPS[mode, "bf16" if bf16 else mh]
         B, N, Din = X.shape
         Dout = pv.shape[-1]
         r = U.shape[0]
-        rank_arg = [r // heads, heads] if mh else [r]
+        rank_arg = (r // heads, heads) if mh else (r,)
         dev = X.device
         need = ctx.needs_input_grad
         ds_used = g_ds is not None  # projected_state reaches delta_state only
-        with torch.cuda.device(dev):
+        with _on(dev):
+            stream = _stream(dev)
             vdt = torch.bfloat16 if bf16 else torch.float32
-            g_ds = torch.zeros(B, N, device=dev) if g_ds is None else g_ds.float().contiguous()
+            g_ds = torch.zeros(B, N, device=dev) if g_ds is None else _f32(g_ds)
             g_dv = torch.zeros(B, N, Dout, device=dev, dtype=vdt) if g_dv is None else g_dv.to(vdt).contiguous()
             gX = torch.empty_like(X) if need[0] else None
             gps = torch.empty_like(ps) if need[1] and ds_used else None
             gpv = torch.empty_like(pv) if (not pv_is_x and need[2]) else None
             gV = torch.empty_like(V)
             gU = torch.empty_like(U)
-            gw = torch.empty_like(w_hat)
+            gw = torch.empty_like(w)
             gb = torch.empty((heads,) if mh else (), device=dev, dtype=torch.float32) if has_bias else None
             ws_bytes = int(getattr(_LIB, ws_name)(B, N, Din, Dout, *rank_arg, param))
-            ws = torch.empty(max(ws_bytes, 1), device=dev, dtype=torch.uint8)
-            edge_args = [_ptr(idx), _ptr(score)] + ([_ptr(head)] if mh else [])
-            layout_arg = [_ptr(ctx.edge_layout)] if mode == "topk" else []
-            _check(
-                getattr(_LIB, bwd_name)(
-                    _ptr(X), _ptr(ps), _ptr(pv), _ptr(U), _ptr(V), _ptr(w_hat),
-                    _ptr(proj), *edge_args, _ptr(g_ds), _ptr(g_dv),
-                    B, N, Din, Dout, *rank_arg, param, compress, 1 if pv_is_x else 0,
-                    _ptr(gX), _ptr(gps), _ptr(gpv), _ptr(gU), _ptr(gV), _ptr(gw), _ptr(gb),
-                    *layout_arg, _ptr(ws), ws_bytes, _stream(dev),
-                )
-            )
+            # with raw weights, the scale's gradient sits behind the workspace
+            scale_at = (ws_bytes + 255) // 256 * 256
+            ws = torch.empty(scale_at + 4 * r if raw else max(ws_bytes, 1), device=dev, dtype=torch.uint8)
+            w_ptr = proj.data_ptr() if raw else w.data_ptr()
+            gw_ptr = ws.data_ptr() + scale_at if raw else gw.data_ptr()
+            idx_ptr = idx.data_ptr()
+            score_ptr = score.data_ptr() if score is not None else (
+                idx_ptr + 4 * _pad64(B * N * _edges_per_row(mode, param, N)))
+            args = [
+                X.data_ptr(), ps.data_ptr(), pv.data_ptr(), U.data_ptr(), V.data_ptr(), w_ptr,
+                proj.data_ptr() + (4 * _pad64(r) if raw else 0), idx_ptr, score_ptr,
+            ]
+            if mh:
+                args.append(head.data_ptr())
+            args += [
+                g_ds.data_ptr(), g_dv.data_ptr(), B, N, Din, Dout, *rank_arg, param, compress, 1 if pv_is_x else 0,
+                _ptr(gX), _ptr(gps), _ptr(gpv), gU.data_ptr(), gV.data_ptr(), gw_ptr, _ptr(gb),
+            ]
+            if mode == "topk":
+                args.append(_ptr(ctx.edge_layout))
+            _check(getattr(_LIB, bwd_name)(*args, ws.data_ptr(), ws_bytes, stream))
+            if raw and need[5]:
+                _check(_LIB.jn_unit_scale_backward(w.data_ptr(), gw_ptr, raw, r // raw, UNIT_SCALE_EPS, gw.data_ptr(),
+                                                   stream))
         return (
             gX,
             gps,
@@ -498,11 +609,7 @@ class _PropagationEdges(torch.autograd.Function):
             gU if need[4] else None,
             gw if need[5] else None,
             gb if (has_bias and need[6]) else None,
-            None,
-            None,
-            None,
-            None,
-            None,
+            None, None, None, None, None, None, None,
         )
 
 
@@ -516,7 +623,7 @@ class _UnitScale(torch.autograd.Function):
     @staticmethod
     def forward(ctx, w):  # noqa: D401
         out = torch.empty_like(w)
-        with torch.cuda.device(w.device):
+        with _on(w.device):
             _check(_LIB.jn_unit_scale_forward(_ptr(w), w.shape[0], w.shape[1], UNIT_SCALE_EPS, _ptr(out),
                                               _stream(w.device)))
         ctx.save_for_backward(w)
@@ -527,7 +634,7 @@ class _UnitScale(torch.autograd.Function):
         (w,) = ctx.saved_tensors
         g = g.float().contiguous()
         gw = torch.empty_like(w)
-        with torch.cuda.device(w.device):
+        with _on(w.device):
             _check(_LIB.jn_unit_scale_backward(_ptr(w), _ptr(g), w.shape[0], w.shape[1], UNIT_SCALE_EPS,
                                                _ptr(gw), _stream(w.device)))
         return gw
@@ -541,8 +648,27 @@ def unit_scale(weight: Tensor) -> Tensor:
     if not weight.is_cuda or weight.dtype != torch.float32 or weight.dim() not in (1, 2):
         raise NotImplementedError("unit_scale takes an fp32 [r] or [H, r] tensor on a HIP device")
     w2 = weight.contiguous().view(1, -1) if weight.dim() == 1 else weight.contiguous()
-    out = _UnitScale.apply(w2)
+    out = _run(_UnitScale, w2)
     return out.view(-1) if weight.dim() == 1 else out
+
+
+class _RawScale:
+    """A raw score weight ([r], or an [H, r] stack) in the place of w_hat: the
+    op takes its unit norm itself."""
+
+    __slots__ = ("weight",)
+
+    def __init__(self, weight: Tensor) -> None:
+        self.weight = weight
+
+
+def raw_scale(weight: Tensor) -> _RawScale:
+    """Stands for unit_scale(weight) as the weight of propagation_topk,
+    propagation_window and propagation_dense, which then scale it in the same
+    call (one autograd node instead of two).  Same limits as unit_scale."""
+    if not weight.is_cuda or weight.dtype != torch.float32 or weight.dim() not in (1, 2):
+        raise NotImplementedError("unit_scale takes an fp32 [r] or [H, r] tensor on a HIP device")
+    return _RawScale(weight)
 
 
 def _bf16_rows(*tensors: Tensor | None) -> bool:
@@ -601,7 +727,7 @@ class _PropagationDense(torch.autograd.Function):
         dev = X.device
         edge_bytes = N * N * 4
         chunk = B if B * edge_bytes <= DENSE_EDGE_BYTES else max(1, DENSE_EDGE_BYTES // edge_bytes)
-        with torch.cuda.device(dev):
+        with _on(dev):
             ds = torch.empty(B, N, device=dev, dtype=torch.float32)
             dv = torch.empty(B, N, Dout, device=dev, dtype=torch.bfloat16 if bf16 else torch.float32)
             proj = torch.empty(B * N, 2 * r, device=dev, dtype=torch.float32)
@@ -650,7 +776,7 @@ class _PropagationDense(torch.autograd.Function):
         dev = X.device
         need = ctx.needs_input_grad
         ds_used = g_ds is not None  # projected_state reaches delta_state only
-        with torch.cuda.device(dev):
+        with _on(dev):
             vdt = torch.bfloat16 if bf16 else torch.float32
             g_ds = torch.zeros(B, N, device=dev) if g_ds is None else g_ds.float().contiguous()
             g_dv = torch.zeros(B, N, Dout, device=dev, dtype=vdt) if g_dv is None else g_dv.to(vdt).contiguous()
@@ -686,7 +812,7 @@ class _PropagationDense(torch.autograd.Function):
         dev = X.device
         need = ctx.needs_input_grad
         ds_used = g_ds is not None  # projected_state reaches delta_state only
-        with torch.cuda.device(dev):
+        with _on(dev):
             vdt = torch.bfloat16 if bf16 else torch.float32
             g_ds = torch.zeros(B, N, device=dev) if g_ds is None else g_ds.float().contiguous()
             g_dv = torch.zeros(B, N, Dout, device=dev, dtype=vdt) if g_dv is None else g_dv.to(vdt).contiguous()
@@ -727,7 +853,7 @@ class _PropagationDenseMultihead(torch.autograd.Function):
         dev = X.device
         per = N * N * 5  # fp32 edge and uint8 head per pair
         chunk = B if B * per <= DENSE_EDGE_BYTES else max(1, DENSE_EDGE_BYTES // per)
-        with torch.cuda.device(dev):
+        with _on(dev):
             ds = torch.empty(B, N, device=dev, dtype=torch.float32)
             dv = torch.empty(B, N, Dout, device=dev, dtype=torch.float32)
             proj = torch.empty(B * N, 2 * R, device=dev, dtype=torch.float32)
@@ -760,7 +886,7 @@ class _PropagationDenseMultihead(torch.autograd.Function):
         dev = X.device
         need = ctx.needs_input_grad
         ds_used = g_ds is not None  # projected_state reaches delta_state only
-        with torch.cuda.device(dev):
+        with _on(dev):
             g_ds = torch.zeros(B, N, device=dev) if g_ds is None else g_ds.float().contiguous()
             g_dv = torch.zeros(B, N, Dout, device=dev) if g_dv is None else g_dv.float().contiguous()
             gX = torch.empty_like(X) if need[0] else None
@@ -815,6 +941,8 @@ def propagation_dense(
     With ``source_state`` the edges are weighted by it per source, which
     equals the unweighted op on (source_state, source_state * projected_val)
     (jakal_net_native.cpp:5991-6015); the fold is done here, differentiably."""
+    if isinstance(weight, _RawScale):
+        weight = unit_scale(weight.weight)
     w_hat, bias, V, U, heads = _lowrank_pairwise_args(pairwise_kind, weight, bias, in_weight, in_bias, out_weight,
                                                       out_bias)
     if edge_compress_name not in _COMPRESS_KINDS:
@@ -837,11 +965,11 @@ def propagation_dense(
     ps = _f32(projected_state.reshape(-1, N))
     pv = None if pv_is_x else rows(projected_val.reshape(-1, N, Dout))
     if heads > 1:
-        ds, dv = _PropagationDenseMultihead.apply(X, ps, pv, _f32(V), _f32(U), _f32(w_hat), _f32(bias),
-                                                  _COMPRESS_KINDS[edge_compress_name], _causal, heads)
+        ds, dv = _run(_PropagationDenseMultihead, X, ps, pv, _f32(V), _f32(U), _f32(w_hat), _f32(bias),
+                      _COMPRESS_KINDS[edge_compress_name], _causal, heads)
     else:
-        ds, dv = _PropagationDense.apply(X, ps, pv, _f32(V), _f32(U), _f32(w_hat), _f32(bias),
-                                         _COMPRESS_KINDS[edge_compress_name], _causal, bf16)
+        ds, dv = _run(_PropagationDense, X, ps, pv, _f32(V), _f32(U), _f32(w_hat), _f32(bias),
+                      _COMPRESS_KINDS[edge_compress_name], _causal, bf16)
     return (ds.reshape(*batch_shape, N).to(projected_state.dtype),
             dv.reshape(*batch_shape, N, Dout).to(projected_val.dtype))
 
@@ -897,35 +1025,43 @@ def _check_select(k: int, limit: int = MAX_TOPK_LARGE) -> None:
 
 def _propagation_edges(mode, pairwise_kind, weight, bias, in_weight, in_bias, out_weight, out_bias,
                        edge_compress_name, layer_val, projected_state, projected_val, param, target_block_size,
-                       source_block_size):
-    w_hat, bias, V, U, heads = _lowrank_pairwise_args(pairwise_kind, weight, bias, in_weight, in_bias, out_weight,
-                                                      out_bias)
+                       source_block_size, keep_edges=True):
+    """(delta_state, delta_val, idx, score); without keep_edges the edge list is not returned."""
+    raw = isinstance(weight, _RawScale)
+    if raw:
+        weight = weight.weight
+    w, bias, V, U, heads = _lowrank_pairwise_args(pairwise_kind, weight, bias, in_weight, in_bias, out_weight,
+                                                  out_bias)
     if edge_compress_name not in _COMPRESS_KINDS:
         raise RuntimeError(f"Unsupported edge_compress_name for the HIP backend: {edge_compress_name!r}.")
     if target_block_size <= 0 or source_block_size <= 0:
         raise RuntimeError("block sizes must be positive.")
-    _require_gpu(layer_val, projected_state, projected_val, w_hat, V, U, bias)
-    batch_shape = tuple(layer_val.shape[:-2])
-    N, Din = layer_val.shape[-2], layer_val.shape[-1]
+    _require_gpu(layer_val, projected_state, projected_val, w, V, U, bias)
+    batch_shape = layer_val.shape[:-2]
+    N, Din = layer_val.shape[-2:]
     Dout = projected_val.shape[-1]
     pv_is_x = _same_storage_view(projected_val, layer_val)
     # bf16 layers keep bf16 value rows (one head); anything else computes in fp32
     bf16 = heads == 1 and _bf16_rows(layer_val, projected_val)
     rows = _bf16 if bf16 else _f32
-    X = rows(layer_val.reshape(-1, N, Din))
-    ps = _f32(projected_state.reshape(-1, N))
-    pv = None if pv_is_x else rows(projected_val.reshape(-1, N, Dout))
-    ds, dv, idx, score = _PropagationEdges.apply(
-        X, ps, pv, _f32(V), _f32(U), _f32(w_hat), _f32(bias), mode, int(param), _COMPRESS_KINDS[edge_compress_name],
-        heads, bf16,
-    )
-    k = idx.shape[-1]
-    return (
-        ds.reshape(*batch_shape, N).to(projected_state.dtype),
-        dv.reshape(*batch_shape, N, Dout).to(projected_val.dtype),
-        idx.reshape(*batch_shape, N, k),
-        score.reshape(*batch_shape, N, k),
-    )
+    X = rows(_rows(layer_val, N, Din))
+    ps = _f32(_rows(projected_state, N))
+    pv = None if pv_is_x else rows(_rows(projected_val, N, Dout))
+    V, U, w, bias = _f32(V), _f32(U), _f32(w), _f32(bias)
+    compress = _COMPRESS_KINDS[edge_compress_name]
+    if _records(X, ps, pv, V, U, w, bias):
+        out = _PropagationEdges.apply(X, ps, pv, V, U, w, bias, mode, int(param), compress, heads, bf16,
+                                      heads if raw else 0, keep_edges)
+    else:
+        ds, dv, _, idx, score, _, _ = _edges_forward(X, ps, X if pv is None else pv, V, U, w, bias, mode, int(param),
+                                                     compress, heads, bf16, heads if raw else 0, keep_edges, 0)
+        out = (ds, dv, idx, score)
+    ds = _like(out[0], batch_shape, projected_state.dtype)
+    dv = _like(out[1], batch_shape, projected_val.dtype)
+    if not keep_edges:
+        return ds, dv, None, None
+    k = out[2].shape[-1]
+    return ds, dv, out[2].reshape(*batch_shape, N, k), out[3].reshape(*batch_shape, N, k)
 
 
 def propagation_topk_selection(
@@ -1018,11 +1154,11 @@ def propagation_window(
         return propagation_dense(pairwise_kind, weight, bias, in_weight, in_bias, out_weight, out_bias,
                                  edge_compress_name, layer_val, projected_state, projected_val, None,
                                  target_block_size, source_block_size, _causal=True)
-    ds, dv, _, _ = propagation_window_edges(
-        pairwise_kind, weight, bias, in_weight, in_bias, out_weight, out_bias, edge_compress_name, layer_val,
-        projected_state, projected_val, window, target_block_size, source_block_size,
-    )
-    return ds, dv
+    if window < 0:
+        raise RuntimeError("window must be non-negative.")
+    return _propagation_edges("window", pairwise_kind, weight, bias, in_weight, in_bias, out_weight, out_bias,
+                              edge_compress_name, layer_val, projected_state, projected_val, int(window),
+                              target_block_size, source_block_size, keep_edges=False)[:2]
 
 
 def propagation_topk(
@@ -1051,79 +1187,102 @@ def propagation_topk(
         return propagation_dense(pairwise_kind, weight, bias, in_weight, in_bias, out_weight, out_bias,
                                  edge_compress_name, layer_val, projected_state, projected_val, None,
                                  target_block_size, source_block_size)
-    ds, dv, _, _ = propagation_topk_selection(
-        pairwise_kind, weight, bias, in_weight, in_bias, out_weight, out_bias, edge_compress_name, layer_val,
-        projected_state, projected_val, topk, target_block_size, source_block_size,
-    )
-    return ds, dv
+    if topk <= 0:
+        raise RuntimeError("topk must be positive.")
+    _check_select(int(topk))
+    return _propagation_edges("topk", pairwise_kind, weight, bias, in_weight, in_bias, out_weight, out_bias,
+                              edge_compress_name, layer_val, projected_state, projected_val, int(topk),
+                              target_block_size, source_block_size, keep_edges=False)[:2]
 
 
 # ---------------------------------------------------------------------------
 # sparse transition (low-rank pairwise route, top-k destinations per source)
 # ---------------------------------------------------------------------------
+def _routes_forward(rho, src, dst, ps, pv, Ws, Wt, w, bias, temperature: float, topk: int, compress: int,  # noqa: N803
+                    heads: int, bf16: bool, keep_routes: bool):
+    """The forward of a sparse transition (see _TransitionTopK).
+
+    Returns (delta_state, delta_val, proj, idx, logit, head): proj holds the
+    source projections and then the destinations'; with keep_routes idx and
+    logit are the [B, Ns, k] routes, otherwise idx is one flat buffer of both
+    and logit is None."""
+    B, Ns, Dsrc = src.shape
+    _, Nd, Ddst = dst.shape
+    Dv = pv.shape[-1]
+    r = Ws.shape[0]
+    mh = heads > 1
+    rank_arg = (r // heads, heads) if mh else (r,)
+    k = min(topk, Nd)
+    dev = src.device
+    with _on(dev):
+        ds = torch.empty(B, Nd, device=dev, dtype=torch.float32)
+        dv = torch.empty(B, Nd, Dv, device=dev, dtype=torch.bfloat16 if bf16 else torch.float32)
+        proj = torch.empty(_pad64(B * Ns * r) + B * Nd * r, device=dev, dtype=torch.float32)
+        if keep_routes:
+            idx = torch.empty(B, Ns, k, device=dev, dtype=torch.int32)
+            logit = torch.empty(B, Ns, k, device=dev, dtype=torch.float32)
+            logit_ptr = logit.data_ptr()
+        else:
+            idx = torch.empty(2 * _pad64(B * Ns * k), device=dev, dtype=torch.int32)
+            logit = None
+            logit_ptr = idx.data_ptr() + 4 * _pad64(B * Ns * k)
+        head = torch.empty(B, Ns, k, device=dev, dtype=torch.uint8) if mh else None
+        ws_fn = _LIB.jn_transition_topk_multihead_workspace_bytes if mh else _LIB.jn_transition_topk_workspace_bytes
+        ws_bytes = int(ws_fn(B, Ns, Nd, Dsrc, Ddst, Dv, *rank_arg, topk))
+        ws = torch.empty(max(ws_bytes, 1), device=dev, dtype=torch.uint8)
+        fwd = (_LIB.jn_transition_topk_forward_multihead if mh else
+               _LIB.jn_transition_topk_forward_bf16 if bf16 else _LIB.jn_transition_topk_forward)
+        sp = proj.data_ptr()
+        _check(
+            fwd(
+                rho.data_ptr(), src.data_ptr(), dst.data_ptr(), ps.data_ptr(), pv.data_ptr(), Ws.data_ptr(),
+                Wt.data_ptr(), w.data_ptr(), _ptr(bias), temperature, B, Ns, Nd, Dsrc, Ddst, Dv, *rank_arg, topk,
+                compress, ds.data_ptr(), dv.data_ptr(), sp, sp + 4 * _pad64(B * Ns * r), idx.data_ptr(), logit_ptr,
+                *((head.data_ptr(),) if mh else ()), ws.data_ptr(), ws_bytes, _stream(dev),
+            )
+        )
+    return ds, dv, proj, idx, logit, head
+
+
 class _TransitionTopK(torch.autograd.Function):
     """Differentiable SparseTransition routing on the HIP library.
 
     Inputs (fp32, contiguous): sender strength rho [B,Ns], src_val [B,Ns,Dsrc],
     dst_val [B,Nd,Ddst], projected_state [B,Ns], projected_val [B,Ns,Dv],
-    Ws [r,Dsrc], Wt [r,Ddst], w [r] (raw), bias [] or None."""
+    Ws [r,Dsrc], Wt [r,Ddst], w [r] (raw), bias [] or None.  The routes are
+    outputs only with keep_routes."""
 
     @staticmethod
     def forward(ctx, rho, src, dst, ps, pv, Ws, Wt, w, bias, temperature: float, topk: int, compress: int,  # noqa: N803
-                heads: int = 1, bf16: bool = False):
-        B, Ns, Dsrc = src.shape
-        Nd, Ddst = dst.shape[1], dst.shape[2]
-        Dv = pv.shape[-1]
-        r = Ws.shape[0]
-        mh = heads > 1
-        rank_arg = [r // heads, heads] if mh else [r]
-        k = min(int(topk), Nd)
-        dev = src.device
-        with torch.cuda.device(dev):
-            ds = torch.empty(B, Nd, device=dev, dtype=torch.float32)
-            dv = torch.empty(B, Nd, Dv, device=dev, dtype=torch.bfloat16 if bf16 else torch.float32)
-            sp = torch.empty(B * Ns, r, device=dev, dtype=torch.float32)
-            dp = torch.empty(B * Nd, r, device=dev, dtype=torch.float32)
-            idx = torch.empty(B, Ns, k, device=dev, dtype=torch.int32)
-            logit = torch.empty(B, Ns, k, device=dev, dtype=torch.float32)
-            head = torch.empty(B, Ns, k, device=dev, dtype=torch.uint8) if mh else None
-            ws_fn = _LIB.jn_transition_topk_multihead_workspace_bytes if mh else _LIB.jn_transition_topk_workspace_bytes
-            ws_bytes = int(ws_fn(B, Ns, Nd, Dsrc, Ddst, Dv, *rank_arg, topk))
-            ws = torch.empty(max(ws_bytes, 1), device=dev, dtype=torch.uint8)
-            fwd = (_LIB.jn_transition_topk_forward_multihead if mh else
-                   _LIB.jn_transition_topk_forward_bf16 if bf16 else _LIB.jn_transition_topk_forward)
-            _check(
-                fwd(
-                    _ptr(rho), _ptr(src), _ptr(dst), _ptr(ps), _ptr(pv), _ptr(Ws), _ptr(Wt), _ptr(w), _ptr(bias),
-                    float(temperature), B, Ns, Nd, Dsrc, Ddst, Dv, *rank_arg, topk, compress,
-                    _ptr(ds), _ptr(dv), _ptr(sp), _ptr(dp), _ptr(idx), _ptr(logit), *([_ptr(head)] if mh else []),
-                    _ptr(ws), ws_bytes, _stream(dev),
-                )
-            )
-        ctx.save_for_backward(rho, src, dst, ps, pv, Ws, Wt, w, sp, dp, idx, logit, head)
+                heads: int = 1, bf16: bool = False, keep_routes: bool = True):
+        ds, dv, proj, idx, logit, head = _routes_forward(rho, src, dst, ps, pv, Ws, Wt, w, bias, float(temperature),
+                                                         int(topk), compress, heads, bf16, keep_routes)
+        ctx.save_for_backward(rho, src, dst, ps, pv, Ws, Wt, w, proj, idx, logit, head)
         ctx.meta = (float(temperature), int(topk), compress, bias is not None, heads, bf16)
+        ctx.set_materialize_grads(False)  # no zero-filled gradients for unused outputs
+        if not keep_routes:
+            return ds, dv
         ctx.mark_non_differentiable(idx, logit)
-        ctx.set_materialize_grads(False)  # no zero-filled gradients for the edge-list outputs
         return ds, dv, idx, logit
 
     @staticmethod
     def backward(ctx, g_ds, g_dv, _g_idx=None, _g_logit=None):
-        rho, src, dst, ps, pv, Ws, Wt, w, sp, dp, idx, logit, head = ctx.saved_tensors
+        rho, src, dst, ps, pv, Ws, Wt, w, proj, idx, logit, head = ctx.saved_tensors
         temperature, topk, compress, has_bias, heads, bf16 = ctx.meta
         B, Ns, Dsrc = src.shape
-        Nd, Ddst = dst.shape[1], dst.shape[2]
+        _, Nd, Ddst = dst.shape
         Dv = pv.shape[-1]
         r = Ws.shape[0]
         mh = heads > 1
-        rank_arg = [r // heads, heads] if mh else [r]
+        rank_arg = (r // heads, heads) if mh else (r,)
         dev = src.device
         need = ctx.needs_input_grad
         # the projected source state reaches delta_state only
         need_in = list(need[:5])
         need_in[3] = need_in[3] and g_ds is not None
-        with torch.cuda.device(dev):
+        with _on(dev):
             vdt = torch.bfloat16 if bf16 else torch.float32
-            g_ds = torch.zeros(B, Nd, device=dev) if g_ds is None else g_ds.float().contiguous()
+            g_ds = torch.zeros(B, Nd, device=dev) if g_ds is None else _f32(g_ds)
             g_dv = torch.zeros(B, Nd, Dv, device=dev, dtype=vdt) if g_dv is None else g_dv.to(vdt).contiguous()
             out = [torch.empty_like(t) if n else None for t, n in zip((rho, src, dst, ps, pv), need_in)]
             gWs = torch.empty_like(Ws) if need[5] else None
@@ -1135,17 +1294,20 @@ class _TransitionTopK(torch.autograd.Function):
             ws = torch.empty(max(ws_bytes, 1), device=dev, dtype=torch.uint8)
             bwd = (_LIB.jn_transition_topk_backward_multihead if mh else
                    _LIB.jn_transition_topk_backward_bf16 if bf16 else _LIB.jn_transition_topk_backward)
+            sp, idx_ptr = proj.data_ptr(), idx.data_ptr()
+            logit_ptr = logit.data_ptr() if logit is not None else idx_ptr + 4 * _pad64(B * Ns * min(topk, Nd))
             _check(
                 bwd(
-                    _ptr(rho), _ptr(src), _ptr(dst), _ptr(ps), _ptr(pv), _ptr(Ws), _ptr(Wt), _ptr(w),
-                    _ptr(sp), _ptr(dp), _ptr(idx), _ptr(logit), *([_ptr(head)] if mh else []), _ptr(g_ds), _ptr(g_dv),
-                    float(temperature), B, Ns, Nd, Dsrc, Ddst, Dv, *rank_arg, topk, compress,
-                    _ptr(out[0]), _ptr(out[1]), _ptr(out[2]), _ptr(out[3]), _ptr(out[4]), _ptr(gWs), _ptr(gWt),
-                    _ptr(gw), _ptr(gb), _ptr(ws), ws_bytes, _stream(dev),
+                    rho.data_ptr(), src.data_ptr(), dst.data_ptr(), ps.data_ptr(), pv.data_ptr(), Ws.data_ptr(),
+                    Wt.data_ptr(), w.data_ptr(), sp, sp + 4 * _pad64(B * Ns * r), idx_ptr, logit_ptr,
+                    *((head.data_ptr(),) if mh else ()), g_ds.data_ptr(), g_dv.data_ptr(),
+                    temperature, B, Ns, Nd, Dsrc, Ddst, Dv, *rank_arg, topk, compress,
+                    *(_ptr(o) for o in out), _ptr(gWs), _ptr(gWt), gw.data_ptr(), _ptr(gb), ws.data_ptr(), ws_bytes,
+                    _stream(dev),
                 )
             )
         return (*out, gWs, gWt, gw if need[7] else None, gb if (has_bias and need[8]) else None, None, None, None,
-                None, None)
+                None, None, None)
 
 
 def transition_pairwise_topk_routes(
@@ -1170,12 +1332,13 @@ def transition_pairwise_topk_routes(
     src_block_size: int,
     dst_block_size: int,
     route_compress_name: str = "softmax",
-) -> tuple[Tensor, Tensor, Tensor, Tensor]:
+    _keep_routes: bool = True,
+) -> tuple[Tensor, Tensor, Tensor | None, Tensor | None]:
     """Sparse transition returning (delta_state, delta_val, route_index, route_logit).
 
     Same arguments as ``transition_pairwise_topk``; route_index/route_logit
     [..., Ns, k] are each source's selected destinations (best first) and
-    their logits."""
+    their logits (None without ``_keep_routes``)."""
     if route_kind not in ("low_rank_bilinear_route", "multihead_max_low_rank_bilinear_route"):
         raise TypeError(f"jakal_net_native supports route kinds 'low_rank_bilinear_route' and "
                         f"'multihead_max_low_rank_bilinear_route', got {route_kind!r}.")
@@ -1197,7 +1360,7 @@ def transition_pairwise_topk_routes(
         raise RuntimeError("temperature must be positive.")
     _require_gpu(sender_strength, src_val, dst_val, projected_state, projected_val, source_weight, target_weight,
                  core_weight, bias)
-    batch_shape = tuple(src_val.shape[:-2])
+    batch_shape = src_val.shape[:-2]
     Ns, Dsrc = src_val.shape[-2], src_val.shape[-1]
     Nd, Ddst = dst_val.shape[-2], dst_val.shape[-1]
     Dv = projected_val.shape[-1]
@@ -1211,18 +1374,22 @@ def transition_pairwise_topk_routes(
     # bf16 layers keep bf16 value rows (one head); anything else computes in fp32
     bf16 = heads == 1 and _bf16_rows(src_val, dst_val, projected_val)
     rows = _bf16 if bf16 else _f32
-    ds, dv, idx, logit = _TransitionTopK.apply(
-        _f32(sender_strength.reshape(-1, Ns)), rows(src_val.reshape(-1, Ns, Dsrc)),
-        rows(dst_val.reshape(-1, Nd, Ddst)), _f32(projected_state.reshape(-1, Ns)),
-        rows(projected_val.reshape(-1, Ns, Dv)), _f32(source_weight), _f32(target_weight), _f32(core_weight),
-        _f32(bias), float(temperature), k, _ROUTE_COMPRESS_KINDS[route_compress_name], heads, bf16,
+    tensors = (
+        _f32(_rows(sender_strength, Ns)), rows(_rows(src_val, Ns, Dsrc)), rows(_rows(dst_val, Nd, Ddst)),
+        _f32(_rows(projected_state, Ns)), rows(_rows(projected_val, Ns, Dv)), _f32(source_weight),
+        _f32(target_weight), _f32(core_weight), _f32(bias),
     )
-    return (
-        ds.reshape(*batch_shape, Nd).to(projected_state.dtype),
-        dv.reshape(*batch_shape, Nd, Dv).to(projected_val.dtype),
-        idx.reshape(*batch_shape, Ns, k),
-        logit.reshape(*batch_shape, Ns, k),
-    )
+    rest = (float(temperature), k, _ROUTE_COMPRESS_KINDS[route_compress_name], heads, bf16, _keep_routes)
+    if _records(*tensors):
+        out = _TransitionTopK.apply(*tensors, *rest)
+    else:
+        ds, dv, _, idx, logit, _ = _routes_forward(*tensors, *rest)
+        out = (ds, dv, idx, logit)
+    ds = _like(out[0], batch_shape, projected_state.dtype)
+    dv = _like(out[1], batch_shape, projected_val.dtype)
+    if not _keep_routes:
+        return ds, dv, None, None
+    return ds, dv, out[2].reshape(*batch_shape, Ns, k), out[3].reshape(*batch_shape, Ns, k)
 
 
 def transition_pairwise_topk(
@@ -1288,7 +1455,7 @@ class _TransitionDense(torch.autograd.Function):
         r = Ws.shape[0]
         dev = src.device
         mh = heads > 1
-        with torch.cuda.device(dev):
+        with _on(dev):
             ds = torch.empty(B, Nd, device=dev, dtype=torch.float32)
             dv = torch.empty(B, Nd, Dv, device=dev, dtype=torch.bfloat16 if bf16 else torch.float32)
             sp = torch.empty(B * Ns, r, device=dev, dtype=torch.float32)
@@ -1324,7 +1491,7 @@ class _TransitionDense(torch.autograd.Function):
         # the projected source state reaches delta_state only
         need_in = list(need[:5])
         need_in[3] = need_in[3] and g_ds is not None
-        with torch.cuda.device(dev):
+        with _on(dev):
             vdt = torch.bfloat16 if bf16 else torch.float32
             g_ds = torch.zeros(B, Nd, device=dev) if g_ds is None else g_ds.float().contiguous()
             g_dv = torch.zeros(B, Nd, Dv, device=dev, dtype=vdt) if g_dv is None else g_dv.to(vdt).contiguous()
@@ -1422,8 +1589,8 @@ def transition_pairwise_dense(
     bf16 = (heads == 1 and _bf16_rows(src_val, dst_val, projected_val)
             and dense_transition_bf16_shapes_ok(Ns, Nd, Dv))
     rows = _bf16 if bf16 else _f32
-    ds, dv = _TransitionDense.apply(
-        _f32(sender_strength.reshape(-1, Ns)), rows(src_val.reshape(-1, Ns, Dsrc)),
+    ds, dv = _run(
+        _TransitionDense, _f32(sender_strength.reshape(-1, Ns)), rows(src_val.reshape(-1, Ns, Dsrc)),
         rows(dst_val.reshape(-1, Nd, Ddst)), _f32(projected_state.reshape(-1, Ns)),
         rows(projected_val.reshape(-1, Ns, Dv)), _f32(source_weight), _f32(target_weight), _f32(core_weight),
         _f32(bias), float(temperature), _ROUTE_COMPRESS_KINDS[route_compress_name], heads, bf16,
@@ -1456,7 +1623,7 @@ def low_rank_topk_select(
     score = torch.empty(B, Nq, topk, device=dev, dtype=torch.float32)
     sc = _f32(scale)
     bi = _f32(bias)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ws_bytes = int(_LIB.jn_lowrank_topk_select_workspace_bytes(B, Nk, r))
         ws = torch.empty(max(ws_bytes, 1), device=dev, dtype=torch.uint8)
         _check(
@@ -1522,7 +1689,7 @@ def softsign_backward_cuda(scores: Tensor, grad_edges: Tensor) -> Tensor:
     s = _raw_f32("scores", scores)
     g = _raw_f32("grad_edges", grad_edges)
     out = torch.empty(s.shape, device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _check(_LIB.jn_softsign_backward(_ptr(s), _ptr(g), s.numel(), _ptr(out), _stream(dev)))
     return out
 
@@ -1538,7 +1705,7 @@ def softmax_backward_cuda(routes: Tensor, grad_routes: Tensor) -> Tensor:
     out = torch.empty(p.shape, device=dev, dtype=torch.float32)
     rows, k = p.shape[0] * p.shape[1], p.shape[2]
     if rows and k:
-        with torch.cuda.device(dev):
+        with _on(dev):
             _check(_LIB.jn_softmax_backward(_ptr(p), _ptr(g), rows, k, _ptr(out), _stream(dev)))
     return out
 
@@ -1551,7 +1718,7 @@ def _edge_aggregate(index: Tensor, score: Tensor, compress: int, ps: Tensor, pv:
     dv = torch.empty(B, Nq, D, device=dev, dtype=torch.float32)
     if B * Nq * k == 0 or Ns == 0:
         return ds.zero_(), dv.zero_()
-    with torch.cuda.device(dev):
+    with _on(dev):
         _check(_LIB.jn_edge_aggregate(_ptr(index), _ptr(score), B, Nq, Ns, k, D, compress, _ptr(ps), _ptr(pv),
                                       _ptr(ds), _ptr(dv), _stream(dev)))
     return ds, dv
@@ -1605,7 +1772,7 @@ def query_topk_reduce_backward_cuda(edges: Tensor, indices: Tensor, projected_st
     g_pv = torch.empty(B, Ns, D, device=dev, dtype=torch.float32)
     if B * Nq * k == 0:
         return g_edges, g_ps.zero_(), g_pv.zero_()
-    with torch.cuda.device(dev):
+    with _on(dev):
         ws_bytes = int(_LIB.jn_edge_reduce_backward_workspace_bytes(B, Nq, Ns, k))
         if ws_bytes == 0:
             raise NotImplementedError("query_topk_reduce_backward_cuda: edge list too large for the edge grouping.")
@@ -1644,7 +1811,7 @@ def _raw_select(wps: Tensor, pt: Tensor, topk: int, score_bias: float, limit: in
     bias = torch.full((H,), float(score_bias), device=dev, dtype=torch.float32)
     idx = torch.empty(B, Nq, k, device=dev, dtype=torch.int32)
     score = torch.empty(B, Nq, k, device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ws_bytes = int(_LIB.jn_lowrank_topk_select_heads_workspace_bytes(B, Nk, rh, H))
         ws = torch.empty(max(ws_bytes, 1), device=dev, dtype=torch.uint8)
         _check(_LIB.jn_lowrank_topk_select_heads(_ptr(q), _ptr(kk), _ptr(bias), B, Nq, Nk, rh, H, k, _ptr(idx),
@@ -1703,7 +1870,7 @@ def low_rank_pairwise_topk_forward_cuda(weighted_projected_source: Tensor, proje
     ws_val = weighted_projected_val.contiguous()
     ds = torch.empty(B, Nd, device=dev, dtype=torch.float32)
     dv = torch.empty(B, Nd, D, device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ws_bytes = int(_LIB.jn_route_topk_aggregate_workspace_bytes(B, Ns, Nd, k))
         if ws_bytes == 0:
             raise NotImplementedError("low_rank_pairwise_topk_forward_cuda: route list too large for the grouping.")
@@ -1755,7 +1922,7 @@ def low_rank_pairwise_topk_backward_cuda(query_val: Tensor, source_val: Tensor, 
     g_q, g_s = torch.empty(B, Nq, Dq, **f32), torch.empty(B, Ns, Ds, **f32)
     g_ws, g_wt = torch.empty(r, Ds, **f32), torch.empty(r, Dq, **f32)
     g_w, g_b = torch.empty(r, **f32), torch.empty((), **f32)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ws_bytes = int(_LIB.jn_lowrank_pair_backward_workspace_bytes(B, Nq, Ns, Dq, Ds, r, k))
         if ws_bytes == 0:
             raise NotImplementedError("low_rank_pairwise_topk_backward_cuda: edge list too large for the grouping.")
