@@ -39,7 +39,7 @@ typedef void* jn_stream_t;
 /* Message of the last failing call on this host thread ("" if none). */
 const char* jn_last_error(void);
 
-/* ABI revision of this header (bumped on any signature or accepted-range change); this is 15. */
+/* ABI revision of this header (bumped on any signature or accepted-range change); this is 16. */
 int jn_abi_version(void);
 
 /*
@@ -684,6 +684,12 @@ int jn_propagation_dense_backward_bf16(
     int32_t projected_val_is_layer_val, int32_t reuse_edges, uint16_t* grad_layer_val, float* grad_projected_state,
     uint16_t* grad_projected_val, float* grad_target_weight, float* grad_source_weight, float* grad_core_weight,
     float* grad_bias, void* workspace, size_t workspace_bytes, jn_stream_t stream);
+/* 1 when the chunked bf16 entry points run a layer of these sizes without an
+ * edge matrix (softsign, out_dim a multiple of 128 up to 512, rank <= 64): the
+ * forward's workspace and the backward's edge_chunk (chunk_batch * nodes * nodes
+ * floats, both) are then scratch, hold no edges afterwards, and chunk_resident
+ * is ignored.  No counterpart in the reference. */
+int32_t jn_propagation_dense_edgeless_bf16(int64_t nodes, int64_t out_dim, int64_t rank, int32_t compress_kind);
 int jn_propagation_dense_forward_chunked_bf16(const uint16_t* layer_val, const float* projected_state,
                                               const uint16_t* projected_val, const float* target_weight,
                                               const float* source_weight, const float* core_weight, const float* bias,

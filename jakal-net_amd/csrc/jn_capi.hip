@@ -398,6 +398,27 @@ inline const float* value_rows(const float* p, int64_t e, bool bf16) {
   return bf16 ? reinterpret_cast<const float*>(reinterpret_cast<const bf16_t*>(p) + e) : p + e;
 }
 
+// Batch elements [b0, b0 + nb) of a bf16 dense layer for the kernels that build
+// no edge matrix (the outputs are the caller's to set).
+DenseFused dense_fused_range(const float* projected_state, const float* projected_val, const float* core_weight,
+                             const float* bias, const float* projections, int b0, int nb, int N, int D, int r,
+                             bool causal, void* scratch) {
+  const int64_t pr = (int64_t)b0 * N;
+  DenseFused f{};
+  f.projections = projections + pr * 2 * r;
+  f.core_weight = core_weight;
+  f.bias = bias;
+  f.projected_state = projected_state + pr;
+  f.projected_val = value_rows(projected_val, pr * D, true);
+  f.nb = nb;
+  f.N = N;
+  f.D = D;
+  f.r = r;
+  f.causal = causal;
+  f.scratch = scratch;
+  return f;
+}
+
 // Max-aggregated multi-head scores of batch elements [b0, b0 + nb)
 // (jakal_net_native.cpp:724-752): S = max_h (P_t,h diag(w_h) P_s,h^T + b_h)
 // over the heads' rank slices of the [N, 2r] projection rows (r = heads *
@@ -516,7 +537,27 @@ int dense_backward(const float* layer_val, const float* projected_state, const f
   const int upper = causal ? kCausalKUpper : kCausalKNone;  // A = E^T: A(j, i) = 0 for i < j
   float* gpv = projected_val_is_layer_val ? grad_layer_val : grad_projected_val;
   int rc;
-  const int nchunks = (B + chunk_batch - 1) / chunk_batch;
+  // a bf16 softsign layer whose forward kept no edges: nothing is rebuilt
+  const int64_t edgeless =
+      bf16 && recompute ? dense_fused_batch(B, N, D, r, compress_kind, (size_t)chunk_batch * N * N * sizeof(float)) : 0;
+  for (int b0 = 0; edgeless > 0 && b0 < B; b0 += (int)edgeless) {
+    const int nb = (int)std::min<int64_t>(edgeless, B - b0);
+    const int64_t pr = (int64_t)b0 * N;
+    DenseFused f = dense_fused_range(projected_state, projected_val, core_weight, bias, projections, b0, nb, N, D, r,
+                                     causal != 0, E);
+    f.grad_delta_state = grad_delta_state + pr;
+    f.grad_delta_val = value_rows(grad_delta_val, pr * D, true);
+    f.grad_projected_state = grad_projected_state ? grad_projected_state + pr : nullptr;
+    f.grad_projected_val = gpv ? const_cast<float*>(value_rows(gpv, pr * D, true)) : nullptr;
+    f.dP = s.dP + pr * 2 * r;
+    f.rowsum = s.rowsum + pr;
+    rc = launch_dense_fused_backward(f, st);
+    if (rc) return rc;
+    rc = launch_scale_grad_partials(s.dP + pr * 2 * r + r, 2 * r, projections + pr * 2 * r + r, 2 * r, core_weight, r,
+                                    (int64_t)nb * N, s.part_c + pr * r, st);
+    if (rc) return rc;
+  }
+  const int nchunks = edgeless > 0 ? 0 : (B + chunk_batch - 1) / chunk_batch;
   for (int c = nchunks - 1; c >= 0; --c) {
     const int b0 = c * chunk_batch;
     const int nb = std::min(chunk_batch, B - b0);
@@ -622,7 +663,7 @@ int dense_backward(const float* layer_val, const float* projected_state, const f
                                     (int64_t)nb * N, s.part_c + pr * r, st);
     if (rc) return rc;
   }
-  const int64_t n_rowsum = fused ? (int64_t)M * parts : M;
+  const int64_t n_rowsum = fused && edgeless == 0 ? (int64_t)M * parts : M;
 
   // 4. projection weight and input grads
   if (grad_target_weight && grad_source_weight) {
@@ -1220,7 +1261,7 @@ extern "C" {
 
 const char* jn_last_error(void) { return jakal::last_error(); }
 
-int jn_abi_version(void) { return 15; }
+int jn_abi_version(void) { return 16; }
 
 int jn_unit_scale_forward(const float* weight, int64_t rows, int64_t rank, float eps, float* weight_hat,
                           jn_stream_t stream) {
@@ -2159,6 +2200,10 @@ int jn_propagation_dense_backward_bf16(
       grad_bias, workspace, workspace_bytes, static_cast<hipStream_t>(stream), true);
 }
 
+int32_t jn_propagation_dense_edgeless_bf16(int64_t nodes, int64_t out_dim, int64_t rank, int32_t compress_kind) {
+  return dense_fused_batch(1, nodes, out_dim, rank, compress_kind, (size_t)nodes * nodes * sizeof(float)) > 0 ? 1 : 0;
+}
+
 size_t jn_propagation_dense_chunked_workspace_bytes(int64_t batch, int64_t nodes, int64_t in_dim, int64_t out_dim,
                                                     int64_t rank, int32_t compress_kind, int64_t chunk_batch,
                                                     int32_t backward) {
@@ -2191,6 +2236,18 @@ static int propagation_dense_forward_chunked_impl(
   rc = gemm_project(layer_val, in_dim, target_weight, source_weight, r, in_dim, projections, 2 * r, B * N, 2 * r,
                     (int)in_dim, st, bf16);
   if (rc) return rc;
+  if (bf16) {
+    const int64_t nb = dense_fused_batch(B, N, D, r, compress_kind, (size_t)cb * N * N * sizeof(float));
+    for (int b0 = 0; nb > 0 && b0 < B; b0 += (int)nb) {
+      DenseFused f = dense_fused_range(projected_state, projected_val, core_weight, bias, projections, b0,
+                                       (int)std::min<int64_t>(nb, B - b0), N, D, r, causal != 0, E);
+      f.delta_state = delta_state + (int64_t)b0 * N;
+      f.delta_val = const_cast<float*>(value_rows(delta_val, (int64_t)b0 * N * D, true));
+      rc = launch_dense_fused_forward(f, st);
+      if (rc) return rc;
+    }
+    if (nb > 0) return kOk;
+  }
   for (int b0 = 0; b0 < B; b0 += cb) {
     rc = dense_forward_range(projected_state, projected_val, core_weight, bias, b0, std::min(cb, B - b0), N, D, r,
                              compress_kind, causal != 0, projections, E, delta_state, delta_val, st, 1, nullptr,

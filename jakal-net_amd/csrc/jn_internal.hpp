@@ -1,6 +1,8 @@
 // Launch interfaces shared between the kernel translation units and the C ABI.
 #pragma once
 
+#include <algorithm>
+
 #include "jn_common.hpp"
 
 namespace jakal {
@@ -378,6 +380,34 @@ int launch_head_rowsum(const float* G, const uint8_t* head, int N, int64_t ld, i
 // out[b, j] = sum_i M[b, i, j] a[b, i] (c[b, i] if given), i < Nr, j < Nc, fixed order
 int launch_colsum_rows(const float* M, const float* a, const float* c, int B, int Nr, int Nc, float* out,
                        const char* name, hipStream_t stream);
+
+// bf16 dense softsign layers of one head without an edge matrix
+// (jn_dense_fused.hip), nb batch elements at a time.
+struct DenseFused {
+  const float* projections;  // [nb][N] rows of 2 r: targets, sources
+  const float* core_weight;  // [r]
+  const float* bias;         // scalar or null
+  const float* projected_state;   // [nb][N]
+  const void* projected_val;      // [nb][N][D] bf16
+  int nb, N, D, r;
+  bool causal;
+  void* scratch;             // the operand layouts (dense_fused_batch)
+  // forward
+  float* delta_state;
+  void* delta_val;
+  // backward
+  const float* grad_delta_state;
+  const void* grad_delta_val;     // bf16
+  float* grad_projected_state;    // or null
+  void* grad_projected_val;       // bf16, or null
+  float* dP;                      // [nb][N] rows of 2 r: w_hat (G P_s), G^T P_t
+  float* rowsum;                  // [nb][N] sums of G
+};
+// Batch elements per launch of these kernels with that much scratch; 0 where
+// they do not apply (the edge matrix is then built).
+int64_t dense_fused_batch(int64_t batch, int64_t N, int64_t D, int64_t r, int compress_kind, size_t scratch_bytes);
+int launch_dense_fused_forward(const DenseFused& f, hipStream_t stream);
+int launch_dense_fused_backward(const DenseFused& f, hipStream_t stream);
 
 // ---- dense transitions (jn_route_dense.hip) --------------------------------
 int launch_route_dense_compress(float* L, const float* bias, float inv_temp, int B, int Ns, int Nd, int kind,

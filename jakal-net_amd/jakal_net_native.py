@@ -130,6 +130,7 @@ _declare(
      _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P],
 )
 
+_declare("jn_propagation_dense_edgeless_bf16", [_I64, _I64, _I64, _I32], _I32)
 _declare("jn_propagation_dense_multihead_chunk_bytes", [_I64] * 3, _SZ)
 _declare("jn_propagation_dense_multihead_workspace_bytes", [_I64] * 6 + [_I32, _I64], _SZ)
 _declare(
@@ -727,11 +728,13 @@ class _PropagationDense(torch.autograd.Function):
         dev = X.device
         edge_bytes = N * N * 4
         chunk = B if B * edge_bytes <= DENSE_EDGE_BYTES else max(1, DENSE_EDGE_BYTES // edge_bytes)
+        # a bf16 softsign layer builds no edges: the chunk buffer is scratch
+        edgeless = bf16 and _LIB.jn_propagation_dense_edgeless_bf16(N, Dout, r, compress) == 1
         with _on(dev):
             ds = torch.empty(B, N, device=dev, dtype=torch.float32)
             dv = torch.empty(B, N, Dout, device=dev, dtype=torch.bfloat16 if bf16 else torch.float32)
             proj = torch.empty(B * N, 2 * r, device=dev, dtype=torch.float32)
-            if chunk >= B:
+            if chunk >= B and not edgeless:
                 edges = torch.empty(B, N, N, device=dev, dtype=torch.float32)
                 _check(
                     _PropagationDense._entry("jn_propagation_dense_forward", bf16)(
@@ -754,7 +757,7 @@ class _PropagationDense(torch.autograd.Function):
                 )
         ctx.save_for_backward(X, ps, pv_t, V, U, w_hat, proj, edges, bias)
         ctx.meta = (compress, pv_is_x, bias is not None, bool(causal), chunk, bool(bf16))
-        ctx.edges_consumed = False
+        ctx.edges_consumed = edgeless
         ctx.set_materialize_grads(False)  # an unused delta_state arrives as None
         return ds, dv
 
