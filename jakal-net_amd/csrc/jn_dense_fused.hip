@@ -20,8 +20,9 @@
 // has a fixed order.
 //
 // Measured at C4 sizes (16 x 4096 nodes, 512 values, rank 64, forward and
-// backward): 5.50 -> 3.27 ms against the GEMMs over edge matrices in two batch
-// chunks; aggregate 0.54 and 0.48 ms, score gradient 1.03 and 0.99 ms.
+// backward) against the GEMMs over edge matrices in two batch chunks: step 5.48
+// -> 2.85 ms; aggregate 0.42 and 0.41 ms (0.46 MFMA busy), score gradient 0.90
+// and 0.89 ms (0.31 MFMA busy).
 //
 // The split operands are laid out by dense_planes_kernel and dense_pack_kernel
 // before: rows of three 64-rank planes, their transposes in blocks of 32 rows,
@@ -33,18 +34,27 @@ namespace jakal {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // (arrays of uint4 in flight go through scratch memory)
 
-constexpr int kDfRows = 128;             // rows of a workgroup
-constexpr int kDfThreads = 512;          // 8 waves: 4 row groups of 32 x 2 column groups
+constexpr int kDfRows = 128;             // rows of an aggregate workgroup
+constexpr int kDfThreads = 512;          // 8 waves of 16 rows (scores) or D / 8 columns (E . V)
+constexpr int kDfGradRows = 64;          // rows of a score-gradient workgroup
+constexpr int kDfGradThreads = 256;      // 4 waves: 2 row groups of 32 x 2 column groups of 16
 constexpr int kDfRank = 64;              // ranks of a plane row (zeros past the rank)
-constexpr int kDfPlaneRow = 3 * kDfRank; // elements of a plane row: h, m, l
+constexpr int kDfPlaneRow = 3 * kDfRank; // elements of a row's planes: h, m, l
+constexpr int kDfFrag = 512;             // elements of an MFMA fragment: 64 lanes of 8
 
 // ---- operand layouts -----------------------------------------------------------
 
-// Rows [b][j] of one projection (stride ld, r ranks) times scale (or 1) into
-// planes [b][Npad][3][64], and unscaled into the transposed blocks
-// [b][Npad / 32][3][64 ranks][32 rows].  A workgroup takes 32 rows; blockIdx.z
-// picks the projection (0: targets, scaled planes; 1: sources).
+// Rows [b][j] of one projection (stride ld, r ranks) into three-term planes in
+// MFMA fragment order, so that a wave's fragment is one contiguous kilobyte in
+// global memory and in LDS (no bank conflicts):
+//   planes [b][Npad / 16][2][3][64 lanes][8]: rows times scale (or 1); lane l of
+//     a 16-row tile holds ranks 32 s + 8 (l / 16) .. + 7 of row l % 16;
+//   blocks [b][Npad / 32][4][3][64 lanes][8]: transposed, unscaled; lane l of a
+//     16-rank tile holds rows 8 (l / 16) .. + 7 of rank l % 16.
+// A workgroup takes 32 rows; blockIdx.z picks the projection (0: targets, with
+// the scale; 1: sources).
 struct DensePlanesArgs {
   const float* proj[2];
   int64_t ld;
@@ -53,6 +63,20 @@ struct DensePlanesArgs {
   bf16_t* blocks[2];   // or null
   int N, Npad, r;
 };
+
+// eight values into one lane's piece of the h, m and l fragments at `to`
+__device__ __forceinline__ void df_store_planes(const float (&x)[8], bf16_t* to) {
+  uint32_t h[8], m[8], l[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x3_split(__float_as_uint(x[i]), h[i], m[i], l[i]);
+  auto put = [&](int plane, const uint32_t(&v)[8]) {
+    *reinterpret_cast<uint4*>(to + plane * kDfFrag) =
+        make_uint4(x3_pair(v[0], v[1]), x3_pair(v[2], v[3]), x3_pair(v[4], v[5]), x3_pair(v[6], v[7]));
+  };
+  put(0, h);
+  put(1, m);
+  put(2, l);
+}
 
 __global__ __launch_bounds__(256) void dense_planes_kernel(DensePlanesArgs a) {
   __shared__ float tile[32][kDfRank + 1];
@@ -63,34 +87,23 @@ __global__ __launch_bounds__(256) void dense_planes_kernel(DensePlanesArgs a) {
     tile[j][k] = j0 + j < a.N && k < a.r ? src[(int64_t)j * a.ld + k] : 0.f;
   }
   __syncthreads();
-  // two elements (k, k + 1) of a row, or (j, j + 1) of a transposed block, per step
-  uint32_t* planes = reinterpret_cast<uint32_t*>(a.planes[z] + ((int64_t)b * a.Npad + j0) * kDfPlaneRow);
-  for (int e = tid; e < 32 * kDfRank / 2; e += 256) {
-    const int j = e / (kDfRank / 2), k = e % (kDfRank / 2) * 2;
-    float x0 = tile[j][k], x1 = tile[j][k + 1];
-    if (z == 0) {
-      x0 *= k < a.r ? a.scale[k] : 0.f;
-      x1 *= k + 1 < a.r ? a.scale[k + 1] : 0.f;
+  const int64_t base = ((int64_t)b * a.Npad + j0) * kDfPlaneRow;
+  float x[8];
+  {  // thread: row j, ranks k .. k + 7
+    const int j = tid / 8, k = tid % 8 * 8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      x[i] = tile[j][k + i];
+      if (z == 0) x[i] *= k + i < a.r ? a.scale[k + i] : 0.f;
     }
-    uint32_t h[2], m[2], l[2];
-    x3_split(__float_as_uint(x0), h[0], m[0], l[0]);
-    x3_split(__float_as_uint(x1), h[1], m[1], l[1]);
-    uint32_t* to = planes + (j * kDfPlaneRow + k) / 2;
-    to[0] = x3_pair(h[0], h[1]);
-    to[kDfRank / 2] = x3_pair(m[0], m[1]);
-    to[kDfRank] = x3_pair(l[0], l[1]);
+    df_store_planes(x, a.planes[z] + base + ((j / 16 * 2 + k / 32) * 3 * 64 + j % 16 + k % 32 / 8 * 16) * 8);
   }
   if (!a.blocks[z]) return;
-  uint32_t* blocks = reinterpret_cast<uint32_t*>(a.blocks[z] + ((int64_t)b * a.Npad + j0) * kDfPlaneRow);
-  for (int e = tid; e < 32 * kDfRank / 2; e += 256) {
-    const int k = e / 16, j = e % 16 * 2;
-    uint32_t h[2], m[2], l[2];
-    x3_split(__float_as_uint(tile[j][k]), h[0], m[0], l[0]);
-    x3_split(__float_as_uint(tile[j + 1][k]), h[1], m[1], l[1]);
-    uint32_t* to = blocks + (k * 32 + j) / 2;
-    to[0] = x3_pair(h[0], h[1]);
-    to[kDfRank * 16] = x3_pair(m[0], m[1]);
-    to[kDfRank * 32] = x3_pair(l[0], l[1]);
+  {  // thread: rank k, rows j .. j + 7
+    const int k = tid / 4, j = tid % 4 * 8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = tile[j + i][k];
+    df_store_planes(x, a.blocks[z] + base + (k / 16 * 3 * 64 + k % 16 + j / 8 * 16) * 8);
   }
 }
 
@@ -138,23 +151,24 @@ __device__ __forceinline__ floatx4 mfma_x3(const bf16x8v (&a)[3], const bf16x8v 
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], c, 0, 0, 0);
 }
 
-// whether row i keeps column j (kDfAll; kDfLower: j <= i; kDfUpper: j >= i)
+// which columns j row i keeps: all, j <= i, j >= i.  Causal kernels test without
+// a branch (a branch per element splits the schedule of a whole step).
 constexpr int kDfAll = 0, kDfLower = 1, kDfUpper = 2;
 __device__ __forceinline__ bool df_keep(int mode, int i, int j) {
-  return mode == kDfAll || (mode == kDfLower ? j <= i : j >= i);
+  return (mode == kDfLower ? i - j : j - i) >= 0;
 }
 
 // the workgroup's batch element and first row (longest column ranges first)
-__device__ __forceinline__ void df_tile(int Npad, int mode, int& b, int& i0) {
-  const int id = xcd_swizzle(blockIdx.x, gridDim.x), per = Npad / kDfRows;
+__device__ __forceinline__ void df_tile(int Npad, int rows, int mode, int& b, int& i0) {
+  const int id = xcd_swizzle(blockIdx.x, gridDim.x), per = Npad / rows;
   b = id / per;
   const int t = id - b * per;
-  i0 = (mode == kDfLower ? per - 1 - t : t) * kDfRows;
+  i0 = (mode == kDfLower ? per - 1 - t : t) * rows;
 }
 
 // ---- E . V and E . x ---------------------------------------------------------------
 struct DenseAggregateArgs {
-  const bf16_t* rows;    // planes of the row operand [nb][Npad][3][64]
+  const bf16_t* rows;    // planes of the row operand (dense_planes_kernel)
   const bf16_t* cols;    // planes of the column operand
   const bf16_t* values;  // packed values of the columns (dense_pack_kernel)
   const float* bias;     // scalar or null
@@ -166,50 +180,44 @@ struct DenseAggregateArgs {
 
 // 64 columns per step.  Scores are taken transposed (columns on M, rows on N),
 // so that a lane holds four consecutive columns of one row: its edges go to LDS
-// as 8-byte pieces and come back as the B operand of the aggregate, whose A
-// operand (the packed values: every wave owns D / 8 columns of V) loads straight
-// into fragments.  Two buffers each for the column planes and the edges: one
-// barrier per step, and a wave may run its scores beside another's aggregate.
+// as 8-byte pieces of the aggregate's B fragments, whose A operand (the packed
+// values: every wave owns D / 8 columns of V) loads straight into fragments.
+// Two buffers each for the column planes and the edges: one barrier per step,
+// and a wave may run its scores beside another's aggregate.
 // Bound: MFMA (per 128 x 64 edges and SIMD 1536 cycles of scores, 2048 of
 // aggregate at D = 512) plus the softsign's VALU work.
-template <int NTW, int KS>
+template <int NTW, int KS, bool CAUSAL>
 __global__ __launch_bounds__(kDfThreads) void dense_aggregate_kernel(DenseAggregateArgs a) {
-  constexpr int CT = 64, SB = CT * 2 + 16;  // bytes of an LDS row of 64 bf16
-  constexpr int PB = CT * SB, EB = kDfRows * SB;
-  __shared__ __align__(16) char planes[2][3 * PB];
-  __shared__ __align__(16) char edges[2][EB];
-  __shared__ float state[2][kDfRows];
+  constexpr int CT = 64;
+  __shared__ __align__(16) bf16_t planes[2][CT * kDfPlaneRow];  // [4 tiles][2][3] fragments
+  __shared__ __align__(16) bf16_t edges[2][16 * kDfFrag];       // [8 row tiles][2] fragments
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
-  const int wr = wave >> 1, wc = wave & 1, col = lane & 15, kg = lane >> 4;
+  const int col = lane & 15, kg = lane >> 4;
   int b, i0;
-  df_tile(a.Npad, a.mode, b, i0);
+  df_tile(a.Npad, kDfRows, a.mode, b, i0);
   const int jbeg = a.mode == kDfUpper ? i0 : 0;
   const int jend = a.mode == kDfLower ? min(a.N, i0 + kDfRows) : a.N;
   const float bias = a.bias ? a.bias[0] : 0.f;
 
-  bf16x8v q[2][KS][3];  // this wave's 32 rows
+  const int row = wave * 16 + col;  // of the scores
+  bf16x8v q[KS][3];
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int s = 0; s < KS; ++s)
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int p = 0; p < 3; ++p)
-        q[t][s][p] = *reinterpret_cast<const bf16x8v*>(
-            a.rows + ((int64_t)b * a.Npad + i0 + wr * 32 + t * 16 + col) * kDfPlaneRow + p * kDfRank + s * 32 + kg * 8);
+    for (int p = 0; p < 3; ++p)
+      q[s][p] = *reinterpret_cast<const bf16x8v*>(
+          a.rows + ((int64_t)b * a.Npad + i0 + wave * 16) * kDfPlaneRow + (s * 3 + p) * kDfFrag + lane * 8);
 
-  const uint4* cols = reinterpret_cast<const uint4*>(a.cols + (int64_t)b * a.Npad * kDfPlaneRow);
+  const u32x4* cols = reinterpret_cast<const u32x4*>(a.cols + (int64_t)b * a.Npad * kDfPlaneRow);
   const auto rs_x = make_rsrc(a.x + (int64_t)b * a.N, (uint32_t)a.N * 4u);
-  uint4 stage[3];
-  auto load = [&](int j0) {  // 64 plane rows are 24 KB in one piece
+  u32x4 stage[3];
+  auto load = [&](int j0) {  // the planes of 64 rows are 24 KB in one piece
 #pragma unroll
     for (int u = 0; u < 3; ++u) stage[u] = cols[(int64_t)j0 * (kDfPlaneRow / 8) + tid + kDfThreads * u];
   };
   auto store = [&](int buf) {
 #pragma unroll
-    for (int u = 0; u < 3; ++u) {
-      const int e = tid + kDfThreads * u, j = e / 24, p = e % 24;
-      *reinterpret_cast<uint4*>(&planes[buf][(p >> 3) * PB + j * SB + (p & 7) * 16]) = stage[u];
-    }
+    for (int u = 0; u < 3; ++u) reinterpret_cast<u32x4*>(planes[buf])[tid + kDfThreads * u] = stage[u];
   };
 
   floatx4 acc[NTW][8];
@@ -217,7 +225,7 @@ __global__ __launch_bounds__(kDfThreads) void dense_aggregate_kernel(DenseAggreg
   for (int d = 0; d < NTW; ++d)
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[d][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float rsum[2] = {0.f, 0.f};
+  float rsum = 0.f;
 
   load(jbeg);
   store(0);
@@ -226,46 +234,38 @@ __global__ __launch_bounds__(kDfThreads) void dense_aggregate_kernel(DenseAggreg
   for (int j0 = jbeg; j0 < jend; j0 += CT, buf ^= 1) {
     const bool more = j0 + CT < jend;
     if (more) load(j0 + CT);
-    bf16x8v v[NTW];
-    auto load_values = [&](int s) {
+    bf16x8v v[2][NTW];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int d = 0; d < NTW; ++d)
-        v[d] = *reinterpret_cast<const bf16x8v*>(
+        v[s][d] = *reinterpret_cast<const bf16x8v*>(
             a.values + (((int64_t)b * (a.Npad / 32) + j0 / 32 + s) * (a.D / 16) + wave * NTW + d) * 512 + lane * 8);
-    };
-    load_values(0);
-    float4 x[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) x[t] = buf_load4(rs_x, (uint32_t)(j0 + wc * 32 + t * 16 + kg * 4) * 4u);
 
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {  // 16 columns
-      bf16x8v c[KS][3];
+    for (int t = 0; t < 4; ++t) {  // 16 columns
+      const int j = t * 16 + kg * 4;
+      const float4 x = buf_load4(rs_x, (uint32_t)(j0 + j) * 4u);
+      floatx4 sc = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s < KS; ++s)
+      for (int s = 0; s < KS; ++s) {
+        bf16x8v c[3];
 #pragma unroll
         for (int p = 0; p < 3; ++p)
-          c[s][p] = *reinterpret_cast<const bf16x8v*>(&planes[buf][p * PB + (wc * 32 + t * 16 + col) * SB + s * 64 +
-                                                                  kg * 16]);
-      floatx4 sc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-      for (int s = 0; s < KS; ++s)
-#pragma unroll
-        for (int n = 0; n < 2; ++n) sc[n] = mfma_x3(c[s], q[n][s], sc[n]);
-#pragma unroll
-      for (int n = 0; n < 2; ++n) {
-        const int i = wr * 32 + n * 16 + col, j = wc * 32 + t * 16 + kg * 4;
-        float e[4];
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const float s = sc[n][w] + bias;
-          e[w] = s * recip_f(1.0f + fabsf(s));
-          if (a.mode != kDfAll && !df_keep(a.mode, i0 + i, j0 + j + w)) e[w] = 0.f;
-        }
-        rsum[n] += (e[0] * x[t].x + e[1] * x[t].y) + (e[2] * x[t].z + e[3] * x[t].w);
-        *reinterpret_cast<uint2*>(&edges[buf][i * SB + j * 2]) =
-            make_uint2(pack_bf16x2(e[0], e[1]), pack_bf16x2(e[2], e[3]));
+          c[p] = *reinterpret_cast<const bf16x8v*>(&planes[buf][((t * 2 + s) * 3 + p) * kDfFrag + lane * 8]);
+        sc = mfma_x3(c, q[s], sc);
       }
+      float e[4];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float s = sc[w] + bias;
+        e[w] = s * recip_f(1.0f + fabsf(s));
+        if constexpr (CAUSAL) e[w] = df_keep(a.mode, i0 + row, j0 + j + w) ? e[w] : 0.f;
+      }
+      rsum += (e[0] * x.x + e[1] * x.y) + (e[2] * x.z + e[3] * x.w);
+      *reinterpret_cast<uint2*>(&edges[buf][(wave * 2 + t / 2) * kDfFrag + (col + (t % 2 * 2 + kg / 2) * 16) * 8 +
+                                            kg % 2 * 4]) =
+          make_uint2(pack_bf16x2(e[0], e[1]), pack_bf16x2(e[2], e[3]));
     }
     if (more) store(buf ^ 1);
     __syncthreads();
@@ -273,41 +273,34 @@ __global__ __launch_bounds__(kDfThreads) void dense_aggregate_kernel(DenseAggreg
     for (int s = 0; s < 2; ++s) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const bf16x8v e = *reinterpret_cast<const bf16x8v*>(&edges[buf][(i * 16 + col) * SB + s * 64 + kg * 16]);
+        const bf16x8v e = *reinterpret_cast<const bf16x8v*>(&edges[buf][(i * 2 + s) * kDfFrag + lane * 8]);
 #pragma unroll
-        for (int d = 0; d < NTW; ++d) acc[d][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[d], e, acc[d][i], 0, 0, 0);
+        for (int d = 0; d < NTW; ++d)
+          acc[d][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[s][d], e, acc[d][i], 0, 0, 0);
       }
-      if (s == 0) load_values(1);
     }
   }
 
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const int row = i0 + i * 16 + col;
-    if (row >= a.N || !a.out) continue;
-    bf16_t* out = a.out + ((int64_t)b * a.N + row) * a.D + wave * NTW * 16 + kg * 4;
+    const int m = i0 + i * 16 + col;
+    if (m >= a.N || !a.out) continue;
+    bf16_t* out = a.out + ((int64_t)b * a.N + m) * a.D + wave * NTW * 16 + kg * 4;
 #pragma unroll
     for (int d = 0; d < NTW; ++d)
       *reinterpret_cast<uint2*>(out + d * 16) =
           make_uint2(pack_bf16x2(acc[d][i][0], acc[d][i][1]), pack_bf16x2(acc[d][i][2], acc[d][i][3]));
   }
-  if (!a.out_state) return;
-#pragma unroll
-  for (int n = 0; n < 2; ++n) {
-    float s = rsum[n];
-    s += xor16_f(s);
-    s += xor32_f(s);
-    if (kg == 0) state[wc][wr * 32 + n * 16 + col] = s;
-  }
-  __syncthreads();
-  if (tid < kDfRows && i0 + tid < a.N) a.out_state[(int64_t)b * a.N + i0 + tid] = state[0][tid] + state[1][tid];
+  rsum += xor16_f(rsum);
+  rsum += xor32_f(rsum);
+  if (a.out_state && kg == 0 && i0 + row < a.N) a.out_state[(int64_t)b * a.N + i0 + row] = rsum;
 }
 
 // ---- G . P ---------------------------------------------------------------------------
 struct DenseScoreGradArgs {
-  const bf16_t* rows;     // planes of the row operand [nb][Npad][3][64]
+  const bf16_t* rows;     // planes of the row operand (dense_planes_kernel)
   const bf16_t* cols;     // planes of the column operand
-  const bf16_t* blocks;   // transposed planes of the columns' raw projections [nb][Npad / 32][3][64][32]
+  const bf16_t* blocks;   // transposed planes of the columns' raw projections
   const bf16_t* row_val;  // [nb][N][D]
   const bf16_t* col_val;  // [nb][N][D]
   const float* row_x;     // [nb][N]
@@ -321,31 +314,28 @@ struct DenseScoreGradArgs {
 };
 
 // 32 columns per step, everything transposed as above.  The rows' value
-// fragments stay in registers (2 x D / 32 fragments), their score planes in
-// LDS; the columns' values, planes and transposed planes are staged per step.
+// fragments stay in registers (2 x D / 32 of them), their score planes in LDS;
+// the columns' values are staged in LDS (pieces of a row exchanged by its row
+// number, so that 16 rows' pieces lie in distinct banks), the columns' planes
+// and transposed planes load straight into fragments.  64 rows per workgroup:
+// 70 KB of LDS, so that two share a CU and one's barriers and LDS phases run
+// beside the other's MFMAs (128 rows in one workgroup of eight waves: 1.03 ms
+// against 0.90 at C4; in one of four waves of 32 x 32: 1.6).
 // Bound: MFMA (per 128 x 32 pairs and SIMD 768 cycles of scores, 1024 of
 // gdv . pv^T at D = 512, 768 of G . P), the VALU work of the derivative and of
-// splitting G, and LDS reads (2950 cycles) side by side.
-template <int NK, int KS>
-__global__ __launch_bounds__(kDfThreads) void dense_score_grad_kernel(DenseScoreGradArgs a) {
+// splitting G, and LDS reads (2200 cycles).
+template <int NK, int KS, bool CAUSAL>
+__global__ __launch_bounds__(kDfGradThreads, 2) void dense_score_grad_kernel(DenseScoreGradArgs a) {
   constexpr int D = NK * 32, CT = 32;
-  constexpr int VB = D * 2 + 16;              // bytes of a staged value row
-  constexpr int SB = kDfRank * 2 + 16;        // of a plane row of 64 ranks
-  constexpr int TB = CT * 2 + 16;             // of a row of 32 columns (transposed planes, G)
-  constexpr int QB = kDfRows * SB, PB = CT * SB, KB = kDfRank * TB, GB = kDfRows * TB;
-  __shared__ __align__(16) char smem[3 * QB + CT * VB + 3 * PB + 3 * KB + 3 * GB];
-  static_assert(sizeof(smem) <= 160 * 1024, "LDS of one CU");
-  char* qs = smem;              // rows' planes
-  char* vals = qs + 3 * QB;     // columns' values
-  char* ps = vals + CT * VB;    // columns' planes
-  char* ts = ps + 3 * PB;       // columns' transposed planes
-  char* gs = ts + 3 * KB;       // planes of G
+  __shared__ __align__(16) bf16_t qs[kDfGradRows * kDfPlaneRow];   // rows' planes: [4 tiles][2][3] fragments
+  __shared__ __align__(16) bf16_t vals[CT * D];                    // columns' values: rows of swizzled pieces
+  __shared__ __align__(16) bf16_t gs[kDfGradRows / 16 * 3 * kDfFrag];  // G: [4 row tiles][3] fragments
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const int wr = wave >> 1, wc = wave & 1, col = lane & 15, kg = lane >> 4;
   int b, i0;
-  df_tile(a.Npad, a.mode, b, i0);
+  df_tile(a.Npad, kDfGradRows, a.mode, b, i0);
   const int jbeg = a.mode == kDfUpper ? i0 : 0;
-  const int jend = a.mode == kDfLower ? min(a.N, i0 + kDfRows) : a.N;
+  const int jend = a.mode == kDfLower ? min(a.N, i0 + kDfGradRows) : a.N;
   const float bias = a.bias ? a.bias[0] : 0.f;
 
   const auto rs_rv = make_rsrc(a.row_val + (int64_t)b * a.N * D, (uint32_t)a.N * (D * 2u));
@@ -353,7 +343,7 @@ __global__ __launch_bounds__(kDfThreads) void dense_score_grad_kernel(DenseScore
   const auto rs_rx = make_rsrc(a.row_x + (int64_t)b * a.N, (uint32_t)a.N * 4u);
   const auto rs_cx = make_rsrc(a.col_x + (int64_t)b * a.N, (uint32_t)a.N * 4u);
   auto load16 = [](__amdgpu_buffer_rsrc_t rs, uint32_t off) {
-    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
   };
 
   bf16x8v rv[2][NK];  // this wave's 32 rows of values
@@ -368,42 +358,21 @@ __global__ __launch_bounds__(kDfThreads) void dense_score_grad_kernel(DenseScore
   }
   {
     const uint4* src = reinterpret_cast<const uint4*>(a.rows + ((int64_t)b * a.Npad + i0) * kDfPlaneRow);
-    for (int e = tid; e < kDfRows * 24; e += kDfThreads) {
-      const int i = e / 24, p = e % 24;
-      *reinterpret_cast<uint4*>(qs + (p >> 3) * QB + i * SB + (p & 7) * 16) = src[e];
-    }
+    for (int e = tid; e < kDfGradRows * kDfPlaneRow / 8; e += kDfGradThreads) reinterpret_cast<uint4*>(qs)[e] = src[e];
   }
 
-  constexpr int VN = CT * D / 8 / kDfThreads;  // 16-byte pieces per thread of a value tile
-  const uint4* cols = reinterpret_cast<const uint4*>(a.cols + (int64_t)b * a.Npad * kDfPlaneRow);
-  const uint4* blocks = reinterpret_cast<const uint4*>(a.blocks + (int64_t)b * a.Npad * kDfPlaneRow);
-  uint4 sv[VN], sp[2], st[2];
+  constexpr int VN = CT * D / 8 / kDfGradThreads, VP = D / 8;  // 16-byte pieces: per thread of a tile, of a row
+  u32x4 sv[VN];
   auto load = [&](int j0) {
 #pragma unroll
     for (int u = 0; u < VN; ++u)
-      sv[u] = load16(rs_cv, (uint32_t)j0 * (D * 2u) + (uint32_t)(tid + kDfThreads * u) * 16u);
-    const int64_t at = (int64_t)j0 * (kDfPlaneRow / 8);  // 32 rows of planes, or a block: 768 pieces
-    sp[0] = cols[at + tid];
-    st[0] = blocks[at + tid];
-    if (tid < 256) {
-      sp[1] = cols[at + 512 + tid];
-      st[1] = blocks[at + 512 + tid];
-    }
+      sv[u] = load16(rs_cv, (uint32_t)j0 * (D * 2u) + (uint32_t)(tid + kDfGradThreads * u) * 16u);
   };
   auto store = [&]() {
 #pragma unroll
     for (int u = 0; u < VN; ++u) {
-      const int e = tid + kDfThreads * u;
-      *reinterpret_cast<uint4*>(vals + e / (D / 8) * VB + e % (D / 8) * 16) = sv[u];
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int e = tid + kDfThreads * u;
-      if (u == 0 || tid < 256) {
-        const int j = e / 24, p = e % 24;
-        *reinterpret_cast<uint4*>(ps + (p >> 3) * PB + j * SB + (p & 7) * 16) = sp[u];
-        *reinterpret_cast<uint4*>(ts + e / 256 * KB + e / 4 % 64 * TB + e % 4 * 16) = st[u];
-      }
+      const int e = tid + kDfGradThreads * u, j = e / VP, p = e % VP;
+      reinterpret_cast<u32x4*>(vals)[j * VP + (p ^ (j & 15))] = sv[u];
     }
   };
 
@@ -413,6 +382,8 @@ __global__ __launch_bounds__(kDfThreads) void dense_score_grad_kernel(DenseScore
 #pragma unroll
     for (int n = 0; n < 2; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
   float rsum[2] = {0.f, 0.f}, rpart[2] = {0.f, 0.f};
+  const bf16_t* cols = a.cols + (int64_t)b * a.Npad * kDfPlaneRow + lane * 8;
+  const bf16_t* blocks = a.blocks + (int64_t)b * a.Npad * kDfPlaneRow + lane * 8;
 
   load(jbeg);
   int step = 0;
@@ -422,69 +393,76 @@ __global__ __launch_bounds__(kDfThreads) void dense_score_grad_kernel(DenseScore
     __syncthreads();
     if (j0 + CT < jend) load(j0 + CT);
     const float4 cx = buf_load4(rs_cx, (uint32_t)(j0 + wc * 16 + kg * 4) * 4u);
+    bf16x8v c[KS][3];
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        c[s][p] = *reinterpret_cast<const bf16x8v*>(cols + (int64_t)(j0 + wc * 16) * kDfPlaneRow +
+                                                    (s * 3 + p) * kDfFrag);
 
-    // scores and gdv . pv^T: 16 columns (wc) x 32 rows
+    // gdv . pv^T and the scores: 16 columns (wc) x 32 rows
     floatx4 sc[2], gv[2];
 #pragma unroll
     for (int n = 0; n < 2; ++n) sc[n] = gv[n] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      bf16x8v c[3];
+    for (int s = 0; s < NK; ++s) {
+      const bf16x8v v =
+          reinterpret_cast<const bf16x8v*>(vals)[(wc * 16 + col) * VP + ((s * 4 + kg) ^ col)];
 #pragma unroll
-      for (int p = 0; p < 3; ++p)
-        c[p] = *reinterpret_cast<const bf16x8v*>(ps + p * PB + (wc * 16 + col) * SB + s * 64 + kg * 16);
+      for (int n = 0; n < 2; ++n) gv[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, rv[n][s], gv[n], 0, 0, 0);
+    }
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
 #pragma unroll
       for (int n = 0; n < 2; ++n) {
         bf16x8v q[3];
 #pragma unroll
         for (int p = 0; p < 3; ++p)
-          q[p] = *reinterpret_cast<const bf16x8v*>(qs + p * QB + (wr * 32 + n * 16 + col) * SB + s * 64 + kg * 16);
-        sc[n] = mfma_x3(c, q, sc[n]);
+          q[p] = *reinterpret_cast<const bf16x8v*>(&qs[(((wr * 2 + n) * 2 + s) * 3 + p) * kDfFrag + lane * 8]);
+        sc[n] = mfma_x3(c[s], q, sc[n]);
       }
-    }
+    bf16x8v t[2][3];
 #pragma unroll
-    for (int s = 0; s < NK; ++s) {
-      const bf16x8v c = *reinterpret_cast<const bf16x8v*>(vals + (wc * 16 + col) * VB + s * 64 + kg * 16);
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
-      for (int n = 0; n < 2; ++n) gv[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, rv[n][s], gv[n], 0, 0, 0);
-    }
+      for (int p = 0; p < 3; ++p)
+        t[m][p] = *reinterpret_cast<const bf16x8v*>(blocks + (int64_t)j0 * kDfPlaneRow +
+                                                    ((wc * 2 + m) * 3 + p) * kDfFrag);
     const float cxv[4] = {cx.x, cx.y, cx.z, cx.w};
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
-      const int i = wr * 32 + n * 16 + col, j = wc * 16 + kg * 4;
-      uint32_t h[4], m[4], l[4];
+      uint32_t h[4], mi[4], l[4];
       float g[4];
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
         const float d = recip_f(1.0f + fabsf(sc[n][w] + bias));  // 1 - |softsign|
         g[w] = (gv[n][w] + rx[n] * cxv[w]) * d * d;
-        if (a.mode != kDfAll && !df_keep(a.mode, i0 + i, j0 + j + w)) g[w] = 0.f;
-        x3_split(__float_as_uint(g[w]), h[w], m[w], l[w]);
+        if constexpr (CAUSAL)
+          g[w] = df_keep(a.mode, i0 + wr * 32 + n * 16 + col, j0 + wc * 16 + kg * 4 + w) ? g[w] : 0.f;
+        x3_split(__float_as_uint(g[w]), h[w], mi[w], l[w]);
       }
       rpart[n] += (g[0] + g[1]) + (g[2] + g[3]);
-      char* to = gs + i * TB + j * 2;
+      bf16_t* to = &gs[(wr * 2 + n) * 3 * kDfFrag + (col + (wc * 2 + kg / 2) * 16) * 8 + kg % 2 * 4];
       *reinterpret_cast<uint2*>(to) = make_uint2(x3_pair(h[0], h[1]), x3_pair(h[2], h[3]));
-      *reinterpret_cast<uint2*>(to + GB) = make_uint2(x3_pair(m[0], m[1]), x3_pair(m[2], m[3]));
-      *reinterpret_cast<uint2*>(to + 2 * GB) = make_uint2(x3_pair(l[0], l[1]), x3_pair(l[2], l[3]));
-      if ((step & 7) == 7) {  // short partial sums: their rounding does not grow with N
+      *reinterpret_cast<uint2*>(to + kDfFrag) = make_uint2(x3_pair(mi[0], mi[1]), x3_pair(mi[2], mi[3]));
+      *reinterpret_cast<uint2*>(to + 2 * kDfFrag) = make_uint2(x3_pair(l[0], l[1]), x3_pair(l[2], l[3]));
+    }
+    if ((step & 7) == 7) {  // short partial sums: their rounding does not grow with N
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
         rsum[n] += rpart[n];
         rpart[n] = 0.f;
       }
     }
     __syncthreads();
     // G . P: 32 ranks (wc) x 32 rows (wr) over the 32 columns
-    bf16x8v t[2][3];
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-#pragma unroll
-      for (int p = 0; p < 3; ++p)
-        t[m][p] = *reinterpret_cast<const bf16x8v*>(ts + p * KB + (wc * 32 + m * 16 + col) * TB + kg * 16);
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
       bf16x8v g[3];
 #pragma unroll
       for (int p = 0; p < 3; ++p)
-        g[p] = *reinterpret_cast<const bf16x8v*>(gs + p * GB + (wr * 32 + n * 16 + col) * TB + kg * 16);
+        g[p] = *reinterpret_cast<const bf16x8v*>(&gs[((wr * 2 + n) * 3 + p) * kDfFrag + lane * 8]);
 #pragma unroll
       for (int m = 0; m < 2; ++m) acc[m][n] = mfma_x3(t[m], g, acc[m][n]);
     }
@@ -505,16 +483,16 @@ __global__ __launch_bounds__(kDfThreads) void dense_score_grad_kernel(DenseScore
   }
   if (!a.rowsum) return;
   __syncthreads();  // the rows' planes are no longer read
-  float* state = reinterpret_cast<float*>(smem);
+  float* state = reinterpret_cast<float*>(qs);
 #pragma unroll
   for (int n = 0; n < 2; ++n) {
     float s = rsum[n] + rpart[n];
     s += xor16_f(s);
     s += xor32_f(s);
-    if (kg == 0) state[wc * kDfRows + wr * 32 + n * 16 + col] = s;
+    if (kg == 0) state[wc * kDfGradRows + wr * 32 + n * 16 + col] = s;
   }
   __syncthreads();
-  if (tid < kDfRows && i0 + tid < a.N) a.rowsum[(int64_t)b * a.N + i0 + tid] = state[tid] + state[kDfRows + tid];
+  if (tid < kDfGradRows && i0 + tid < a.N) a.rowsum[(int64_t)b * a.N + i0 + tid] = state[tid] + state[kDfGradRows + tid];
 }
 
 // ---- host ------------------------------------------------------------------------------
@@ -586,8 +564,11 @@ static int df_prepare(const DenseFused& f, const DenseLayouts& l, int Npad, cons
 template <int NTW>
 static void df_launch_aggregate(const DenseAggregateArgs& a, int nb, int r, hipStream_t stream) {
   const dim3 grid(nb * (a.Npad / kDfRows)), block(kDfThreads);
-  if (r <= 32) hipLaunchKernelGGL((dense_aggregate_kernel<NTW, 1>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((dense_aggregate_kernel<NTW, 2>), grid, block, 0, stream, a);
+  const bool causal = a.mode != kDfAll;
+  if (r <= 32 && causal) hipLaunchKernelGGL((dense_aggregate_kernel<NTW, 1, true>), grid, block, 0, stream, a);
+  else if (r <= 32) hipLaunchKernelGGL((dense_aggregate_kernel<NTW, 1, false>), grid, block, 0, stream, a);
+  else if (causal) hipLaunchKernelGGL((dense_aggregate_kernel<NTW, 2, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((dense_aggregate_kernel<NTW, 2, false>), grid, block, 0, stream, a);
 }
 
 static int df_aggregate(const DenseAggregateArgs& a, int nb, int r, const char* name, hipStream_t stream) {
@@ -604,7 +585,9 @@ static int df_aggregate(const DenseAggregateArgs& a, int nb, int r, const char* 
 
 template <int NK, int KS>
 static int df_launch_score_grad(const DenseScoreGradArgs& a, int nb, hipStream_t stream) {
-  hipLaunchKernelGGL((dense_score_grad_kernel<NK, KS>), dim3(nb * (a.Npad / kDfRows)), dim3(kDfThreads), 0, stream, a);
+  const dim3 grid(nb * (a.Npad / kDfGradRows)), block(kDfGradThreads);
+  if (a.mode != kDfAll) hipLaunchKernelGGL((dense_score_grad_kernel<NK, KS, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((dense_score_grad_kernel<NK, KS, false>), grid, block, 0, stream, a);
   JN_LAUNCH_CHECK();
   return kOk;
 }
