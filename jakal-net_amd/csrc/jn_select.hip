@@ -20,8 +20,8 @@
 //   * cooperative (rank <= 64, large grids): the workgroup stages each key
 //     chunk once in LDS and every wave reads its fragments from there, with a
 //     barrier per chunk and workgroup-wide merges (see the kernel template);
-//   * key-split (k <= 16, small grids): the four waves share 16 query rows,
-//     each over a quarter of the keys, merged by one sort per row at the end.
+//   * key-split (k <= 32, small grids): the four waves share 16 query rows,
+//     each over a quarter of the keys, merged by sorts per row at the end.
 //
 // Layout of one per-wave workgroup (256 threads = 4 waves, 64 query rows):
 //   * 16 query rows per wave.  A wave keeps the query fragment of its rows in
@@ -634,13 +634,13 @@ __device__ __forceinline__ halfx8 as_halfx8(float a, float b, float c, float d) 
 // merges after it, so a merge holds up no other wave at the next barrier.
 // CW = 4 is the same with 4 waves (64 rows) and one staging buffer (two
 // barriers per chunk), two workgroups per CU whose phases drift apart.
-// CW = -1 (k <= 16, small grids): the per-wave form with the four waves of a
+// CW = -1 (k <= 32, small grids): the per-wave form with the four waves of a
 // workgroup on the same 16 query rows, each over a quarter of the key chunks;
-// each keeps the exact top-k of its quarter, and a 64-entry sort per row
-// merges the four lists at the end.  Four times the workgroups and a quarter
-// of the serial chunk chain per wave.
-// MH (split keys, per-wave form only): multi-head max aggregation.  Head h owns
-// K-steps [h * head_ks, (h + 1) * head_ks) of the split rows; after a head's
+// each keeps the exact top-k of its quarter, and one 64-entry sort per row
+// (three for k > 16) merges the four lists at the end.  Four times the
+// workgroups and a quarter of the serial chunk chain per wave.
+// MH (split keys, per-wave and key-split forms): multi-head max aggregation.
+// Head h owns K-steps [h * head_ks, (h + 1) * head_ks) of the split rows; after a head's
 // last K-step its scores, unscaled and with its bias, are folded into a
 // running maximum, so the filter and merges see max_h (dot_h + bias[h]) / T.
 // BF (split layout, one plane): bf16 key rows and bf16 MFMAs (bf16 layers).
@@ -659,9 +659,9 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
   constexpr int RP = 32 * KS;                         // split row: ranks per plane
   constexpr int ROWS = COOP ? CW * kSelRowsPerWave : KSP ? kSelRowsPerWave : kSelRows;  // query rows per workgroup
   constexpr int SLOTS = COOP ? CW * kSelRowsPerWave : kSelRows;  // row slots (16 per wave)
-  static_assert(!KSP || KEEP == 48, "the key-split form serves k <= 16");
+  static_assert(!KSP || KEEP == 48, "the key-split form serves k <= 32");
   static_assert(!COOP || (KS >= 1 && KS <= 2), "the cooperative select stages split keys of rank <= 64");
-  static_assert(!MH || (SPLIT && CW == 0), "multi-head scores run on the per-wave split kernel");
+  static_assert(!MH || (SPLIT && CW <= 0), "multi-head scores run on the per-wave split kernels");
   static_assert(!BF || (SPLIT && !MH), "bf16 operands use the split layout with one head");
   // staged chunk: kSelChunk split rows of PLANES RP halves plus 8 halves of
   // padding, so the 16 rows one fragment read touches start 4 banks apart
@@ -1123,22 +1123,46 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
     __shared__ int s_kcnt[kSelRows];
     if (lane < kSelRowsPerWave) s_kcnt[wave * kSelRowsPerWave + lane] = kept;
     __syncthreads();
-    const int src = lane >> 4, e = lane & 15;
     for (int t = 0; t < kSelRowsPerWave / kSelWaves; ++t) {
       const int rcol = (kSelRowsPerWave / kSelWaves) * wave + t;
       const int row = row0 + rcol;
-      const int slot = src * kSelRowsPerWave + rcol;
-      float vs = -INFINITY;
-      int vi = 0x7fffffff;
-      if (e < s_kcnt[slot]) {
-        vs = key_to_float(s_kept_k[slot * KST + e]);
-        vi = s_kept_i[slot * KIST + e];
+      // entry e of the list of wave src (past its end: -inf, last in order)
+      auto entry = [&](int src, int e, float& s, int& i) {
+        const int slot = src * kSelRowsPerWave + rcol;
+        s = -INFINITY;
+        i = 0x7fffffff;
+        if (e < s_kcnt[slot]) {
+          s = key_to_float(s_kept_k[slot * KST + e]);
+          i = s_kept_i[slot * KIST + e];
+        }
+      };
+      float vs;
+      int vi;
+      if (k <= 16) {  // uniform: the four lists fill one wave
+        entry(lane >> 4, lane & 15, vs, vi);
+        bitonic_sort64_desc(vs, vi);
+      } else {
+        // lists 0 and 1 sorted together, lists 2 and 3 together: the 32 best of
+        // each pair, one pair's on each half-wave, sorted once more
+        const int h = lane >> 5, e = lane & 31;
+        float ws;
+        int wi;
+        entry(h, e, vs, vi);
+        entry(2 + h, e, ws, wi);
+        bitonic_sort64_desc(vs, vi);
+        bitonic_sort64_desc(ws, wi);
+        const float us = xor32_f(ws);
+        const int ui = xor32_i(wi);
+        if (h) {
+          vs = us;
+          vi = ui;
+        }
+        bitonic_sort64_desc(vs, vi);
       }
-      bitonic_sort64_desc(vs, vi);
       if (scaled_domain) vs = ldexpf(vs, -readlane_i(score_exp, rcol));
       if (lane < k && row < a.Nq) {
         const int64_t o = ((int64_t)b * a.Nq + row) * k + lane;
-        a.out_idx[o] = vi;
+        a.out_idx[o] = vi < a.Nk ? vi : lane;  // fewer than k comparable scores: some index in range (k < Nk)
         a.out_score[o] = vs;
       }
     }
@@ -1203,8 +1227,10 @@ static void launch_rq(const SelectArgs& a, bool vec, dim3 grid, hipStream_t stre
 }
 
 template <int KS>
-static void launch_split_heads(const SelectArgs& a, dim3 grid, hipStream_t stream) {
-  if (a.k <= 32)
+static void launch_split_heads(const SelectArgs& a, bool ksp, dim3 grid, hipStream_t stream) {
+  if (ksp)
+    hipLaunchKernelGGL((lowrank_topk_select_kernel<1, false, 48, KS, -1, true>), grid, dim3(256), 0, stream, a);
+  else if (a.k <= 32)
     hipLaunchKernelGGL((lowrank_topk_select_kernel<1, false, 48, KS, 0, true>), grid, dim3(256), 0, stream, a);
   else
     hipLaunchKernelGGL((lowrank_topk_select_kernel<1, false, 80, KS, 0, true>), grid, dim3(256), 0, stream, a);
@@ -1225,12 +1251,12 @@ static void launch_split(const SelectArgs& a, dim3 grid, hipStream_t stream) {
 
 // The split-layout kernels of one select: cooperative, key-split or per-wave.
 template <bool BF>
-static void launch_split_forms(const SelectArgs& a, int RP, bool coop4, bool ksp, dim3 grid, hipStream_t stream) {
+static void launch_split_forms(const SelectArgs& a, int RP, bool coop4, bool ksp, dim3 grid, dim3 kgrid,
+                               hipStream_t stream) {
   if (coop4) {
     if (RP == 32) launch_split<1, 4, BF>(a, grid, stream);
     else launch_split<2, 4, BF>(a, grid, stream);
   } else if (ksp) {
-    const dim3 kgrid((unsigned)((int64_t)((a.Nq + kSelRowsPerWave - 1) / kSelRowsPerWave) * a.B));
     switch (RP / 32) {
       case 1: launch_split<1, -1, BF>(a, kgrid, stream); break;
       case 2: launch_split<2, -1, BF>(a, kgrid, stream); break;
@@ -1252,9 +1278,20 @@ static void launch_split_forms(const SelectArgs& a, int RP, bool coop4, bool ksp
 // 0.53 for the per-wave kernel); on smaller grids (C3's 128 and 32
 // workgroups) the per-wave kernel is as fast or faster.
 constexpr int64_t kSelCoop4MinBlocks = 512;
+// fp32 keys of 33 to 64 ranks load twice the bytes per score: there the staging
+// wins from the first workgroup beyond one per CU (4096 keys, k = 32: 320
+// workgroups 177 us against 257 per wave, 256 workgroups 154 against 155; bf16
+// keys and ranks <= 32 are level, 152 against 156 and 155 against 155).
+constexpr int64_t kSelCoop4MinBlocksWide = 257;
 // Below one 64-row workgroup per CU, with k <= 16 and at least four key chunks,
-// the key-split per-wave form runs a quarter of the serial chunk chain.
+// the key-split per-wave form runs a quarter of the serial chunk chain.  Lists
+// of up to 32 take longer to merge: it serves them while its workgroups of 16
+// rows fit the chip at two per CU (4096 keys, k = 32: 64 workgroups of 64 rows
+// 77 us against 150 per wave, 128: 104 against 155, 192: 157 against 154; rank
+// 128: 103 against 254 and 200 against 260; two heads of rank 32: 105 against
+// 157 at 128).
 constexpr int64_t kSelKspMaxBlocks = 256;
+constexpr int64_t kSelKspMaxBlocks32 = 129;
 constexpr int kSelKspMinKeys = 4 * kSelChunk;
 
 namespace {
@@ -1327,10 +1364,11 @@ int launch_topk_select(const SelectArgs& a_in, hipStream_t stream) {
   JN_REQUIRE(!mh || (select_heads_fit(a.head_rank, a.heads) && a.heads * a.head_rank == a.r), kUnsupported,
              "multi-head top-k select: %d heads of rank %d must fill 4 K-steps of 32 ranks at most (rank %d)",
              a.heads, a.head_rank, a.r);
-  // multi-head scores always run on the per-wave split kernel; bf16 operands
-  // take the split kernels' forms whatever the mode
-  int mode = mh ? kSelectSplitF16Wave : select_mode();
+  // multi-head scores always run on the per-wave and key-split kernels; bf16
+  // operands take the split kernels' forms whatever the mode
+  int mode = select_mode();
   if (mode == kSelectSplitF16Register) mode = kSelectSplitF16;
+  if (mh && mode != kSelectSplitF16 && mode != kSelectSplitF16KeySplit) mode = kSelectSplitF16Wave;
   if (a.bf16 && mode == kSelectF32) mode = kSelectSplitF16;
 
   if (mode != kSelectF32) {
@@ -1361,22 +1399,28 @@ int launch_topk_select(const SelectArgs& a_in, hipStream_t stream) {
     }
     a.split_key = s.split;
     a.split_exp = s.kexp;
-    const bool coop4 = RP <= 64 && (mode == kSelectSplitF16Coop4 ||
-                                    (mode == kSelectSplitF16 && blocks >= kSelCoop4MinBlocks));
-    const bool ksp = !coop4 && a.k <= 16 &&
+    const int64_t coop4_min = RP > 32 && !a.bf16 ? kSelCoop4MinBlocksWide : kSelCoop4MinBlocks;
+    const int64_t ksp_max = a.k <= 16 ? kSelKspMaxBlocks : kSelKspMaxBlocks32;
+    const bool coop4 = !mh && RP <= 64 &&
+                       (mode == kSelectSplitF16Coop4 || (mode == kSelectSplitF16 && blocks >= coop4_min));
+    const bool ksp = !coop4 && a.k <= 32 &&
                      (mode == kSelectSplitF16KeySplit ||
-                      (mode == kSelectSplitF16 && blocks < kSelKspMaxBlocks && a.Nk >= kSelKspMinKeys));
+                      (mode == kSelectSplitF16 && blocks < ksp_max && a.Nk >= kSelKspMinKeys));
+    const int64_t kblocks = (int64_t)((a.Nq + kSelRowsPerWave - 1) / kSelRowsPerWave) * a.B;
+    JN_REQUIRE(!ksp || kblocks < (1LL << 31), kInvalidArgument, "bad grid size");
+    const dim3 kgrid((unsigned)kblocks);
     JN_PROFILE("lowrank_topk_select_kernel", stream);
     if (mh) {
+      const dim3 hgrid = ksp ? kgrid : grid;
       switch (RP / 32) {
-        case 2: launch_split_heads<2>(a, grid, stream); break;
-        case 3: launch_split_heads<3>(a, grid, stream); break;
-        default: launch_split_heads<4>(a, grid, stream); break;
+        case 2: launch_split_heads<2>(a, ksp, hgrid, stream); break;
+        case 3: launch_split_heads<3>(a, ksp, hgrid, stream); break;
+        default: launch_split_heads<4>(a, ksp, hgrid, stream); break;
       }
     } else if (a.bf16) {
-      launch_split_forms<true>(a, RP, coop4, ksp, grid, stream);
+      launch_split_forms<true>(a, RP, coop4, ksp, grid, kgrid, stream);
     } else {
-      launch_split_forms<false>(a, RP, coop4, ksp, grid, stream);
+      launch_split_forms<false>(a, RP, coop4, ksp, grid, kgrid, stream);
     }
     JN_LAUNCH_CHECK();
     return kOk;

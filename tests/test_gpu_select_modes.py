@@ -246,3 +246,59 @@ def test_split_kernels_agree(dev, r, k, B, Nq, Nk, dominant):
     assert int(wi.min()) >= 0 and int(wi.max()) < Nk
     srt = wi.sort(dim=-1).values
     assert bool((srt[..., 1:] != srt[..., :-1]).all())
+
+
+@pytest.mark.parametrize("r,k,B,Nq,Nk,case", [(64, 32, 1, 1000, 4096, "close"), (64, 17, 2, 33, 193, "close"),
+                                              (20, 31, 3, 16, 1531, "ties"), (128, 32, 1, 65, 2000, "ties"),
+                                              (64, 32, 2, 48, 800, "nan"), (64, 12, 2, 48, 800, "nan")])
+def test_key_split_merges_lists_of_more_than_16(dev, r, k, B, Nq, Nk, case):
+    """The key-split kernel's four lists of up to 32 entries merge to the k
+    best of the row: bit-identical to the per-wave kernel, also where equal
+    scores lie in several quarters.  Rows without a comparable score come back
+    with indices in range, and leave the other rows alone."""
+    import jakal_net_native as jn
+
+    g = torch.Generator().manual_seed(9100 + r + k + Nk)
+    q = torch.randn(B, Nq, r, generator=g)
+    key = torch.randn(B, Nk, r, generator=g)
+    if case == "ties":  # every score eight times, spread over the key quarters
+        key = key[:, : (Nk + 7) // 8].repeat(1, 8, 1)[:, :Nk].contiguous()
+    if case == "nan":
+        q[:, 5] = float("nan")
+    scale = torch.rand(r, generator=g) + 0.5
+    out = {}
+    try:
+        for m in (jn.SELECT_SPLIT_F16_WAVE, jn.SELECT_SPLIT_F16_KEYSPLIT):
+            jn.set_select_mode(m)
+            idx, score = jn.low_rank_topk_select(q.to(dev), key.to(dev), scale.to(dev), None, False, 1.0, k)
+            out[m] = (idx.cpu(), score.cpu())
+    finally:
+        jn.set_select_mode(jn.SELECT_SPLIT_F16)
+    (wi, ws), (ki, ks) = out[jn.SELECT_SPLIT_F16_WAVE], out[jn.SELECT_SPLIT_F16_KEYSPLIT]
+    rows = torch.tensor([i for i in range(Nq) if case != "nan" or i != 5])
+    assert torch.equal(wi[:, rows], ki[:, rows])
+    assert torch.equal(ws[:, rows], ks[:, rows])
+    assert int(ki.min()) >= 0 and int(ki.max()) < Nk
+
+
+@pytest.mark.parametrize("heads,head_rank,k,N", [(2, 24, 13, 777), (2, 32, 32, 1300), (4, 12, 20, 193)])
+def test_key_split_heads(dev, heads, head_rank, k, N):
+    """Several heads on the key-split kernel: the same edges in the same order
+    as on the per-wave kernel, so the same propagation bit for bit."""
+    import jakal_net_native as jn
+    from jakal_net import Layer, LowRankBilinearPairwise, MultiHeadPairwise, SparsePropagation
+
+    torch.manual_seed(9200 + heads + k)
+    layer = Layer(dim=16, num_nodes=N, state=torch.randn(2, N, device=dev), val=torch.randn(2, N, 16, device=dev))
+    pairwise = MultiHeadPairwise([LowRankBilinearPairwise(16, head_rank).to(dev) for _ in range(heads)])
+    op = SparsePropagation(pairwise, sparse_type="topk", topk=k, implementation="native")
+    out = {}
+    try:
+        for m in (jn.SELECT_SPLIT_F16_WAVE, jn.SELECT_SPLIT_F16_KEYSPLIT):
+            jn.set_select_mode(m)
+            with torch.no_grad():
+                out[m] = op(layer)
+    finally:
+        jn.set_select_mode(jn.SELECT_SPLIT_F16)
+    a, b = out[jn.SELECT_SPLIT_F16_WAVE], out[jn.SELECT_SPLIT_F16_KEYSPLIT]
+    assert torch.equal(a.delta_state, b.delta_state) and torch.equal(a.delta_val, b.delta_val)
