@@ -18,7 +18,8 @@
 //                                    of the scores GEMM's softsign epilogue
 // Softsign (elementwise) instead runs inside the two score GEMMs' epilogues
 // (jn_gemm.hip), which saves the two in-place passes over the N x N matrix.
-//   colsum_rows_kernel             : grad ps[j] = sum_i E[i, j] gds[i] (fixed order)
+//   colsum_rows_kernel             : grad ps[j] = sum_i E[i, j] gds[i] (fixed order);
+//                                    colsum_narrow_kernel for few columns
 //   scale_grad_partials_kernel     : w_hat partials and scaling of dP_s
 #include "jn_internal.hpp"
 
@@ -237,19 +238,75 @@ __global__ __launch_bounds__(1024) void colsum_rows_kernel(const float* M, const
   }
 }
 
+// The same sums for matrices of few columns: a workgroup of 16 waves owns 16
+// columns (four lanes of float4), its other lanes 16 rows at a time, so four
+// times the workgroups of a 64-column tile share the rows.  Row i belongs to
+// (wave, row lane) = (i / 16 % 16, i % 16); the 16 row lanes are added by
+// halving exchanges, the waves in order.  The 64-column tile left most of the
+// chip idle here and each wave with a chain of Nr / 16 loads: the sums of 8 x
+// 1024 x 256 and 8 x 256 x 1024 matrices 20 -> 2 us each (25.4 -> 7.1 with the
+// events around the launch), the two bf16 transitions around them 188 -> 154.
+
+__global__ __launch_bounds__(1024) void colsum_narrow_kernel(const float* M, const float* a, const float* c, int B,
+                                                             int Nr, int Nc, float* out) {
+  __shared__ float4 red[16][4];
+  const int lane = lane_id(), wave = wave_id();
+  const int tiles = (Nc + 15) / 16;
+  const int b = blockIdx.x / tiles;
+  const int j = (blockIdx.x % tiles) * 16 + 4 * (lane & 3);
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (j < Nc) {
+    const float* mb = M + (int64_t)b * Nr * Nc + j;
+    const float* ab = a + (int64_t)b * Nr;
+    const float* cb = c ? c + (int64_t)b * Nr : nullptr;
+    auto wt = [&](int i) { return cb ? ab[i] * cb[i] : ab[i]; };
+    int i = 16 * wave + (lane >> 2);
+    for (; i + 768 < Nr; i += 1024) {
+      float4 v[4];
+      float f[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        v[u] = load_w<4>(mb + (int64_t)(i + 256 * u) * Nc);
+        f[u] = wt(i + 256 * u);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) fma4(s, f[u], v[u]);
+    }
+    for (; i < Nr; i += 256) fma4(s, wt(i), load_w<4>(mb + (int64_t)i * Nc));
+  }
+#pragma unroll
+  for (int m = 4; m < kWave; m <<= 1) {
+    s.x += shfl_xor_f(s.x, m);
+    s.y += shfl_xor_f(s.y, m);
+    s.z += shfl_xor_f(s.z, m);
+    s.w += shfl_xor_f(s.w, m);
+  }
+  if (lane < 4) red[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && lane < 4 && j < Nc) {
+    float4 t = red[0][lane];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) t = add4(t, red[w][lane]);
+    store_w<4>(out + (int64_t)b * Nc + j, t);
+  }
+}
+
 int launch_colsum_rows(const float* M, const float* a, const float* c, int B, int Nr, int Nc, float* out,
                        const char* name, hipStream_t stream) {
-  // 256-column tiles with float4 loads when they still give every CU a workgroup
-  const bool vec = (Nc % 4 == 0) && ((reinterpret_cast<uintptr_t>(M) & 15) == 0) &&
-                   ((reinterpret_cast<uintptr_t>(out) & 15) == 0) && (int64_t)B * ((Nc + 255) / 256) >= 256;
-  const int ct = vec ? 256 : 64;
+  // 256-column tiles with float4 loads when they still give every CU a
+  // workgroup, 16-column tiles when 64-column ones do not
+  const bool al = (Nc % 4 == 0) && ((reinterpret_cast<uintptr_t>(M) & 15) == 0) &&
+                  ((reinterpret_cast<uintptr_t>(out) & 15) == 0);
+  const bool vec = al && (int64_t)B * ((Nc + 255) / 256) >= 256;
+  const bool narrow = al && (int64_t)B * ((Nc + 63) / 64) < 256;
+  const int ct = vec ? 256 : narrow ? 16 : 64;
   const int64_t blocks = (int64_t)B * ((Nc + ct - 1) / ct);
   JN_REQUIRE(blocks < (1LL << 31), kUnsupported, "too many columns");
   JN_PROFILE(name, stream);
-  if (vec) hipLaunchKernelGGL(colsum_rows_kernel<true>, dim3((unsigned)blocks), dim3(1024), 0, stream, M, a, c, B, Nr,
-                              Nc, out);
-  else hipLaunchKernelGGL(colsum_rows_kernel<false>, dim3((unsigned)blocks), dim3(1024), 0, stream, M, a, c, B, Nr,
-                          Nc, out);
+  const dim3 grid((unsigned)blocks), block(1024);
+  if (vec) hipLaunchKernelGGL(colsum_rows_kernel<true>, grid, block, 0, stream, M, a, c, B, Nr, Nc, out);
+  else if (narrow) hipLaunchKernelGGL(colsum_narrow_kernel, grid, block, 0, stream, M, a, c, B, Nr, Nc, out);
+  else hipLaunchKernelGGL(colsum_rows_kernel<false>, grid, block, 0, stream, M, a, c, B, Nr, Nc, out);
   JN_LAUNCH_CHECK();
   return kOk;
 }

@@ -124,3 +124,11 @@ def test_dense_transition_api_native_matches_reference(dev):
         a, b = ref.compute_delta(src, dst), nat.compute_delta(src, dst)
         assert torch.allclose(a.delta_state, b.delta_state, atol=1e-5, rtol=1e-5)
         assert torch.allclose(a.delta_val, b.delta_val, atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("B,Ns,Nd", [(1, 1, 4), (2, 257, 20), (1, 1029, 252), (1, 1793, 36), (3, 255, 100)])
+def test_column_sums_of_few_columns(dev, B, Ns, Nd):
+    """The state sums of matrices with too few columns to fill the chip run on
+    16-column tiles: tiles and row strides that do not divide, row counts on
+    both sides of the unrolled loop, the smallest matrix."""
+    _run(dev, 880 + Ns, B, Ns, Nd, 16, 12, 8, 1.0, "softmax")
