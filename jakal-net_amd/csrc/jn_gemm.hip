@@ -20,6 +20,8 @@
 // v_mfma_f32_16x16x4f32 tiles; lane group l/16 owns a 4-wide k sub-slice so
 // operand fetches are single ds_read_b128s.
 #include <atomic>
+#include <type_traits>
+
 #include "jn_internal.hpp"
 
 namespace jakal {
@@ -924,14 +926,14 @@ __global__ __launch_bounds__(256, 4) void gemm_f32_fast_kernel(GemmArgs g, int t
 // The projection of bf16 layer values and its two gradients, and a bf16
 // dense layer's three N x N products (E . pv, E^T . gdv, gdv . pv^T, causal
 // K ranges included), on
-// v_mfma_f32_16x16x32_bf16: workgroup tile 128 x 128, 2 x 2 waves of 64 x 64
-// (4 x 4 tiles of 16 x 16), K in slices of 64 (two K-steps of 32), LDS double
+// v_mfma_f32_16x16x32_bf16: workgroup tile T x T, T = 128 or 64 (kTile64Below),
+// 2 x 2 waves of T/2 x T/2 (tiles of 16 x 16), K in slices of 64 (two K-steps of 32), LDS double
 // buffered with register prefetch.  Both operands sit in LDS as [row][k]
 // bf16 (row = m for A, n for B; 8 elements of padding per row), so a lane's
 // fragment -- 8 consecutive k of one row -- is one 16-byte LDS read.  fp32
 // operands are rounded to bf16 (nearest even) on their way into LDS; K-major
 // operands are transposed there in 4 x 4 (fp32) or 4 x 8 (bf16) blocks.
-// Accumulation is fp32.  The epilogue stages each wave's 64 x 64 block in LDS
+// Accumulation is fp32.  The epilogue stages each wave's block in LDS
 // and writes whole 8-element rows (one 16-byte store of bf16, two of fp32);
 // the dense score gradient's softsign epilogue works from the accumulators.
 // Preconditions (host-checked, else the fp32 kernels run): M, N >= 128, N and
@@ -941,28 +943,40 @@ __global__ __launch_bounds__(256, 4) void gemm_f32_fast_kernel(GemmArgs g, int t
 // buffer resources: a vector outside its operand reads as zeros.
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
 constexpr int kBfT = 128;           // tile M and N
+// Grids of fewer 128-wide tiles than CUs take 64-wide ones (2 x 2 waves of 32 x
+// 32, also for gemm_x3_kernel): four times the workgroups, every element's K
+// chain as before, so the same results bit for bit.  Measured on both tiles,
+// 128 and 64 wide: bf16 route aggregates of 64 and 256 tiles 29.5 against 19.7
+// us (mean), of 32 tiles over K = 4096 147 against 71; fp32 dense aggregate and
+// value gradient of 32 tiles 75 and 87 against 39 and 50; input gradients of 128
+// tiles 20 against 14.  From 256 tiles on the wide ones win where K is long
+// (route aggregate 79 against 86, weight gradient 20.1 against 22.7).
+constexpr int64_t kTile64Below = 256;
 constexpr int kBfK = 64;            // K per slice
 constexpr int kBfS = kBfK + 8;      // LDS row stride in bf16 elements (144 bytes)
-constexpr int kBfStage = 64 + 4;    // epilogue row stride in floats
+constexpr int bf_stage(int tile) { return tile / 2 + 4; }  // epilogue row stride in floats
 
-// Operand loader of one slice: R = 128 rows (m or n) x 64 k into LDS [row][k].
+// Operand loader of one slice: T rows (m or n) x 64 k into LDS [row][k].
 //   KC: row-major with k contiguous (row stride ld); else k-major (k rows of stride ld).
 //   BF: the source holds bf16; else fp32, rounded to bf16.
 //   KS: (k-major fp32 only) each element is first multiplied by a scale per k.
-template <bool KC, bool BF, bool KS = false>
+template <bool KC, bool BF, bool KS, int T>
 struct BfLoader {
   static_assert(!KS || (!KC && !BF), "k scales apply to k-major fp32 operands");
-  // 16-byte loads per thread and slice
-  static constexpr int kLoads = KC ? (BF ? 4 : 8) : (BF ? 4 : 8);
+  // 16-byte loads per thread and slice (k-major bf16 rows: 4 x 8 blocks of the first 2 T threads)
+  static constexpr int kLoads = KC ? (BF ? T / 32 : T / 16) : (BF ? 4 : T / 16);
+  static constexpr int kBlocks = T / 64;       // 4 x 4 blocks of a k-major fp32 thread
+  static constexpr int kRow4 = T / 4, kRow8 = T / 8;  // row groups of 4 and of 8
+  __device__ __forceinline__ static bool idle(int tid) { return !KC && BF && T < 128 && tid >= 2 * T; }
   uint4 r[kLoads];
-  float4 sc[KS ? 2 : 1];  // the scales of a thread's two 4 x 4 blocks (k = 4 kb .. 4 kb + 3)
+  float4 sc[KS ? kBlocks : 1];  // the scales of a thread's 4 x 4 blocks (k = 4 kb .. 4 kb + 3)
 
   // the k scales of the slice's (from k0; ks_rs addresses the scale of k0)
   __device__ __forceinline__ void load_scales(__amdgpu_buffer_rsrc_t ks_rs, int k0, int kend, int tid) {
     if constexpr (KS) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int kb = (tid + 256 * h) >> 5;
+      for (int h = 0; h < kBlocks; ++h) {
+        const int kb = (tid + 256 * h) / kRow4;
         sc[h] = buf_load4(ks_rs, k0 + 4 * kb < kend ? (uint32_t)(16 * kb) : kOobOffset);
       }
     }
@@ -978,26 +992,27 @@ struct BfLoader {
                                        int row0, int rows, int k0, int kend, int tid) {
     constexpr uint32_t EB = BF ? 2 : 4;
     [[maybe_unused]] const int wbase = tid & ~63;
-    if constexpr (KC && BF) {  // 128 rows x 8 groups of 8 k
+    if constexpr (KC && BF) {  // T rows x 8 groups of 8 k
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < kLoads; ++u) {
         const int e = tid + 256 * u, row = e >> 3, kq = (e & 7) * 8;
         const bool ok = row0 + row < rows && k0 + kq < kend;
         const auto rs = ((wbase + 256 * u) >> 3) < split_row ? rs0 : rs1;
         r[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
                                              rs, ok ? (uint32_t)(row * ld + kq) * EB : kOobOffset, 0, 0));
       }
-    } else if constexpr (KC) {  // 128 rows x 16 groups of 4 k
+    } else if constexpr (KC) {  // T rows x 16 groups of 4 k
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < kLoads; ++u) {
         const int e = tid + 256 * u, row = e >> 4, kq = (e & 15) * 4;
         const bool ok = row0 + row < rows && k0 + kq < kend;
         const auto rs = ((wbase + 256 * u) >> 4) < split_row ? rs0 : rs1;
         r[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
                                              rs, ok ? (uint32_t)(row * ld + kq) * EB : kOobOffset, 0, 0));
       }
-    } else if constexpr (BF) {  // 16 groups of 4 k x 16 groups of 8 rows: one 4 x 8 block per thread
-      const int kb = tid >> 4, rb = (tid & 15) * 8;
+    } else if constexpr (BF) {  // 16 groups of 4 k x T / 8 groups of 8 rows: one 4 x 8 block per thread
+      if (idle(tid)) return;
+      const int kb = tid / kRow8, rb = (tid % kRow8) * 8;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int kk = 4 * kb + i;
@@ -1005,10 +1020,10 @@ struct BfLoader {
         r[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
                                              rs0, ok ? (uint32_t)(kk * ld + rb) * EB : kOobOffset, 0, 0));
       }
-    } else {  // 16 groups of 4 k x 32 groups of 4 rows: two 4 x 4 blocks per thread
+    } else {  // 16 groups of 4 k x T / 4 groups of 4 rows: T / 64 4 x 4 blocks per thread
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int blk = tid + 256 * h, kb = blk >> 5, rb = (blk & 31) * 4;
+      for (int h = 0; h < kBlocks; ++h) {
+        const int blk = tid + 256 * h, kb = blk / kRow4, rb = (blk % kRow4) * 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int kk = 4 * kb + i;
@@ -1027,19 +1042,20 @@ struct BfLoader {
   __device__ __forceinline__ void store(bf16_t* s, int tid) const {
     if constexpr (KC && BF) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < kLoads; ++u) {
         const int e = tid + 256 * u, row = e >> 3, kq = (e & 7) * 8;
         *reinterpret_cast<uint4*>(&s[row * kBfS + kq]) = r[u];
       }
     } else if constexpr (KC) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < kLoads; ++u) {
         const int e = tid + 256 * u, row = e >> 4, kq = (e & 15) * 4;
         *reinterpret_cast<uint2*>(&s[row * kBfS + kq]) = make_uint2(pack2(r[u].x, r[u].y), pack2(r[u].z, r[u].w));
       }
     } else if constexpr (BF) {
       // r[i] holds k = 4 kb + i, rows rb .. rb + 7 (two bf16 per word)
-      const int kb = tid >> 4, rb = (tid & 15) * 8;
+      if (idle(tid)) return;
+      const int kb = tid / kRow8, rb = (tid % kRow8) * 8;
       const uint32_t w[4][4] = {{r[0].x, r[0].y, r[0].z, r[0].w}, {r[1].x, r[1].y, r[1].z, r[1].w},
                                 {r[2].x, r[2].y, r[2].z, r[2].w}, {r[3].x, r[3].y, r[3].z, r[3].w}};
 #pragma unroll
@@ -1051,8 +1067,8 @@ struct BfLoader {
       }
     } else {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int blk = tid + 256 * h, kb = blk >> 5, rb = (blk & 31) * 4;
+      for (int h = 0; h < kBlocks; ++h) {
+        const int blk = tid + 256 * h, kb = blk / kRow4, rb = (blk % kRow4) * 4;
         const uint4* v = &r[4 * h];  // v[i]: k = 4 kb + i, rows rb .. rb + 3
         uint32_t c[4][4] = {{v[0].x, v[0].y, v[0].z, v[0].w}, {v[1].x, v[1].y, v[1].z, v[1].w},
                             {v[2].x, v[2].y, v[2].z, v[2].w}, {v[3].x, v[3].y, v[3].z, v[3].w}};
@@ -1074,12 +1090,14 @@ struct BfLoader {
 
 // C_BF: C and the addend hold bf16 (the input gradient, the dense aggregate
 // and value gradient).
-template <bool A_KC, bool A_BF, bool B_KC, bool B_BF, bool C_BF, int USE>
+template <bool A_KC, bool A_BF, bool B_KC, bool B_BF, bool C_BF, int USE, int T>
 __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(GemmArgs g, int tiles_m, int tiles_n) {
-  __shared__ __align__(16) bf16_t smem[4 * kBfT * kBfS];  // A[2], B[2]; the epilogue reuses it
-  auto sA = [&](int i) { return smem + i * kBfT * kBfS; };
-  auto sB = [&](int i) { return smem + (2 + i) * kBfT * kBfS; };
-  static_assert(4 * 64 * kBfStage * 4 <= 4 * kBfT * kBfS * 2, "epilogue strips must fit in LDS");
+  constexpr int W = T / 2, MT = W / 16;      // a wave's block and its 16 x 16 tiles a side
+  constexpr int STAGE = bf_stage(T);
+  __shared__ __align__(16) bf16_t smem[4 * T * kBfS];  // A[2], B[2]; the epilogue reuses it
+  auto sA = [&](int i) { return smem + i * T * kBfS; };
+  auto sB = [&](int i) { return smem + (2 + i) * T * kBfS; };
+  static_assert(4 * W * STAGE * 4 <= 4 * T * kBfS * 2, "epilogue strips must fit in LDS");
 
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const int wm = wave >> 1, wn = wave & 1;
@@ -1096,14 +1114,14 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(GemmArgs g, int tiles
   int mi = band * kBand + tb % bm;
   // causal products: the longest K ranges (or the epilogue's non-empty rows) first
   if (g.causal_k == kCausalKLower || (g.epi && g.epi_causal)) mi = tiles_m - 1 - mi;
-  const int m0 = mi * kBfT;
-  const int n0 = (tb / bm) * kBfT;
+  const int m0 = mi * T;
+  const int n0 = (tb / bm) * T;
   const bool batched = g.batch > 1;
   const int split = batched ? 0 : z;
   const int64_t bz = batched ? z : 0;
   int kbeg = split * g.k_chunk;
   int kend = min(g.K, kbeg + g.k_chunk);
-  causal_k_range<kBfT>(g, m0, n0, kbeg, kend);
+  causal_k_range<T>(g, m0, n0, kbeg, kend);
 
   constexpr uint32_t AEB = A_BF ? 2 : 4, BEB = B_BF ? 2 : 4;
   const int lda = (int)g.lda, ldb = (int)g.ldb;
@@ -1124,8 +1142,8 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(GemmArgs g, int tiles
   };
 
   constexpr bool KS = kGemmUses[USE].a_kscale;  // A scaled along k (k-major fp32 A)
-  BfLoader<A_KC, A_BF, KS> la;
-  BfLoader<B_KC, B_BF> lb;
+  BfLoader<A_KC, A_BF, KS, T> la;
+  BfLoader<B_KC, B_BF, false, T> lb;
   [[maybe_unused]] const float* kscale = KS ? g.a_kscale + bz * g.ks_bs : nullptr;
   auto load_slice = [&](int k0) {
     const auto ars = at_k(abase, A_KC, lda, k0, AEB);
@@ -1145,11 +1163,11 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(GemmArgs g, int tiles
     }
   };
 
-  floatx4 acc[4][4];
+  floatx4 acc[MT][MT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < MT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   const int nslices = kend > kbeg ? (kend - kbeg + kBfK - 1) / kBfK : 0;
   if (nslices > 0) {
@@ -1163,16 +1181,16 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(GemmArgs g, int tiles
     if (s + 1 < nslices) load_slice(kbeg + (s + 1) * kBfK);
 #pragma unroll
     for (int ks = 0; ks < kBfK / 32; ++ks) {
-      bf16x8v av[4], bv[4];
+      bf16x8v av[MT], bv[MT];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        av[i] = *reinterpret_cast<const bf16x8v*>(&sA(cur)[(wm * 64 + i * 16 + col) * kBfS + ks * 32 + grp * 8]);
-        bv[i] = *reinterpret_cast<const bf16x8v*>(&sB(cur)[(wn * 64 + i * 16 + col) * kBfS + ks * 32 + grp * 8]);
+      for (int i = 0; i < MT; ++i) {
+        av[i] = *reinterpret_cast<const bf16x8v*>(&sA(cur)[(wm * W + i * 16 + col) * kBfS + ks * 32 + grp * 8]);
+        bv[i] = *reinterpret_cast<const bf16x8v*>(&sB(cur)[(wn * W + i * 16 + col) * kBfS + ks * 32 + grp * 8]);
       }
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
+        for (int nt = 0; nt < MT; ++nt)
           acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[mt], bv[nt], acc[mt][nt], 0, 0, 0);
     }
     if (s + 1 < nslices) {
@@ -1187,31 +1205,31 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(GemmArgs g, int tiles
   // from the accumulators (the 16 x 16 output layout of every MFMA shape)
   if constexpr (USE == kGemmDenseEdgeGradBf16) {
     if (g.epi) {
-      dense_epilogue_tiles<kGemmDenseEdgeGrad, 4>(g, bz, acc, m0 + wm * 64, n0 + wn * 64, C, lane);
+      dense_epilogue_tiles<kGemmDenseEdgeGrad, MT>(g, bz, acc, m0 + wm * W, n0 + wn * W, C, lane);
       return;
     }
   }
 
-  // epilogue: each wave's 64 x 64 block through LDS, then rows of 8 elements
-  float* stage = reinterpret_cast<float*>(smem) + wave * 64 * kBfStage;
+  // epilogue: each wave's block through LDS, then rows of 8 elements
+  float* stage = reinterpret_cast<float*>(smem) + wave * W * STAGE;
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < MT; ++nt)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) stage[(mt * 16 + grp * 4 + v) * kBfStage + nt * 16 + col] = acc[mt][nt][v];
+      for (int v = 0; v < 4; ++v) stage[(mt * 16 + grp * 4 + v) * STAGE + nt * 16 + col] = acc[mt][nt][v];
   __syncthreads();
   [[maybe_unused]] bf16_t* Cb = reinterpret_cast<bf16_t*>(g.C) + bz * g.c_bs;
   [[maybe_unused]] const bf16_t* addb =
       g.addend ? reinterpret_cast<const bf16_t*>(g.addend) + bz * g.add_bs : nullptr;
   [[maybe_unused]] const float* mscale = g.c_mscale ? g.c_mscale + bz * g.ms_bs : nullptr;
 #pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const int r = it * 8 + (lane >> 3), c0 = (lane & 7) * 8;
-    const int m = m0 + wm * 64 + r, n = n0 + wn * 64 + c0;
+  for (int it = 0; it < W * W / 512; ++it) {
+    const int e = it * kWave + lane, r = e / (W / 8), c0 = e % (W / 8) * 8;
+    const int m = m0 + wm * W + r, n = n0 + wn * W + c0;
     if (m >= g.M || n >= g.N) continue;
-    const float4 x0 = *reinterpret_cast<const float4*>(&stage[r * kBfStage + c0]);
-    const float4 x1 = *reinterpret_cast<const float4*>(&stage[r * kBfStage + c0 + 4]);
+    const float4 x0 = *reinterpret_cast<const float4*>(&stage[r * STAGE + c0]);
+    const float4 x1 = *reinterpret_cast<const float4*>(&stage[r * STAGE + c0 + 4]);
     if constexpr (C_BF) {
       float4 y0 = x0, y1 = x1;
       if (mscale) {  // C row m scaled (the route value gradient's diag(rho))
@@ -1276,7 +1294,7 @@ static bool bf16_path_ok(const GemmArgs& g, int use, int splits) {
 // gemm_x3_kernel is gemm_bf16_kernel for fp32 operands in this form: the three
 // planes of both operands sit in LDS as [row][k] bf16, K in slices of 32, in
 // one LDS buffer (61 KB, 70 KB with the epilogue's strips: two workgroups per
-// CU) refilled from registers that prefetch the next slice, split on their way
+// CU; 31 KB for 64 x 64 tiles) refilled from registers that prefetch the next slice, split on their way
 // into LDS; each slice's operand resources start at the slice, so 32-bit
 // offsets cover any K.  Used for the projection and its gradients and for the
 // dense aggregation E.pv and its value gradient E^T.gdv (causal K ranges
@@ -1288,31 +1306,35 @@ static bool bf16_path_ok(const GemmArgs& g, int use, int splits) {
 // 1.6e4), so the score-gradient product gdv.pv^T stays on fp32 MFMA.
 constexpr int kX3K = 32;                 // K per slice
 constexpr int kX3S = kX3K + 8;           // LDS row stride in bf16 elements (80 bytes: conflict-free fragments)
-constexpr int kX3Plane = kBfT * kX3S;    // one plane of one operand
 
-// Operand loader of one slice: 128 rows (m or n) x 32 k of fp32 into the three
+// Operand loader of one slice: T rows (m or n) x 32 k of fp32 into the three
 // LDS planes [row][k].  KC: rows with k contiguous (row stride ld); else k rows
 // of stride ld.  `base` addresses the slice's (row 0, k 0).
-template <bool KC>
+template <bool KC, int T>
 struct X3Loader {
-  uint4 r[4];
+  static constexpr int kPlane = T * kX3S;              // one plane of one operand
+  static constexpr int kLoads = KC ? T / 32 : 4;       // 16-byte loads per thread and slice
+  static constexpr int kRow4 = T / 4;                  // row groups of 4
+  __device__ __forceinline__ static bool idle(int tid) { return !KC && T < 128 && tid >= 2 * T; }
+  uint4 r[kLoads];
 
   // rs1 serves the rows from split_row on (KC only, a multiple of 8: one wave's
   // load never straddles it)
   __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs0, __amdgpu_buffer_rsrc_t rs1, int split_row, int ld,
                                        int row0, int rows, int k0, int kend, int tid) {
-    if constexpr (KC) {  // 128 rows x 8 groups of 4 k
+    if constexpr (KC) {  // T rows x 8 groups of 4 k
       const int wbase = tid & ~63;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < kLoads; ++u) {
         const int e = tid + 256 * u, row = e >> 3, kq = (e & 7) * 4;
         const bool ok = row0 + row < rows && k0 + kq < kend;
         const auto rs = ((wbase + 256 * u) >> 3) < split_row ? rs0 : rs1;
         r[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
                                              rs, ok ? (uint32_t)(row * ld + kq) * 4u : kOobOffset, 0, 0));
       }
-    } else {  // 8 groups of 4 k x 32 groups of 4 rows: one 4 x 4 block per thread
-      const int kb = tid >> 5, rb = (tid & 31) * 4;
+    } else {  // 8 groups of 4 k x T / 4 groups of 4 rows: one 4 x 4 block per thread (the first 2 T)
+      if (idle(tid)) return;
+      const int kb = tid / kRow4, rb = (tid % kRow4) * 4;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int kk = 4 * kb + i;
@@ -1323,11 +1345,11 @@ struct X3Loader {
     }
   }
 
-  // planes h, m, l at s, s + kX3Plane, s + 2 kX3Plane
+  // planes h, m, l at s, s + kPlane, s + 2 kPlane
   __device__ __forceinline__ void store(bf16_t* s, int tid) const {
     if constexpr (KC) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < kLoads; ++u) {
         const int e = tid + 256 * u, row = e >> 3, kq = (e & 7) * 4;
         uint32_t h[4], m[4], l[4];
         x3_split(r[u].x, h[0], m[0], l[0]);
@@ -1336,12 +1358,13 @@ struct X3Loader {
         x3_split(r[u].w, h[3], m[3], l[3]);
         bf16_t* d = &s[row * kX3S + kq];
         *reinterpret_cast<uint2*>(d) = make_uint2(x3_pair(h[0], h[1]), x3_pair(h[2], h[3]));
-        *reinterpret_cast<uint2*>(d + kX3Plane) = make_uint2(x3_pair(m[0], m[1]), x3_pair(m[2], m[3]));
-        *reinterpret_cast<uint2*>(d + 2 * kX3Plane) = make_uint2(x3_pair(l[0], l[1]), x3_pair(l[2], l[3]));
+        *reinterpret_cast<uint2*>(d + kPlane) = make_uint2(x3_pair(m[0], m[1]), x3_pair(m[2], m[3]));
+        *reinterpret_cast<uint2*>(d + 2 * kPlane) = make_uint2(x3_pair(l[0], l[1]), x3_pair(l[2], l[3]));
       }
     } else {
       // r[i] holds k = 4 kb + i, rows rb .. rb + 3
-      const int kb = tid >> 5, rb = (tid & 31) * 4;
+      if (idle(tid)) return;
+      const int kb = tid / kRow4, rb = (tid % kRow4) * 4;
       const uint32_t c[4][4] = {{r[0].x, r[0].y, r[0].z, r[0].w}, {r[1].x, r[1].y, r[1].z, r[1].w},
                                 {r[2].x, r[2].y, r[2].z, r[2].w}, {r[3].x, r[3].y, r[3].z, r[3].w}};
 #pragma unroll
@@ -1351,21 +1374,23 @@ struct X3Loader {
         for (int i = 0; i < 4; ++i) x3_split(c[i][j], h[i], m[i], l[i]);
         bf16_t* d = &s[(rb + j) * kX3S + 4 * kb];
         *reinterpret_cast<uint2*>(d) = make_uint2(x3_pair(h[0], h[1]), x3_pair(h[2], h[3]));
-        *reinterpret_cast<uint2*>(d + kX3Plane) = make_uint2(x3_pair(m[0], m[1]), x3_pair(m[2], m[3]));
-        *reinterpret_cast<uint2*>(d + 2 * kX3Plane) = make_uint2(x3_pair(l[0], l[1]), x3_pair(l[2], l[3]));
+        *reinterpret_cast<uint2*>(d + kPlane) = make_uint2(x3_pair(m[0], m[1]), x3_pair(m[2], m[3]));
+        *reinterpret_cast<uint2*>(d + 2 * kPlane) = make_uint2(x3_pair(l[0], l[1]), x3_pair(l[2], l[3]));
       }
     }
   }
 };
 
-template <bool A_KC, bool B_KC, int USE>
+template <bool A_KC, bool B_KC, int USE, int T>
 __global__ __launch_bounds__(256, 2) void gemm_x3_kernel(GemmArgs g, int tiles_m, int tiles_n) {
-  // [A, B][plane] (61 KB), or the epilogue's four 64-row strips (70 KB)
-  constexpr int kWords = 4 * 64 * kBfStage > 3 * kX3Plane ? 4 * 64 * kBfStage : 3 * kX3Plane;
+  // [A, B][plane] (61 KB; 31 for 64 x 64), or the epilogue's four strips (70 KB; 18)
+  constexpr int W = T / 2, MT = W / 16;  // a wave's block and its 16 x 16 tiles a side
+  constexpr int STAGE = bf_stage(T), PLANE = T * kX3S;
+  constexpr int kWords = 4 * W * STAGE > 3 * PLANE ? 4 * W * STAGE : 3 * PLANE;
   __shared__ __align__(16) uint32_t smem32[kWords];
   bf16_t* smem = reinterpret_cast<bf16_t*>(smem32);
   auto sA = [&](int) { return smem; };
-  auto sB = [&](int) { return smem + 3 * kX3Plane; };
+  auto sB = [&](int) { return smem + 3 * PLANE; };
 
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const int wm = wave >> 1, wn = wave & 1;
@@ -1381,21 +1406,21 @@ __global__ __launch_bounds__(256, 2) void gemm_x3_kernel(GemmArgs g, int tiles_m
   const int tb = t - band * kBand * tiles_n;
   int mi = band * kBand + tb % bm;
   if (g.causal_k == kCausalKLower) mi = tiles_m - 1 - mi;  // longest K ranges first
-  const int m0 = mi * kBfT;
-  const int n0 = (tb / bm) * kBfT;
+  const int m0 = mi * T;
+  const int n0 = (tb / bm) * T;
   const bool batched = g.batch > 1;
   const int split = batched ? 0 : z;
   const int64_t bz = batched ? z : 0;
   int kbeg = split * g.k_chunk;
   int kend = min(g.K, kbeg + g.k_chunk);
-  causal_k_range<kBfT>(g, m0, n0, kbeg, kend);
+  causal_k_range<T>(g, m0, n0, kbeg, kend);
   const int lda = (int)g.lda, ldb = (int)g.ldb;
   const float* gA = g.A + bz * g.a_bs;
   const float* gB0 = g.B0 + bz * g.b_bs;
   const float* gB1 = g.B1 + bz * g.b_bs;
 
-  X3Loader<A_KC> la;
-  X3Loader<B_KC> lb;
+  X3Loader<A_KC, T> la;
+  X3Loader<B_KC, T> lb;
   auto load_slice = [&](int k0) {
     const auto ars = make_rsrc(gA + (A_KC ? (int64_t)m0 * lda + k0 : (int64_t)k0 * lda + m0), kFastRecords);
     la.load(ars, ars, 1 << 30, lda, m0, g.M, k0, kend, tid);
@@ -1411,11 +1436,11 @@ __global__ __launch_bounds__(256, 2) void gemm_x3_kernel(GemmArgs g, int tiles_m
     }
   };
 
-  floatx4 acc[4][4];
+  floatx4 acc[MT][MT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < MT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   const int nslices = kend > kbeg ? (kend - kbeg + kX3K - 1) / kX3K : 0;
   if (nslices > 0) {
@@ -1427,23 +1452,23 @@ __global__ __launch_bounds__(256, 2) void gemm_x3_kernel(GemmArgs g, int tiles_m
   for (int s = 0; s < nslices; ++s) {
     const int cur = s & 1;
     if (s + 1 < nslices) load_slice(kbeg + (s + 1) * kX3K);
-    const bf16_t* a = sA(cur) + (wm * 64 + col) * kX3S + grp * 8;
-    const bf16_t* b = sB(cur) + (wn * 64 + col) * kX3S + grp * 8;
-    bf16x8v ah[4], am[4], al[4], bh[4], bm[4], bl[4];
+    const bf16_t* a = sA(cur) + (wm * W + col) * kX3S + grp * 8;
+    const bf16_t* b = sB(cur) + (wn * W + col) * kX3S + grp * 8;
+    bf16x8v ah[MT], am[MT], al[MT], bh[MT], bm[MT], bl[MT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < MT; ++i) {
       ah[i] = *reinterpret_cast<const bf16x8v*>(a + i * 16 * kX3S);
-      am[i] = *reinterpret_cast<const bf16x8v*>(a + i * 16 * kX3S + kX3Plane);
-      al[i] = *reinterpret_cast<const bf16x8v*>(a + i * 16 * kX3S + 2 * kX3Plane);
+      am[i] = *reinterpret_cast<const bf16x8v*>(a + i * 16 * kX3S + PLANE);
+      al[i] = *reinterpret_cast<const bf16x8v*>(a + i * 16 * kX3S + 2 * PLANE);
       bh[i] = *reinterpret_cast<const bf16x8v*>(b + i * 16 * kX3S);
-      bm[i] = *reinterpret_cast<const bf16x8v*>(b + i * 16 * kX3S + kX3Plane);
-      bl[i] = *reinterpret_cast<const bf16x8v*>(b + i * 16 * kX3S + 2 * kX3Plane);
+      bm[i] = *reinterpret_cast<const bf16x8v*>(b + i * 16 * kX3S + PLANE);
+      bl[i] = *reinterpret_cast<const bf16x8v*>(b + i * 16 * kX3S + 2 * PLANE);
     }
     // the small terms first
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
+      for (int nt = 0; nt < MT; ++nt) {
         floatx4 c = acc[mt][nt];
         c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[mt], bh[nt], c, 0, 0, 0);
         c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[mt], bl[nt], c, 0, 0, 0);
@@ -1460,24 +1485,24 @@ __global__ __launch_bounds__(256, 2) void gemm_x3_kernel(GemmArgs g, int tiles_m
     }
   }
 
-  // epilogue: each wave's 64 x 64 block through LDS, then rows of 8 elements
-  float* stage = reinterpret_cast<float*>(smem) + wave * 64 * kBfStage;
+  // epilogue: each wave's block through LDS, then rows of 8 elements
+  float* stage = reinterpret_cast<float*>(smem) + wave * W * STAGE;
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < MT; ++nt)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) stage[(mt * 16 + grp * 4 + v) * kBfStage + nt * 16 + col] = acc[mt][nt][v];
+      for (int v = 0; v < 4; ++v) stage[(mt * 16 + grp * 4 + v) * STAGE + nt * 16 + col] = acc[mt][nt][v];
   __syncthreads();
   float* C = g.C + (int64_t)split * g.c_split_stride + bz * g.c_bs;
   const float* add = g.addend ? g.addend + bz * g.add_bs : nullptr;
 #pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const int r = it * 8 + (lane >> 3), c0 = (lane & 7) * 8;
-    const int m = m0 + wm * 64 + r, n = n0 + wn * 64 + c0;
+  for (int it = 0; it < W * W / 512; ++it) {
+    const int e = it * kWave + lane, r = e / (W / 8), c0 = e % (W / 8) * 8;
+    const int m = m0 + wm * W + r, n = n0 + wn * W + c0;
     if (m >= g.M || n >= g.N) continue;
-    float4 x0 = *reinterpret_cast<const float4*>(&stage[r * kBfStage + c0]);
-    float4 x1 = *reinterpret_cast<const float4*>(&stage[r * kBfStage + c0 + 4]);
+    float4 x0 = *reinterpret_cast<const float4*>(&stage[r * STAGE + c0]);
+    float4 x1 = *reinterpret_cast<const float4*>(&stage[r * STAGE + c0 + 4]);
     if (add) {
       const float4 a0 = *reinterpret_cast<const float4*>(&add[(int64_t)m * g.ld_add + n]);
       const float4 a1 = *reinterpret_cast<const float4*>(&add[(int64_t)m * g.ld_add + n + 4]);
@@ -1631,90 +1656,111 @@ int launch_gemm(const GemmArgs& g, GemmUse use, int splits, hipStream_t stream) 
     RowsGemm r;
     if (rows_form(g, use, fast, r)) return launch_gemm_rows(&r, 1, stream);
   }
+  // the 128-wide MFMA tiles of this product, or 64-wide where those leave CUs idle
+  const int64_t tiles128 = (int64_t)((g.M + kBfT - 1) / kBfT) * ((g.N + kBfT - 1) / kBfT) * zdim;
+  const int tile = tiles128 < kTile64Below ? 64 : kBfT;
+  const int tm = (g.M + tile - 1) / tile, tn = (g.N + tile - 1) / tile;
+  const int64_t tiles = (int64_t)tm * tn * zdim;
+  auto at_tile = [&](auto launch) {
+    if (tile == 64) launch(std::integral_constant<int, 64>{});
+    else launch(std::integral_constant<int, kBfT>{});
+  };
+  const dim3 tgrid((unsigned)tiles), tblock(256);
   if (gemm_use_dense_bf16(use)) {
     JN_REQUIRE(bf16_path_ok(g, use, splits), kUnsupported,
                "%s needs M, N >= 128, N and the strides multiples of 8 and 16-byte aligned operands", info.name);
-    const int tm = (g.M + kBfT - 1) / kBfT, tn = (g.N + kBfT - 1) / kBfT;
-    const int64_t blocks = (int64_t)tm * tn * zdim;
-    JN_REQUIRE(blocks < (1LL << 31), kUnsupported, "GEMM grid too large");
+    JN_REQUIRE(tiles < (1LL << 31), kUnsupported, "GEMM grid too large");
     JN_PROFILE(info.name, stream);
-    if (use == kGemmDenseAggregateBf16)
-      hipLaunchKernelGGL((gemm_bf16_kernel<true, false, false, true, true, kGemmDenseAggregateBf16>),
-                         dim3((unsigned)blocks), dim3(256), 0, stream, g, tm, tn);
-    else if (use == kGemmDenseValueGradBf16)
-      hipLaunchKernelGGL((gemm_bf16_kernel<false, false, false, true, true, kGemmDenseValueGradBf16>),
-                         dim3((unsigned)blocks), dim3(256), 0, stream, g, tm, tn);
-    else if (use == kGemmDenseEdgeGradBf16)
-      hipLaunchKernelGGL((gemm_bf16_kernel<true, true, true, true, false, kGemmDenseEdgeGradBf16>),
-                         dim3((unsigned)blocks), dim3(256), 0, stream, g, tm, tn);
-    else if (use == kGemmRouteAggregateBf16)
-      hipLaunchKernelGGL((gemm_bf16_kernel<false, false, false, true, true, kGemmRouteAggregateBf16>),
-                         dim3((unsigned)blocks), dim3(256), 0, stream, g, tm, tn);
-    else if (use == kGemmRouteValueGradBf16)
-      hipLaunchKernelGGL((gemm_bf16_kernel<true, false, false, true, true, kGemmRouteValueGradBf16>),
-                         dim3((unsigned)blocks), dim3(256), 0, stream, g, tm, tn);
-    else
-      hipLaunchKernelGGL((gemm_bf16_kernel<true, true, true, true, false, kGemmRouteEdgeGradBf16>),
-                         dim3((unsigned)blocks), dim3(256), 0, stream, g, tm, tn);
+    at_tile([&](auto tc) {
+      constexpr int T = decltype(tc)::value;
+      switch (use) {
+        case kGemmDenseAggregateBf16:
+          hipLaunchKernelGGL((gemm_bf16_kernel<true, false, false, true, true, kGemmDenseAggregateBf16, T>), tgrid,
+                             tblock, 0, stream, g, tm, tn);
+          break;
+        case kGemmDenseValueGradBf16:
+          hipLaunchKernelGGL((gemm_bf16_kernel<false, false, false, true, true, kGemmDenseValueGradBf16, T>), tgrid,
+                             tblock, 0, stream, g, tm, tn);
+          break;
+        case kGemmDenseEdgeGradBf16:
+          hipLaunchKernelGGL((gemm_bf16_kernel<true, true, true, true, false, kGemmDenseEdgeGradBf16, T>), tgrid,
+                             tblock, 0, stream, g, tm, tn);
+          break;
+        case kGemmRouteAggregateBf16:
+          hipLaunchKernelGGL((gemm_bf16_kernel<false, false, false, true, true, kGemmRouteAggregateBf16, T>), tgrid,
+                             tblock, 0, stream, g, tm, tn);
+          break;
+        case kGemmRouteValueGradBf16:
+          hipLaunchKernelGGL((gemm_bf16_kernel<true, false, false, true, true, kGemmRouteValueGradBf16, T>), tgrid,
+                             tblock, 0, stream, g, tm, tn);
+          break;
+        default:
+          hipLaunchKernelGGL((gemm_bf16_kernel<true, true, true, true, false, kGemmRouteEdgeGradBf16, T>), tgrid,
+                             tblock, 0, stream, g, tm, tn);
+          break;
+      }
+    });
     JN_LAUNCH_CHECK();
     return kOk;
   }
   if (gemm_use_bf16(use) && forced != 32 && forced != 64 && bf16_path_ok(g, use, splits)) {
-    const int tm = (g.M + kBfT - 1) / kBfT, tn = (g.N + kBfT - 1) / kBfT;
-    const int64_t blocks = (int64_t)tm * tn * zdim;
-    JN_REQUIRE(blocks < (1LL << 31), kUnsupported, "GEMM grid too large");
+    JN_REQUIRE(tiles < (1LL << 31), kUnsupported, "GEMM grid too large");
     JN_PROFILE(use == kGemmProjectBf16 ? "gemm_bf16_kernel<project_bf16>"
                : use == kGemmGradInputBf16 ? "gemm_bf16_kernel<grad_input_bf16>"
                                            : "gemm_bf16_kernel<grad_weight_bf16>",
                stream);
-    if (use == kGemmProjectBf16)
-      hipLaunchKernelGGL((gemm_bf16_kernel<true, true, true, false, false, kGemmProjectBf16>), dim3((unsigned)blocks),
-                         dim3(256), 0, stream, g, tm, tn);
-    else if (use == kGemmGradInputBf16)
-      hipLaunchKernelGGL((gemm_bf16_kernel<true, false, false, false, true, kGemmGradInputBf16>),
-                         dim3((unsigned)blocks), dim3(256), 0, stream, g, tm, tn);
-    else
-      hipLaunchKernelGGL((gemm_bf16_kernel<false, false, false, true, false, kGemmGradWeightBf16>),
-                         dim3((unsigned)blocks), dim3(256), 0, stream, g, tm, tn);
+    at_tile([&](auto tc) {
+      constexpr int T = decltype(tc)::value;
+      switch (use) {
+        case kGemmProjectBf16:
+          hipLaunchKernelGGL((gemm_bf16_kernel<true, true, true, false, false, kGemmProjectBf16, T>), tgrid, tblock, 0,
+                             stream, g, tm, tn);
+          break;
+        case kGemmGradInputBf16:
+          hipLaunchKernelGGL((gemm_bf16_kernel<true, false, false, false, true, kGemmGradInputBf16, T>), tgrid, tblock,
+                             0, stream, g, tm, tn);
+          break;
+        default:
+          hipLaunchKernelGGL((gemm_bf16_kernel<false, false, false, true, false, kGemmGradWeightBf16, T>), tgrid,
+                             tblock, 0, stream, g, tm, tn);
+          break;
+      }
+    });
     JN_LAUNCH_CHECK();
     return kOk;
   }
   if ((use == kGemmProject || use == kGemmGradInput || use == kGemmGradWeight || use == kGemmDenseAggregate ||
        use == kGemmDenseValueGrad) &&
       forced == 0 && x3_path_ok(g, use, splits)) {
-    const int tm = (g.M + kBfT - 1) / kBfT, tn = (g.N + kBfT - 1) / kBfT;
-    const int64_t blocks = (int64_t)tm * tn * zdim;
-    JN_REQUIRE(blocks < (1LL << 31), kUnsupported, "GEMM grid too large");
-    const dim3 grid((unsigned)blocks);
-    switch (use) {
-      case kGemmProject: {
-        JN_PROFILE("gemm_x3_kernel<project>", stream);
-        hipLaunchKernelGGL((gemm_x3_kernel<true, true, kGemmProject>), grid, dim3(256), 0, stream, g, tm, tn);
-        break;
+    JN_REQUIRE(tiles < (1LL << 31), kUnsupported, "GEMM grid too large");
+    JN_PROFILE(use == kGemmProject          ? "gemm_x3_kernel<project>"
+               : use == kGemmGradInput      ? "gemm_x3_kernel<grad_input>"
+               : use == kGemmGradWeight     ? "gemm_x3_kernel<grad_weight>"
+               : use == kGemmDenseAggregate ? "gemm_x3_kernel<dense_aggregate>"
+                                            : "gemm_x3_kernel<dense_value_grad>",
+               stream);
+    at_tile([&](auto tc) {
+      constexpr int T = decltype(tc)::value;
+      switch (use) {
+        case kGemmProject:
+          hipLaunchKernelGGL((gemm_x3_kernel<true, true, kGemmProject, T>), tgrid, tblock, 0, stream, g, tm, tn);
+          break;
+        case kGemmGradInput:
+          hipLaunchKernelGGL((gemm_x3_kernel<true, false, kGemmGradInput, T>), tgrid, tblock, 0, stream, g, tm, tn);
+          break;
+        case kGemmGradWeight:
+          hipLaunchKernelGGL((gemm_x3_kernel<false, false, kGemmGradWeight, T>), tgrid, tblock, 0, stream, g, tm, tn);
+          break;
+        case kGemmDenseAggregate:
+          hipLaunchKernelGGL((gemm_x3_kernel<true, false, kGemmDenseAggregate, T>), tgrid, tblock, 0, stream, g, tm,
+                             tn);
+          break;
+        default:
+          hipLaunchKernelGGL((gemm_x3_kernel<false, false, kGemmDenseValueGrad, T>), tgrid, tblock, 0, stream, g, tm,
+                             tn);
+          break;
       }
-      case kGemmGradInput: {
-        JN_PROFILE("gemm_x3_kernel<grad_input>", stream);
-        hipLaunchKernelGGL((gemm_x3_kernel<true, false, kGemmGradInput>), grid, dim3(256), 0, stream, g, tm, tn);
-        break;
-      }
-      case kGemmGradWeight: {
-        JN_PROFILE("gemm_x3_kernel<grad_weight>", stream);
-        hipLaunchKernelGGL((gemm_x3_kernel<false, false, kGemmGradWeight>), grid, dim3(256), 0, stream, g, tm, tn);
-        break;
-      }
-      case kGemmDenseAggregate: {
-        JN_PROFILE("gemm_x3_kernel<dense_aggregate>", stream);
-        hipLaunchKernelGGL((gemm_x3_kernel<true, false, kGemmDenseAggregate>), grid, dim3(256), 0, stream, g, tm,
-                           tn);
-        break;
-      }
-      default: {
-        JN_PROFILE("gemm_x3_kernel<dense_value_grad>", stream);
-        hipLaunchKernelGGL((gemm_x3_kernel<false, false, kGemmDenseValueGrad>), grid, dim3(256), 0, stream, g, tm,
-                           tn);
-        break;
-      }
-    }
+    });
     JN_LAUNCH_CHECK();
     return kOk;
   }

@@ -114,3 +114,31 @@ def test_fp32_projection_gemms_in_bf16_thirds(dev, D, r, separate_pv):
     pv is X, split-K over the rows; the fp32 tolerance of the per-op tests."""
     TT._run_topk(dev, TT._c1_inputs(seed=4500 + D, B=2, N=640, D=D, r=r), "softsign", separate_pv, 16,
                  min_checkable=0.5)
+
+
+@pytest.mark.parametrize("B,N,D", [(1, 128, 128), (63, 132, 136), (64, 132, 136)])
+def test_mfma_tiles_on_both_sides_of_the_line(dev, B, N, D):
+    """The three-term GEMMs take 64 x 64 tiles below 256 tiles of 128 x 128: the
+    smallest product (whole tiles), and ragged ones of 252 and 256 tiles."""
+    TD._check_dense(dev, "softsign", True, N, True, B=B, D=D, r=16)
+
+
+def test_bf16_product_is_the_same_on_both_tiles(dev):
+    """The values of 64 dense bf16 transitions are summed on 256 tiles of 128 x
+    128, those of 63 on 64 x 64 (the scores of both on the same kernel): every
+    element keeps its chain over K, so the results are the same bit for bit."""
+    import jakal_net_native as jn
+
+    B, Ns, Nd, D, r = 64, 264, 136, 136, 16
+    g = torch.Generator().manual_seed(4600)
+    src, dst, pv = (torch.randn(B, n, D, generator=g).bfloat16().to(dev) for n in (Ns, Nd, Ns))
+    ps = torch.randn(B, Ns, generator=g).bfloat16().to(dev)
+    Ws, Wt = ((torch.randn(r, D, generator=g) / D**0.5).to(dev) for _ in range(2))
+    w = (torch.rand(r, generator=g) + 0.5).to(dev)
+
+    def run(n):
+        rho = torch.nn.functional.softplus(ps[:n].float())
+        return jn.transition_pairwise_dense("low_rank_bilinear_route", Ws, None, Wt, None, w, None, None, None, None,
+                                            None, "softmax", 1.0, rho, src[:n], dst[:n], ps[:n], pv[:n], Ns, Nd)[1]
+
+    assert torch.equal(run(64)[:63], run(63))
