@@ -201,3 +201,10 @@ def test_dense_batch_chunks_causal(dev, chunk_batches, compress):
 
     chunk_batches(1, 200)
     TW.test_full_causal_window_runs_dense(dev, compress, True, 0)
+
+
+@pytest.mark.parametrize("r", [200, 256])
+def test_small_gradients_of_many_rows(dev, r):
+    """4,400 partial rows and 30,800 row sums: the two-stage sums of the scale
+    and bias gradients, 17 or 18 rows a thread (two unrolled groups and a rest)."""
+    _check_dense(dev, "softsign", True, 220, True, B=20, D=16, r=r)
