@@ -557,8 +557,9 @@ class DenseC4:
 
 class DenseC4Bf16(DenseC4):
     """c4-dense with bf16 layer states and values: the three N x N products
-    on bf16 MFMA (the edge matrix rounded to bf16 where it multiplies
-    values), the projections on the bf16 projection GEMMs."""
+    on bf16 MFMA in kernels that rebuild the edges tile by tile (rounded to
+    bf16 where they multiply values), the projections on the bf16 projection
+    GEMMs."""
 
     name = "c4-dense-bf16"
     metric = "routed pairs/sec + MFMA TFLOP/s (% peak), Propagation dense N=4096 D=512 r=64 fwd+bwd, bf16 activations"
@@ -572,14 +573,9 @@ class DenseC4Bf16(DenseC4):
     def model(self, name):
         c = self.config
         B, N, D, r = (c[x] for x in ("batch", "nodes", "dim", "rank"))
-        Bc = self.chunk_batch()
-        dense = {
-            "gemm_bf16_kernel<dense_aggregate_bf16>": 2.0 * Bc * N * N * D,
-            "gemm_bf16_kernel<dense_edge_grad_bf16>": 2.0 * Bc * N * N * D,
-            "gemm_bf16_kernel<dense_value_grad_bf16>": 2.0 * Bc * N * N * D,
-        }
-        if name in dense:
-            return "mfma", dense[name], None, BF16_MFMA_PEAK_TFLOPS
+        # no edge matrix: each kernel rebuilds its scores and holds one product over D
+        if name.startswith(("dense_aggregate_kernel", "dense_score_grad_kernel")):
+            return "mfma", 2.0 * B * N * N * D, None, BF16_MFMA_PEAK_TFLOPS
         if name.startswith("gemm_bf16_kernel"):
             return "mfma", 2.0 * B * N * D * 2 * r, None, BF16_MFMA_PEAK_TFLOPS
         return super().model(name)
