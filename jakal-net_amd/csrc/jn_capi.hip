@@ -550,7 +550,7 @@ int dense_backward(const float* layer_val, const float* projected_state, const f
     f.grad_projected_state = grad_projected_state ? grad_projected_state + pr : nullptr;
     f.grad_projected_val = gpv ? const_cast<float*>(value_rows(gpv, pr * D, true)) : nullptr;
     f.dP = s.dP + pr * 2 * r;
-    f.rowsum = s.rowsum + pr;
+    f.rowsum = s.rowsum + pr * parts;
     rc = launch_dense_fused_backward(f, st);
     if (rc) return rc;
     rc = launch_scale_grad_partials(s.dP + pr * 2 * r + r, 2 * r, projections + pr * 2 * r + r, 2 * r, core_weight, r,
@@ -663,7 +663,7 @@ int dense_backward(const float* layer_val, const float* projected_state, const f
                                     (int64_t)nb * N, s.part_c + pr * r, st);
     if (rc) return rc;
   }
-  const int64_t n_rowsum = fused && edgeless == 0 ? (int64_t)M * parts : M;
+  const int64_t n_rowsum = fused ? (int64_t)M * parts : M;
 
   // 4. projection weight and input grads
   if (grad_target_weight && grad_source_weight) {

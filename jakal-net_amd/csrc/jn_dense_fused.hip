@@ -14,20 +14,27 @@
 //     rows = targets: the target projection's gradient (and the row sums of G)
 //     rows = sources: the source projection's
 //
-// Arithmetic: the scores and G . P on three-term bf16 splits (x3_split: six
-// exact products, fp32 accuracy); E . V and gdv . pv^T on bf16 operands, E
-// rounded to bf16 as it enters the product; everything else in fp32.  Every sum
-// has a fixed order.
+// Arithmetic: that of the GEMMs over an edge matrix (jn_gemm.hip), product for
+// product and sum for sum, so a layer gives the same bits on either path (for
+// ranks in multiples of 4; delta_state where N <= 16 D): the scores one chain of
+// fp32 MFMAs over the ranks, E . V and gdv . pv^T on bf16 operands (E rounded
+// to bf16 as it enters the product), G . P four chains of fp32 MFMAs, the row
+// sums of E x and G in blocks of 32 columns, E^T . gds in sixteen chains.
 //
 // Measured at C4 sizes (16 x 4096 nodes, 512 values, rank 64, forward and
 // backward) against the GEMMs over edge matrices in two batch chunks: step 5.48
-// -> 2.85 ms; aggregate 0.42 and 0.41 ms (0.46 MFMA busy), score gradient 0.90
-// and 0.89 ms (0.31 MFMA busy).
+// -> 3.19 ms; aggregate 0.62 and 0.60 ms, score gradient 0.97 and 0.95 ms.  An
+// fp32 MFMA and vector instructions do not run side by side (33 cycles and 4.5
+// for each of them, a bf16 MFMA 18 and little more for one or two), so vector
+// work stands beside bf16 MFMAs or by itself.  The scores and G . P on
+// three-term bf16 splits were faster (2.84 ms), but further from 64 bits on the
+// same projections: delta_state 1.3 to 2.3 times as far as here, the projections'
+// gradients 1.6 to 4.6 times, the score scale's 1.4 to 2.1 times.
 //
-// The split operands are laid out by dense_planes_kernel and dense_pack_kernel
-// before: rows of three 64-rank planes, their transposes in blocks of 32 rows,
-// and value rows in MFMA fragment order.  Rows are padded to Npad (a multiple
-// of 128) with zeros, which contribute nothing.
+// The operands are laid out by dense_ranks_kernel and dense_pack_kernel before:
+// projections in fp32 MFMA fragment order, their transposes likewise, and value
+// rows in bf16 fragment order.  Rows are padded to Npad (a multiple of 128) with
+// zeros, which contribute nothing.
 #include "jn_internal.hpp"
 
 namespace jakal {
@@ -39,46 +46,35 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // (arrays of uint4
 constexpr int kDfRows = 128;             // rows of an aggregate workgroup
 constexpr int kDfThreads = 512;          // 8 waves of 16 rows (scores) or D / 8 columns (E . V)
 constexpr int kDfGradRows = 64;          // rows of a score-gradient workgroup
-constexpr int kDfGradThreads = 256;      // 4 waves: 2 row groups of 32 x 2 column groups of 16
-constexpr int kDfRank = 64;              // ranks of a plane row (zeros past the rank)
-constexpr int kDfPlaneRow = 3 * kDfRank; // elements of a row's planes: h, m, l
-constexpr int kDfFrag = 512;             // elements of an MFMA fragment: 64 lanes of 8
+constexpr int kDfGradThreads = 256;      // 4 waves of 16 rows
+constexpr int kDfRank = 64;              // ranks of a laid-out row (zeros past the rank)
+constexpr int kDfFrag = 512;             // elements of a bf16 MFMA fragment: 64 lanes of 8
+constexpr int kDfFragF = 256;            // elements of four fp32 MFMA fragments: 64 lanes of 4
+constexpr int kDfTile = 16 * kDfRank;    // elements of a 16-row tile of projections
+constexpr int kDfBlock = 32;             // columns per partial row sum (dense_epi_parts)
 
 // ---- operand layouts -----------------------------------------------------------
 
-// Rows [b][j] of one projection (stride ld, r ranks) into three-term planes in
-// MFMA fragment order, so that a wave's fragment is one contiguous kilobyte in
+// Rows [b][j] of one projection (stride ld, r ranks) in fp32 MFMA fragment
+// order, 16 rows at a time, so that a wave's load is one contiguous kilobyte in
 // global memory and in LDS (no bank conflicts):
-//   planes [b][Npad / 16][2][3][64 lanes][8]: rows times scale (or 1); lane l of
-//     a 16-row tile holds ranks 32 s + 8 (l / 16) .. + 7 of row l % 16;
-//   blocks [b][Npad / 32][4][3][64 lanes][8]: transposed, unscaled; lane l of a
-//     16-rank tile holds rows 8 (l / 16) .. + 7 of rank l % 16.
-// A workgroup takes 32 rows; blockIdx.z picks the projection (0: targets, with
-// the scale; 1: sources).
-struct DensePlanesArgs {
+//   ranks [b][Npad / 16][4][64 lanes][4]: rows times scale (or 1); lane l holds
+//     ranks 16 s + 4 (l / 16) .. + 3 of row l % 16;
+//   cols [b][Npad / 16][4][64 lanes][4]: unscaled; lane l holds rows
+//     4 (l / 16) .. + 3 of rank 16 s + l % 16.
+// Element q of the lanes' four is the operand of the q-th MFMA (the k order of
+// gemm_f32_kernel's fragments).  A workgroup takes 32 rows; blockIdx.z picks the
+// projection (0: targets, with the scale; 1: sources).
+struct DenseRanksArgs {
   const float* proj[2];
   int64_t ld;
-  const float* scale;  // of proj[0]'s planes
-  bf16_t* planes[2];
-  bf16_t* blocks[2];   // or null
+  const float* scale;  // of proj[0]'s ranks
+  float* ranks[2];
+  float* cols[2];      // or null
   int N, Npad, r;
 };
 
-// eight values into one lane's piece of the h, m and l fragments at `to`
-__device__ __forceinline__ void df_store_planes(const float (&x)[8], bf16_t* to) {
-  uint32_t h[8], m[8], l[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) x3_split(__float_as_uint(x[i]), h[i], m[i], l[i]);
-  auto put = [&](int plane, const uint32_t(&v)[8]) {
-    *reinterpret_cast<uint4*>(to + plane * kDfFrag) =
-        make_uint4(x3_pair(v[0], v[1]), x3_pair(v[2], v[3]), x3_pair(v[4], v[5]), x3_pair(v[6], v[7]));
-  };
-  put(0, h);
-  put(1, m);
-  put(2, l);
-}
-
-__global__ __launch_bounds__(256) void dense_planes_kernel(DensePlanesArgs a) {
+__global__ __launch_bounds__(256) void dense_ranks_kernel(DenseRanksArgs a) {
   __shared__ float tile[32][kDfRank + 1];
   const int z = blockIdx.z, b = blockIdx.y, j0 = blockIdx.x * 32, tid = threadIdx.x;
   const float* src = a.proj[z] + ((int64_t)b * a.N + j0) * a.ld;
@@ -87,23 +83,23 @@ __global__ __launch_bounds__(256) void dense_planes_kernel(DensePlanesArgs a) {
     tile[j][k] = j0 + j < a.N && k < a.r ? src[(int64_t)j * a.ld + k] : 0.f;
   }
   __syncthreads();
-  const int64_t base = ((int64_t)b * a.Npad + j0) * kDfPlaneRow;
-  float x[8];
-  {  // thread: row j, ranks k .. k + 7
-    const int j = tid / 8, k = tid % 8 * 8;
+  const int64_t base = ((int64_t)b * a.Npad + j0) * kDfRank;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      x[i] = tile[j][k + i];
-      if (z == 0) x[i] *= k + i < a.r ? a.scale[k + i] : 0.f;
+  for (int u = 0; u < 2; ++u) {  // one 16-row tile each
+    const int s = tid / 64, col = tid % 16, kg = tid % 64 / 16;
+    const int64_t at = base + u * kDfTile + tid * 4;
+    float x[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int k = 16 * s + 4 * kg + q;
+      x[q] = tile[u * 16 + col][k];
+      if (z == 0) x[q] *= k < a.r ? a.scale[k] : 0.f;
     }
-    df_store_planes(x, a.planes[z] + base + ((j / 16 * 2 + k / 32) * 3 * 64 + j % 16 + k % 32 / 8 * 16) * 8);
-  }
-  if (!a.blocks[z]) return;
-  {  // thread: rank k, rows j .. j + 7
-    const int k = tid / 4, j = tid % 4 * 8;
+    *reinterpret_cast<float4*>(a.ranks[z] + at) = make_float4(x[0], x[1], x[2], x[3]);
+    if (!a.cols[z]) continue;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = tile[j + i][k];
-    df_store_planes(x, a.blocks[z] + base + (k / 16 * 3 * 64 + k % 16 + j / 8 * 16) * 8);
+    for (int q = 0; q < 4; ++q) x[q] = tile[u * 16 + 4 * kg + q][16 * s + col];
+    *reinterpret_cast<float4*>(a.cols[z] + at) = make_float4(x[0], x[1], x[2], x[3]);
   }
 }
 
@@ -135,20 +131,11 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(const bf16_t* val, bf16
 
 // ---- shared pieces ---------------------------------------------------------------
 
-// 1 / y to within an ulp (y in [1, inf))
-__device__ __forceinline__ float recip_f(float y) {
-  const float r = __builtin_amdgcn_rcpf(y);
-  return r * (2.0f - y * r);
-}
-
-// c += a . b over one 32-wide K step of three-plane operands, the small terms first
-__device__ __forceinline__ floatx4 mfma_x3(const bf16x8v (&a)[3], const bf16x8v (&b)[3], floatx4 c) {
-  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[2], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[1], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[0], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], c, 0, 0, 0);
+// c += a . b over the 16 k of one laid-out piece (component q is MFMA q's)
+__device__ __forceinline__ floatx4 mfma_f32x4(floatx4 a, floatx4 b, floatx4 c) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], b[q], c, 0, 0, 0);
+  return c;
 }
 
 // which columns j row i keeps: all, j <= i, j >= i.  Causal kernels test without
@@ -166,15 +153,29 @@ __device__ __forceinline__ void df_tile(int Npad, int rows, int mode, int& b, in
   i0 = (mode == kDfLower ? per - 1 - t : t) * rows;
 }
 
+// a + b, never the tail of a fused multiply-add
+__device__ __forceinline__ float df_add(float a, float b) {
+#pragma clang fp contract(off)
+  return a + b;
+}
+
+// the sum of v over the four lanes of a row (lanes l, l ^ 16, l ^ 32, l ^ 48)
+__device__ __forceinline__ float df_row_sum(float v) {
+  v += xor16_f(v);
+  v += xor32_f(v);
+  return v;
+}
+
 // ---- E . V and E . x ---------------------------------------------------------------
 struct DenseAggregateArgs {
-  const bf16_t* rows;    // planes of the row operand (dense_planes_kernel)
-  const bf16_t* cols;    // planes of the column operand
+  const float* rows;     // ranks of the row operand (dense_ranks_kernel)
+  const float* cols;     // ranks of the column operand
   const bf16_t* values;  // packed values of the columns (dense_pack_kernel)
   const float* bias;     // scalar or null
   const float* x;        // [nb][N] of the columns
   bf16_t* out;           // [nb][N][D] or null
-  float* out_state;      // [nb][N] or null
+  float* parts;          // forward: [nb][N][ceil(N / 32)], the sums of E x per 32 columns
+  float* out_state;      // backward: [nb][N] or null
   int N, Npad, D, mode;
 };
 
@@ -182,15 +183,17 @@ struct DenseAggregateArgs {
 // so that a lane holds four consecutive columns of one row: its edges go to LDS
 // as 8-byte pieces of the aggregate's B fragments, whose A operand (the packed
 // values: every wave owns D / 8 columns of V) loads straight into fragments.
-// Two buffers each for the column planes and the edges: one barrier per step,
+// Two buffers each for the column ranks and the edges: one barrier per step,
 // and a wave may run its scores beside another's aggregate.
-// Bound: MFMA (per 128 x 64 edges and SIMD 1536 cycles of scores, 2048 of
-// aggregate at D = 512) plus the softsign's VALU work.
-template <int NTW, int KS, bool CAUSAL>
+// Bound: MFMA (per 128 x 64 edges and SIMD 4096 cycles of scores at rank 64,
+// 2048 of aggregate at D = 512) plus the softsign's VALU work.
+// KB: pieces of 16 ranks.  BWD: E . x in sixteen chains (colsum_rows_kernel's
+// order), else in blocks of 32 columns (the order of the scores' epilogue).
+template <int NTW, int KB, bool CAUSAL, bool BWD>
 __global__ __launch_bounds__(kDfThreads) void dense_aggregate_kernel(DenseAggregateArgs a) {
   constexpr int CT = 64;
-  __shared__ __align__(16) bf16_t planes[2][CT * kDfPlaneRow];  // [4 tiles][2][3] fragments
-  __shared__ __align__(16) bf16_t edges[2][16 * kDfFrag];       // [8 row tiles][2] fragments
+  __shared__ __align__(16) float ranks[2][4 * KB * kDfFragF];  // [4 tiles][KB] pieces
+  __shared__ __align__(16) bf16_t edges[2][16 * kDfFrag];      // [8 row tiles][2] fragments
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const int col = lane & 15, kg = lane >> 4;
   int b, i0;
@@ -200,24 +203,27 @@ __global__ __launch_bounds__(kDfThreads) void dense_aggregate_kernel(DenseAggreg
   const float bias = a.bias ? a.bias[0] : 0.f;
 
   const int row = wave * 16 + col;  // of the scores
-  bf16x8v q[KS][3];
+  floatx4 q[KB];
 #pragma unroll
-  for (int s = 0; s < KS; ++s)
-#pragma unroll
-    for (int p = 0; p < 3; ++p)
-      q[s][p] = *reinterpret_cast<const bf16x8v*>(
-          a.rows + ((int64_t)b * a.Npad + i0 + wave * 16) * kDfPlaneRow + (s * 3 + p) * kDfFrag + lane * 8);
+  for (int s = 0; s < KB; ++s)
+    q[s] = *reinterpret_cast<const floatx4*>(a.rows + ((int64_t)b * a.Npad + i0 + wave * 16) * kDfRank +
+                                             s * kDfFragF + lane * 4);
 
-  const u32x4* cols = reinterpret_cast<const u32x4*>(a.cols + (int64_t)b * a.Npad * kDfPlaneRow);
+  // a step's column ranks: 4 tiles of 256 16-byte words, of which KB / 4 hold ranks
+  constexpr int SN = 4 * KB * 64 / kDfThreads;
+  const u32x4* cols = reinterpret_cast<const u32x4*>(a.cols + (int64_t)b * a.Npad * kDfRank);
   const auto rs_x = make_rsrc(a.x + (int64_t)b * a.N, (uint32_t)a.N * 4u);
-  u32x4 stage[3];
-  auto load = [&](int j0) {  // the planes of 64 rows are 24 KB in one piece
+  u32x4 stage[SN];
+  auto load = [&](int j0) {
 #pragma unroll
-    for (int u = 0; u < 3; ++u) stage[u] = cols[(int64_t)j0 * (kDfPlaneRow / 8) + tid + kDfThreads * u];
+    for (int u = 0; u < SN; ++u) {
+      const int e = tid + kDfThreads * u;
+      stage[u] = cols[(int64_t)j0 * (kDfRank / 4) + e / (KB * 64) * (kDfTile / 4) + e % (KB * 64)];
+    }
   };
   auto store = [&](int buf) {
 #pragma unroll
-    for (int u = 0; u < 3; ++u) reinterpret_cast<u32x4*>(planes[buf])[tid + kDfThreads * u] = stage[u];
+    for (int u = 0; u < SN; ++u) reinterpret_cast<u32x4*>(ranks[buf])[tid + kDfThreads * u] = stage[u];
   };
 
   floatx4 acc[NTW][8];
@@ -225,15 +231,20 @@ __global__ __launch_bounds__(kDfThreads) void dense_aggregate_kernel(DenseAggreg
   for (int d = 0; d < NTW; ++d)
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[d][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float rsum = 0.f;
+  float chain[4] = {0.f, 0.f, 0.f, 0.f};  // BWD: columns 4 kg + w (mod 16)
+  float hold = 0.f;                       // else: the sum of block 4 n + kg of the last four
+  const int P = (a.N + kDfBlock - 1) / kDfBlock;
 
+  __builtin_amdgcn_sched_barrier(0);  // the rows' ranks arrive before the loop
   load(jbeg);
   store(0);
   __syncthreads();
   int buf = 0;
   for (int j0 = jbeg; j0 < jend; j0 += CT, buf ^= 1) {
     const bool more = j0 + CT < jend;
-    if (more) load(j0 + CT);
+    float4 xs[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) xs[t] = buf_load4(rs_x, (uint32_t)(j0 + t * 16 + kg * 4) * 4u);
     bf16x8v v[2][NTW];
 #pragma unroll
     for (int s = 0; s < 2; ++s)
@@ -242,32 +253,58 @@ __global__ __launch_bounds__(kDfThreads) void dense_aggregate_kernel(DenseAggreg
         v[s][d] = *reinterpret_cast<const bf16x8v*>(
             a.values + (((int64_t)b * (a.Npad / 32) + j0 / 32 + s) * (a.D / 16) + wave * NTW + d) * 512 + lane * 8);
 
+    load(more ? j0 + CT : j0);  // (the last step's again: a branch would make every wait one for all loads)
+    __builtin_amdgcn_sched_barrier(0);
+    float half = 0.f;
+    auto scores = [&](int t) {  // 16 columns
+      floatx4 c = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {  // 16 columns
+      for (int s = 0; s < KB; ++s)
+        c = mfma_f32x4(*reinterpret_cast<const floatx4*>(&ranks[buf][(t * KB + s) * kDfFragF + lane * 4]), q[s], c);
+      return c;
+    };
+    floatx4 sc[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) sc[t] = scores(t);
+    __builtin_amdgcn_sched_barrier(0);  // (vector work among fp32 MFMAs runs beside none of them)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
       const int j = t * 16 + kg * 4;
-      const float4 x = buf_load4(rs_x, (uint32_t)(j0 + j) * 4u);
-      floatx4 sc = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        bf16x8v c[3];
-#pragma unroll
-        for (int p = 0; p < 3; ++p)
-          c[p] = *reinterpret_cast<const bf16x8v*>(&planes[buf][((t * 2 + s) * 3 + p) * kDfFrag + lane * 8]);
-        sc = mfma_x3(c, q[s], sc);
-      }
+      const float4 x = xs[t];
       float e[4];
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
-        const float s = sc[w] + bias;
-        e[w] = s * recip_f(1.0f + fabsf(s));
+        e[w] = softsign_f(sc[t][w] + bias);
         if constexpr (CAUSAL) e[w] = df_keep(a.mode, i0 + row, j0 + j + w) ? e[w] : 0.f;
       }
-      rsum += (e[0] * x.x + e[1] * x.y) + (e[2] * x.z + e[3] * x.w);
+      const float xv[4] = {x.x, x.y, x.z, x.w};
+      if constexpr (BWD) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) chain[w] = fmaf(xv[w], e[w], chain[w]);
+      } else {
+        float p = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) p = fmaf(e[w], xv[w], p);
+        p = df_row_sum(p);
+        if (t % 2 == 0) {
+          half = p;
+        } else {
+          const int blk = j0 / kDfBlock + t / 2;
+          hold = (blk & 3) == kg ? half + p : hold;
+        }
+      }
       *reinterpret_cast<uint2*>(&edges[buf][(wave * 2 + t / 2) * kDfFrag + (col + (t % 2 * 2 + kg / 2) * 16) * 8 +
                                             kg % 2 * 4]) =
           make_uint2(pack_bf16x2(e[0], e[1]), pack_bf16x2(e[2], e[3]));
     }
-    if (more) store(buf ^ 1);
+    if constexpr (!BWD) {
+      if ((j0 & CT) != 0 || !more) {  // four blocks (or the last) are summed
+        const int blk = (j0 / (2 * CT)) * 4 + kg;
+        if (i0 + row < a.N && blk < P && blk * kDfBlock < j0 + CT)
+          a.parts[((int64_t)b * a.N + i0 + row) * P + blk] = hold;
+      }
+    }
+    store(buf ^ 1);
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -291,16 +328,27 @@ __global__ __launch_bounds__(kDfThreads) void dense_aggregate_kernel(DenseAggreg
       *reinterpret_cast<uint2*>(out + d * 16) =
           make_uint2(pack_bf16x2(acc[d][i][0], acc[d][i][1]), pack_bf16x2(acc[d][i][2], acc[d][i][3]));
   }
-  rsum += xor16_f(rsum);
-  rsum += xor32_f(rsum);
-  if (a.out_state && kg == 0 && i0 + row < a.N) a.out_state[(int64_t)b * a.N + i0 + row] = rsum;
+  if constexpr (BWD) {
+    // the sixteen chains of a row in order: kg, then w
+    float s = 0.f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float u = (((s + chain[0]) + chain[1]) + chain[2]) + chain[3];
+      s = __shfl(u, col + 16 * g);
+    }
+    if (a.out_state && kg == 0 && i0 + row < a.N) a.out_state[(int64_t)b * a.N + i0 + row] = s;
+  } else if constexpr (CAUSAL) {  // the blocks past the row's last column are empty
+    if (i0 + row < a.N)
+      for (int blk = (jend + kDfBlock - 1) / kDfBlock + kg; blk < P; blk += 4)
+        a.parts[((int64_t)b * a.N + i0 + row) * P + blk] = 0.f;
+  }
 }
 
 // ---- G . P ---------------------------------------------------------------------------
 struct DenseScoreGradArgs {
-  const bf16_t* rows;     // planes of the row operand (dense_planes_kernel)
-  const bf16_t* cols;     // planes of the column operand
-  const bf16_t* blocks;   // transposed planes of the columns' raw projections
+  const float* rows;      // ranks of the row operand (dense_ranks_kernel)
+  const float* cols;      // ranks of the column operand
+  const float* proj;      // transposed raw projections of the columns (dense_ranks_kernel)
   const bf16_t* row_val;  // [nb][N][D]
   const bf16_t* col_val;  // [nb][N][D]
   const float* row_x;     // [nb][N]
@@ -309,29 +357,32 @@ struct DenseScoreGradArgs {
   const float* out_scale; // [r] or null
   float* out;             // [nb][N] rows of stride ld: r values each
   int64_t ld;
-  float* rowsum;          // [nb][N] or null: sums of G over the columns
+  float* parts;           // [nb][N][ceil(N / 32)] or null: the sums of G per 32 columns
   int N, Npad, r, mode;
 };
 
-// 32 columns per step, everything transposed as above.  The rows' value
-// fragments stay in registers (2 x D / 32 of them), their score planes in LDS;
-// the columns' values are staged in LDS (pieces of a row exchanged by its row
-// number, so that 16 rows' pieces lie in distinct banks), the columns' planes
-// and transposed planes load straight into fragments.  64 rows per workgroup:
-// 70 KB of LDS, so that two share a CU and one's barriers and LDS phases run
-// beside the other's MFMAs (128 rows in one workgroup of eight waves: 1.03 ms
-// against 0.90 at C4; in one of four waves of 32 x 32: 1.6).
-// Bound: MFMA (per 128 x 32 pairs and SIMD 768 cycles of scores, 1024 of
-// gdv . pv^T at D = 512, 768 of G . P), the VALU work of the derivative and of
-// splitting G, and LDS reads (2200 cycles).
-template <int NK, int KS, bool CAUSAL>
+// 32 columns per step; a wave owns 16 rows and all of them.  Everything is taken
+// transposed as above, so that the four columns of a row that a lane's G holds
+// are component by component the operands of the four G . P chains: G never
+// leaves its registers.  The rows' value fragments stay in registers; the
+// columns' values (pieces of a row exchanged by its row number, so that 16 rows'
+// pieces lie in distinct banks), ranks and transposed projections are staged in
+// LDS.  64 rows per workgroup and 48 KB of LDS at D = 512: two share a CU, and
+// one's barriers and LDS phases run beside the other's MFMAs.
+// Bound: MFMA (per 64 x 32 pairs and SIMD 1024 cycles of scores and 1024 of
+// G . P at rank 64, 512 of gdv . pv^T at D = 512) and LDS reads (1500 cycles).
+template <int NK, int KB, bool CAUSAL>
 __global__ __launch_bounds__(kDfGradThreads, 2) void dense_score_grad_kernel(DenseScoreGradArgs a) {
   constexpr int D = NK * 32, CT = 32;
-  __shared__ __align__(16) bf16_t qs[kDfGradRows * kDfPlaneRow];   // rows' planes: [4 tiles][2][3] fragments
-  __shared__ __align__(16) bf16_t vals[CT * D];                    // columns' values: rows of swizzled pieces
-  __shared__ __align__(16) bf16_t gs[kDfGradRows / 16 * 3 * kDfFrag];  // G: [4 row tiles][3] fragments
+  constexpr int VP = D / 8, VS = VP + 1;                       // 16-byte words of a row of values, and in LDS
+  __shared__ __align__(16) u32x4 vals[CT * VS];                // columns' values (16 rows' words in distinct banks)
+  __shared__ __align__(16) float ranks[2 * KB * kDfFragF];     // [2 tiles][KB] pieces
+  __shared__ __align__(16) float proj[2 * KB * kDfFragF];
+  // the rows' ranks: in registers, or in LDS where those would spill
+  constexpr bool ROWS_LDS = NK == 16 && KB == 4;
+  __shared__ __align__(16) float rows[ROWS_LDS ? kDfGradRows * kDfRank : 4];
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
-  const int wr = wave >> 1, wc = wave & 1, col = lane & 15, kg = lane >> 4;
+  const int col = lane & 15, kg = lane >> 4;
   int b, i0;
   df_tile(a.Npad, kDfGradRows, a.mode, b, i0);
   const int jbeg = a.mode == kDfUpper ? i0 : 0;
@@ -346,187 +397,199 @@ __global__ __launch_bounds__(kDfGradThreads, 2) void dense_score_grad_kernel(Den
     return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
   };
 
-  bf16x8v rv[2][NK];  // this wave's 32 rows of values
-  float rx[2];
+  const int row = i0 + wave * 16 + col;
+  bf16x8v rv[NK];  // this lane's pieces of its row of values
 #pragma unroll
-  for (int n = 0; n < 2; ++n) {
-    const int i = i0 + wr * 32 + n * 16 + col;
-    rx[n] = buf_load1(rs_rx, (uint32_t)i * 4u);
+  for (int s = 0; s < NK; ++s)
+    rv[s] = __builtin_bit_cast(bf16x8v, load16(rs_rv, (uint32_t)row * (D * 2u) + s * 64u + kg * 16u));
+  const float rx = buf_load1(rs_rx, (uint32_t)row * 4u);
+  floatx4 qr[KB];
+  floatx4* ql = reinterpret_cast<floatx4*>(rows) + (ROWS_LDS ? wave * KB * 64 : 0);  // this wave's, own to it
 #pragma unroll
-    for (int s = 0; s < NK; ++s)
-      rv[n][s] = __builtin_bit_cast(bf16x8v, load16(rs_rv, (uint32_t)i * (D * 2u) + s * 64u + kg * 16u));
-  }
-  {
-    const uint4* src = reinterpret_cast<const uint4*>(a.rows + ((int64_t)b * a.Npad + i0) * kDfPlaneRow);
-    for (int e = tid; e < kDfGradRows * kDfPlaneRow / 8; e += kDfGradThreads) reinterpret_cast<uint4*>(qs)[e] = src[e];
+  for (int s = 0; s < KB; ++s) {
+    qr[s] = *reinterpret_cast<const floatx4*>(a.rows + ((int64_t)b * a.Npad + i0 + wave * 16) * kDfRank +
+                                              s * kDfFragF + lane * 4);
+    if constexpr (ROWS_LDS) ql[s * 64 + lane] = qr[s];
   }
 
-  constexpr int VN = CT * D / 8 / kDfGradThreads, VP = D / 8;  // 16-byte pieces: per thread of a tile, of a row
-  u32x4 sv[VN];
+  // 16-byte words per thread of a step's values, and of its two tiles of 256
+  // words of ranks and projections, of which KB / 4 are in use
+  constexpr int VN = CT * VP / kDfGradThreads, RN = 2 * KB * 64 / kDfGradThreads;
+  const uint32_t operand = (uint32_t)a.Npad * (kDfRank * 4u);
+  const auto rs_c = make_rsrc(a.cols + (int64_t)b * a.Npad * kDfRank, operand);
+  const auto rs_p = make_rsrc(a.proj + (int64_t)b * a.Npad * kDfRank, operand);
+  u32x4 sv[VN], sc[RN], sp[RN];
   auto load = [&](int j0) {
 #pragma unroll
     for (int u = 0; u < VN; ++u)
       sv[u] = load16(rs_cv, (uint32_t)j0 * (D * 2u) + (uint32_t)(tid + kDfGradThreads * u) * 16u);
+#pragma unroll
+    for (int u = 0; u < RN; ++u) {
+      const int tile = kDfGradThreads * u / (KB * 64);  // (wave-uniform: KB is 4, or RN is 1 and the tile tid / 128)
+      const uint32_t off = KB == 4 ? (uint32_t)tid * 16u : (uint32_t)(tid / 128 * 256 + tid % 128) * 16u;
+      const uint32_t at = (uint32_t)j0 * (kDfRank * 4u) + (uint32_t)tile * (kDfTile * 4u);
+      sc[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_c, off, at, 0));
+      sp[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_p, off, at, 0));
+    }
   };
   auto store = [&]() {
 #pragma unroll
     for (int u = 0; u < VN; ++u) {
-      const int e = tid + kDfGradThreads * u, j = e / VP, p = e % VP;
-      reinterpret_cast<u32x4*>(vals)[j * VP + (p ^ (j & 15))] = sv[u];
+      const int e = tid + kDfGradThreads * u;
+      vals[e / VP * VS + e % VP] = sv[u];
+    }
+#pragma unroll
+    for (int u = 0; u < RN; ++u) {
+      reinterpret_cast<u32x4*>(ranks)[tid + kDfGradThreads * u] = sc[u];
+      reinterpret_cast<u32x4*>(proj)[tid + kDfGradThreads * u] = sp[u];
     }
   };
 
-  floatx4 acc[2][2];  // 32 ranks (wc) x 32 rows
+  floatx4 acc[KB][4];  // 16 ranks x 16 rows, four chains
 #pragma unroll
-  for (int m = 0; m < 2; ++m)
+  for (int m = 0; m < KB; ++m)
 #pragma unroll
-    for (int n = 0; n < 2; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float rsum[2] = {0.f, 0.f}, rpart[2] = {0.f, 0.f};
-  const bf16_t* cols = a.cols + (int64_t)b * a.Npad * kDfPlaneRow + lane * 8;
-  const bf16_t* blocks = a.blocks + (int64_t)b * a.Npad * kDfPlaneRow + lane * 8;
+    for (int c = 0; c < 4; ++c) acc[m][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  float hold = 0.f;  // the sum of block 4 n + kg of the last four
+  const int P = (a.N + kDfBlock - 1) / kDfBlock;
+  float* parts = a.parts && row < a.N ? a.parts + ((int64_t)b * a.N + row) * P : nullptr;
 
   load(jbeg);
-  int step = 0;
-  for (int j0 = jbeg; j0 < jend; j0 += CT, ++step) {
+  for (int j0 = jbeg; j0 < jend; j0 += CT) {
     __syncthreads();  // the step before is consumed
     store();
     __syncthreads();
-    if (j0 + CT < jend) load(j0 + CT);
-    const float4 cx = buf_load4(rs_cx, (uint32_t)(j0 + wc * 16 + kg * 4) * 4u);
-    bf16x8v c[KS][3];
+    const bool more = j0 + CT < jend;
+    float4 cx[2];
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int p = 0; p < 3; ++p)
-        c[s][p] = *reinterpret_cast<const bf16x8v*>(cols + (int64_t)(j0 + wc * 16) * kDfPlaneRow +
-                                                    (s * 3 + p) * kDfFrag);
+    for (int t = 0; t < 2; ++t) cx[t] = buf_load4(rs_cx, (uint32_t)(j0 + t * 16 + kg * 4) * 4u);
+    load(more ? j0 + CT : j0);  // (the last step's again: a branch would make every wait one for all loads)
+    __builtin_amdgcn_sched_barrier(0);
 
-    // gdv . pv^T and the scores: 16 columns (wc) x 32 rows
-    floatx4 sc[2], gv[2];
+    // the scores of 2 x 16 columns x 16 rows, and gdv . pv^T
+    auto scores = [&](int t) {
+      floatx4 c = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int n = 0; n < 2; ++n) sc[n] = gv[n] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int s = 0; s < KB; ++s)
+        c = mfma_f32x4(*reinterpret_cast<const floatx4*>(&ranks[(t * KB + s) * kDfFragF + lane * 4]),
+                       ROWS_LDS ? ql[s * 64 + lane] : qr[s], c);
+      return c;
+    };
+    auto slope = [&](floatx4 c) {  // 1 - |edge|
 #pragma unroll
-    for (int s = 0; s < NK; ++s) {
-      const bf16x8v v =
-          reinterpret_cast<const bf16x8v*>(vals)[(wc * 16 + col) * VP + ((s * 4 + kg) ^ col)];
+      for (int w = 0; w < 4; ++w) c[w] = 1.0f - fabsf(softsign_f(c[w] + bias));
+      return c;
+    };
+    floatx4 g[2], d[2];
+    d[0] = scores(0);
+    d[1] = scores(1);
+    __builtin_amdgcn_sched_barrier(0);
+    g[0] = g[1] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int n = 0; n < 2; ++n) gv[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, rv[n][s], gv[n], 0, 0, 0);
+    for (int s = 0; s < NK; ++s)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        g[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8v, vals[(t * 16 + col) * VS + s * 4 + kg]), rv[s], g[t], 0, 0, 0);
+    d[0] = slope(d[0]);
+    d[1] = slope(d[1]);
+    // four reads ahead of the MFMAs, the slopes beside them
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads
+#pragma unroll
+    for (int i = 0; i < 2 * NK - 4; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // VALU
     }
+    __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int n = 0; n < 2; ++n) {
-        bf16x8v q[3];
-#pragma unroll
-        for (int p = 0; p < 3; ++p)
-          q[p] = *reinterpret_cast<const bf16x8v*>(&qs[(((wr * 2 + n) * 2 + s) * 3 + p) * kDfFrag + lane * 8]);
-        sc[n] = mfma_x3(c[s], q, sc[n]);
-      }
-    bf16x8v t[2][3];
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-#pragma unroll
-      for (int p = 0; p < 3; ++p)
-        t[m][p] = *reinterpret_cast<const bf16x8v*>(blocks + (int64_t)j0 * kDfPlaneRow +
-                                                    ((wc * 2 + m) * 3 + p) * kDfFrag);
-    const float cxv[4] = {cx.x, cx.y, cx.z, cx.w};
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      uint32_t h[4], mi[4], l[4];
-      float g[4];
+    for (int t = 0; t < 2; ++t) {
+      const float cxv[4] = {cx[t].x, cx[t].y, cx[t].z, cx[t].w};
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
-        const float d = recip_f(1.0f + fabsf(sc[n][w] + bias));  // 1 - |softsign|
-        g[w] = (gv[n][w] + rx[n] * cxv[w]) * d * d;
-        if constexpr (CAUSAL)
-          g[w] = df_keep(a.mode, i0 + wr * 32 + n * 16 + col, j0 + wc * 16 + kg * 4 + w) ? g[w] : 0.f;
-        x3_split(__float_as_uint(g[w]), h[w], mi[w], l[w]);
-      }
-      rpart[n] += (g[0] + g[1]) + (g[2] + g[3]);
-      bf16_t* to = &gs[(wr * 2 + n) * 3 * kDfFrag + (col + (wc * 2 + kg / 2) * 16) * 8 + kg % 2 * 4];
-      *reinterpret_cast<uint2*>(to) = make_uint2(x3_pair(h[0], h[1]), x3_pair(h[2], h[3]));
-      *reinterpret_cast<uint2*>(to + kDfFrag) = make_uint2(x3_pair(mi[0], mi[1]), x3_pair(mi[2], mi[3]));
-      *reinterpret_cast<uint2*>(to + 2 * kDfFrag) = make_uint2(x3_pair(l[0], l[1]), x3_pair(l[2], l[3]));
-    }
-    if ((step & 7) == 7) {  // short partial sums: their rounding does not grow with N
-#pragma unroll
-      for (int n = 0; n < 2; ++n) {
-        rsum[n] += rpart[n];
-        rpart[n] = 0.f;
+        float x = fmaf(rx, cxv[w], g[t][w]) * d[t][w] * d[t][w];
+        if constexpr (CAUSAL) x = df_keep(a.mode, row, j0 + t * 16 + kg * 4 + w) ? x : 0.f;
+        g[t][w] = x;
       }
     }
-    __syncthreads();
-    // G . P: 32 ranks (wc) x 32 rows (wr) over the 32 columns
+    if (a.parts) {  // the row's sum over the block, in the order of the score gradient's epilogue
+      float s[4];
 #pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      bf16x8v g[3];
-#pragma unroll
-      for (int p = 0; p < 3; ++p)
-        g[p] = *reinterpret_cast<const bf16x8v*>(&gs[((wr * 2 + n) * 3 + p) * kDfFrag + lane * 8]);
-#pragma unroll
-      for (int m = 0; m < 2; ++m) acc[m][n] = mfma_x3(t[m], g, acc[m][n]);
+      for (int w = 0; w < 4; ++w) s[w] = df_add(g[0][w], g[1][w]);
+      const float sum = df_row_sum(df_add(df_add(s[0], s[1]), df_add(s[2], s[3])));
+      const int blk = j0 / kDfBlock;
+      hold = (blk & 3) == kg ? sum : hold;
+      if (parts && ((blk & 3) == 3 || !more) && (blk & ~3) + kg <= blk) parts[(blk & ~3) + kg] = hold;
     }
+    // G . P: all ranks x 16 rows over the 32 columns
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int m = 0; m < KB; ++m) {
+        const floatx4 p = *reinterpret_cast<const floatx4*>(&proj[(t * KB + m) * kDfFragF + lane * 4]);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[c], g[t][c], acc[m][c], 0, 0, 0);
+      }
   }
 
-#pragma unroll
-  for (int n = 0; n < 2; ++n) {
-    const int row = i0 + wr * 32 + n * 16 + col;
-    if (row >= a.N) continue;
+  if (row < a.N) {
     float* out = a.out + ((int64_t)b * a.N + row) * a.ld;
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
+    for (int m = 0; m < KB; ++m)
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
-        const int k = wc * 32 + m * 16 + kg * 4 + w;
-        if (k < a.r) out[k] = a.out_scale ? acc[m][n][w] * a.out_scale[k] : acc[m][n][w];
+        const int k = m * 16 + kg * 4 + w;
+        const float x = (acc[m][0][w] + acc[m][1][w]) + (acc[m][2][w] + acc[m][3][w]);
+        if (k < a.r) out[k] = a.out_scale ? x * a.out_scale[k] : x;
       }
   }
-  if (!a.rowsum) return;
-  __syncthreads();  // the rows' planes are no longer read
-  float* state = reinterpret_cast<float*>(qs);
-#pragma unroll
-  for (int n = 0; n < 2; ++n) {
-    float s = rsum[n] + rpart[n];
-    s += xor16_f(s);
-    s += xor32_f(s);
-    if (kg == 0) state[wc * kDfGradRows + wr * 32 + n * 16 + col] = s;
+  if constexpr (CAUSAL) {  // the blocks past the row's last column are empty
+    if (parts)
+      for (int blk = (jend + kDfBlock - 1) / kDfBlock + kg; blk < P; blk += 4) parts[blk] = 0.f;
   }
-  __syncthreads();
-  if (tid < kDfGradRows && i0 + tid < a.N) a.rowsum[(int64_t)b * a.N + i0 + tid] = state[tid] + state[kDfGradRows + tid];
 }
 
 // ---- host ------------------------------------------------------------------------------
 static int64_t df_npad(int64_t N) { return (N + kDfRows - 1) / kDfRows * kDfRows; }
 
-// bytes of the operand layouts of one batch element (each 256-byte aligned by Npad's size)
+// bytes of one batch element's layouts (a multiple of 256): the ranks of both
+// projections, the packed values, and the transposed projections (backward) or
+// the partial state sums (forward)
 static size_t df_element_bytes(int64_t N, int64_t D) {
-  return (size_t)df_npad(N) * (4 * kDfPlaneRow * sizeof(bf16_t) + (size_t)D * sizeof(bf16_t));
+  const size_t rows = (size_t)df_npad(N), ranks = 2 * kDfRank * sizeof(float);
+  return rows * (ranks + (size_t)D * sizeof(bf16_t)) +
+         std::max(rows * ranks, rows * dense_epi_parts((int)N) * sizeof(float));
 }
 
 // Whole 128-column pieces of value rows (at most 512: a wave's accumulators),
-// one plane of ranks, 32-bit offsets, and scratch for a batch element at least.
+// up to 64 ranks, 32-bit offsets, at least 512 nodes (the smallest measured) and
+// scratch for a batch element at least.
 int64_t dense_fused_batch(int64_t batch, int64_t N, int64_t D, int64_t r, int compress_kind, size_t scratch_bytes) {
-  if (compress_kind != 0 || r > kDfRank || D % 128 != 0 || D > 512 || N < 128 || N * D * 2 >= (1LL << 31)) return 0;
+  if (compress_kind != 0 || r > kDfRank || D % 128 != 0 || D > 512 || N < 512 || N * D * 2 >= (1LL << 31)) return 0;
   const int64_t fit = (int64_t)(scratch_bytes / df_element_bytes(N, D));
   const int64_t nb = std::min(batch, fit);
   return std::min<int64_t>(nb, 65535);
 }
 
 struct DenseLayouts {
-  bf16_t* planes[2];  // targets (scaled), sources
-  bf16_t* blocks[2];
+  float* ranks[2];  // targets (scaled), sources
+  float* cols[2];   // backward
+  float* parts;     // forward: in the place of cols
   bf16_t* packed;
 };
 
-static DenseLayouts df_carve(void* scratch, int nb, int64_t Npad) {
+static DenseLayouts df_carve(void* scratch, int nb, int64_t Npad, int64_t D) {
   DenseLayouts l{};
-  bf16_t* p = static_cast<bf16_t*>(scratch);
-  const int64_t one = (int64_t)nb * Npad * kDfPlaneRow;
-  l.planes[0] = p;
-  l.planes[1] = p + one;
-  l.blocks[0] = p + 2 * one;
-  l.blocks[1] = p + 3 * one;
-  l.packed = p + 4 * one;
+  float* p = static_cast<float*>(scratch);
+  const int64_t one = (int64_t)nb * Npad * kDfRank;
+  l.ranks[0] = p;
+  l.ranks[1] = p + one;
+  l.packed = reinterpret_cast<bf16_t*>(p + 2 * one);
+  l.parts = p + 2 * one + (int64_t)nb * Npad * D / 2;
+  l.cols[0] = l.parts;
+  l.cols[1] = l.parts + one;
   return l;
 }
 
@@ -537,21 +600,21 @@ static int df_prepare(const DenseFused& f, const DenseLayouts& l, int Npad, cons
   JN_REQUIRE(df_aligned(values) && df_aligned(f.projected_val) && df_aligned(f.scratch) && df_aligned(f.delta_val) &&
                  df_aligned(f.grad_projected_val),
              kUnsupported, "bf16 dense layers need 16-byte aligned operands");
-  DensePlanesArgs a{};
+  DenseRanksArgs a{};
   a.proj[0] = f.projections;
   a.proj[1] = f.projections + f.r;
   a.ld = 2 * f.r;
   a.scale = f.core_weight;
   for (int z = 0; z < 2; ++z) {
-    a.planes[z] = l.planes[z];
-    a.blocks[z] = transposed ? l.blocks[z] : nullptr;
+    a.ranks[z] = l.ranks[z];
+    a.cols[z] = transposed ? l.cols[z] : nullptr;
   }
   a.N = f.N;
   a.Npad = Npad;
   a.r = f.r;
   {
-    JN_PROFILE("dense_planes_kernel", stream);
-    hipLaunchKernelGGL(dense_planes_kernel, dim3(Npad / 32, f.nb, 2), dim3(256), 0, stream, a);
+    JN_PROFILE("dense_ranks_kernel", stream);
+    hipLaunchKernelGGL(dense_ranks_kernel, dim3(Npad / 32, f.nb, 2), dim3(256), 0, stream, a);
     JN_LAUNCH_CHECK();
   }
   JN_PROFILE("dense_pack_kernel", stream);
@@ -561,77 +624,81 @@ static int df_prepare(const DenseFused& f, const DenseLayouts& l, int Npad, cons
   return kOk;
 }
 
-template <int NTW>
-static void df_launch_aggregate(const DenseAggregateArgs& a, int nb, int r, hipStream_t stream) {
+template <int NTW, int KB>
+static void df_launch_aggregate(const DenseAggregateArgs& a, int nb, bool backward, hipStream_t stream) {
   const dim3 grid(nb * (a.Npad / kDfRows)), block(kDfThreads);
   const bool causal = a.mode != kDfAll;
-  if (r <= 32 && causal) hipLaunchKernelGGL((dense_aggregate_kernel<NTW, 1, true>), grid, block, 0, stream, a);
-  else if (r <= 32) hipLaunchKernelGGL((dense_aggregate_kernel<NTW, 1, false>), grid, block, 0, stream, a);
-  else if (causal) hipLaunchKernelGGL((dense_aggregate_kernel<NTW, 2, true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((dense_aggregate_kernel<NTW, 2, false>), grid, block, 0, stream, a);
+  if (backward && causal) hipLaunchKernelGGL((dense_aggregate_kernel<NTW, KB, true, true>), grid, block, 0, stream, a);
+  else if (backward) hipLaunchKernelGGL((dense_aggregate_kernel<NTW, KB, false, true>), grid, block, 0, stream, a);
+  else if (causal) hipLaunchKernelGGL((dense_aggregate_kernel<NTW, KB, true, false>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((dense_aggregate_kernel<NTW, KB, false, false>), grid, block, 0, stream, a);
 }
 
-static int df_aggregate(const DenseAggregateArgs& a, int nb, int r, const char* name, hipStream_t stream) {
+static int df_aggregate(const DenseAggregateArgs& a, int nb, int r, bool backward, const char* name,
+                        hipStream_t stream) {
   JN_PROFILE(name, stream);
+  const bool low = r <= 32;
   switch (a.D / 128) {
-    case 1: df_launch_aggregate<1>(a, nb, r, stream); break;
-    case 2: df_launch_aggregate<2>(a, nb, r, stream); break;
-    case 3: df_launch_aggregate<3>(a, nb, r, stream); break;
-    default: df_launch_aggregate<4>(a, nb, r, stream); break;
+    case 1: (low ? df_launch_aggregate<1, 2> : df_launch_aggregate<1, 4>)(a, nb, backward, stream); break;
+    case 2: (low ? df_launch_aggregate<2, 2> : df_launch_aggregate<2, 4>)(a, nb, backward, stream); break;
+    case 3: (low ? df_launch_aggregate<3, 2> : df_launch_aggregate<3, 4>)(a, nb, backward, stream); break;
+    default: (low ? df_launch_aggregate<4, 2> : df_launch_aggregate<4, 4>)(a, nb, backward, stream); break;
   }
   JN_LAUNCH_CHECK();
   return kOk;
 }
 
-template <int NK, int KS>
+template <int NK, int KB>
 static int df_launch_score_grad(const DenseScoreGradArgs& a, int nb, hipStream_t stream) {
   const dim3 grid(nb * (a.Npad / kDfGradRows)), block(kDfGradThreads);
-  if (a.mode != kDfAll) hipLaunchKernelGGL((dense_score_grad_kernel<NK, KS, true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((dense_score_grad_kernel<NK, KS, false>), grid, block, 0, stream, a);
+  if (a.mode != kDfAll) hipLaunchKernelGGL((dense_score_grad_kernel<NK, KB, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((dense_score_grad_kernel<NK, KB, false>), grid, block, 0, stream, a);
   JN_LAUNCH_CHECK();
   return kOk;
 }
 
 static int df_score_grad(const DenseScoreGradArgs& a, int nb, int D, const char* name, hipStream_t stream) {
   JN_PROFILE(name, stream);
-  const bool one = a.r <= 32;
+  const bool low = a.r <= 32;
   switch (D / 128) {
-    case 1: return one ? df_launch_score_grad<4, 1>(a, nb, stream) : df_launch_score_grad<4, 2>(a, nb, stream);
-    case 2: return one ? df_launch_score_grad<8, 1>(a, nb, stream) : df_launch_score_grad<8, 2>(a, nb, stream);
-    case 3: return one ? df_launch_score_grad<12, 1>(a, nb, stream) : df_launch_score_grad<12, 2>(a, nb, stream);
-    default: return one ? df_launch_score_grad<16, 1>(a, nb, stream) : df_launch_score_grad<16, 2>(a, nb, stream);
+    case 1: return low ? df_launch_score_grad<4, 2>(a, nb, stream) : df_launch_score_grad<4, 4>(a, nb, stream);
+    case 2: return low ? df_launch_score_grad<8, 2>(a, nb, stream) : df_launch_score_grad<8, 4>(a, nb, stream);
+    case 3: return low ? df_launch_score_grad<12, 2>(a, nb, stream) : df_launch_score_grad<12, 4>(a, nb, stream);
+    default: return low ? df_launch_score_grad<16, 2>(a, nb, stream) : df_launch_score_grad<16, 4>(a, nb, stream);
   }
 }
 
 int launch_dense_fused_forward(const DenseFused& f, hipStream_t stream) {
   const int Npad = (int)df_npad(f.N);
-  const DenseLayouts l = df_carve(f.scratch, f.nb, Npad);
+  const DenseLayouts l = df_carve(f.scratch, f.nb, Npad, f.D);
   int rc = df_prepare(f, l, Npad, f.projected_val, false, stream);
   if (rc) return rc;
   DenseAggregateArgs a{};
-  a.rows = l.planes[0];
-  a.cols = l.planes[1];
+  a.rows = l.ranks[0];
+  a.cols = l.ranks[1];
   a.values = l.packed;
   a.bias = f.bias;
   a.x = f.projected_state;
   a.out = static_cast<bf16_t*>(f.delta_val);
-  a.out_state = f.delta_state;
+  a.parts = l.parts;
   a.N = f.N;
   a.Npad = Npad;
   a.D = f.D;
   a.mode = f.causal ? kDfLower : kDfAll;
-  return df_aggregate(a, f.nb, f.r, "dense_aggregate_kernel<forward>", stream);
+  rc = df_aggregate(a, f.nb, f.r, false, "dense_aggregate_kernel<forward>", stream);
+  if (rc) return rc;
+  return launch_dense_part_rowsum(l.parts, dense_epi_parts(f.N), (int64_t)f.nb * f.N, f.delta_state, stream);
 }
 
 int launch_dense_fused_backward(const DenseFused& f, hipStream_t stream) {
   const int Npad = (int)df_npad(f.N);
-  const DenseLayouts l = df_carve(f.scratch, f.nb, Npad);
+  const DenseLayouts l = df_carve(f.scratch, f.nb, Npad, f.D);
   int rc = df_prepare(f, l, Npad, f.grad_delta_val, true, stream);
   if (rc) return rc;
   if (f.grad_projected_val || f.grad_projected_state) {
     DenseAggregateArgs a{};  // rows: sources; columns: targets
-    a.rows = l.planes[1];
-    a.cols = l.planes[0];
+    a.rows = l.ranks[1];
+    a.cols = l.ranks[0];
     a.values = l.packed;
     a.bias = f.bias;
     a.x = f.grad_delta_state;
@@ -641,13 +708,13 @@ int launch_dense_fused_backward(const DenseFused& f, hipStream_t stream) {
     a.Npad = Npad;
     a.D = f.D;
     a.mode = f.causal ? kDfUpper : kDfAll;
-    rc = df_aggregate(a, f.nb, f.r, "dense_aggregate_kernel<value_grad>", stream);
+    rc = df_aggregate(a, f.nb, f.r, true, "dense_aggregate_kernel<value_grad>", stream);
     if (rc) return rc;
   }
   DenseScoreGradArgs g{};
-  g.rows = l.planes[0];
-  g.cols = l.planes[1];
-  g.blocks = l.blocks[1];
+  g.rows = l.ranks[0];
+  g.cols = l.ranks[1];
+  g.proj = l.cols[1];
   g.row_val = static_cast<const bf16_t*>(f.grad_delta_val);
   g.col_val = static_cast<const bf16_t*>(f.projected_val);
   g.row_x = f.grad_delta_state;
@@ -656,23 +723,23 @@ int launch_dense_fused_backward(const DenseFused& f, hipStream_t stream) {
   g.out_scale = f.core_weight;
   g.out = f.dP;
   g.ld = 2 * f.r;
-  g.rowsum = f.rowsum;
+  g.parts = f.rowsum;
   g.N = f.N;
   g.Npad = Npad;
   g.r = f.r;
   g.mode = f.causal ? kDfLower : kDfAll;
   rc = df_score_grad(g, f.nb, f.D, "dense_score_grad_kernel<target>", stream);
   if (rc) return rc;
-  g.rows = l.planes[1];
-  g.cols = l.planes[0];
-  g.blocks = l.blocks[0];
+  g.rows = l.ranks[1];
+  g.cols = l.ranks[0];
+  g.proj = l.cols[0];
   g.row_val = static_cast<const bf16_t*>(f.projected_val);
   g.col_val = static_cast<const bf16_t*>(f.grad_delta_val);
   g.row_x = f.projected_state;
   g.col_x = f.grad_delta_state;
   g.out_scale = nullptr;
   g.out = f.dP + f.r;
-  g.rowsum = nullptr;
+  g.parts = nullptr;
   g.mode = f.causal ? kDfUpper : kDfAll;
   return df_score_grad(g, f.nb, f.D, "dense_score_grad_kernel<source>", stream);
 }

@@ -403,7 +403,7 @@ struct DenseFused {
   float* grad_projected_state;    // or null
   void* grad_projected_val;       // bf16, or null
   float* dP;                      // [nb][N] rows of 2 r: w_hat (G P_s), G^T P_t
-  float* rowsum;                  // [nb][N] sums of G
+  float* rowsum;                  // [nb][N][dense_epi_parts(N)] sums of G per 32 columns
 };
 // Batch elements per launch of these kernels with that much scratch; 0 where
 // they do not apply (the edge matrix is then built).

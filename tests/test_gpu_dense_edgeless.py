@@ -7,7 +7,7 @@ The reference is float64 on the operands the layer has: bf16 values, weights
 rounded to bf16, edges rounded to bf16 where they multiply values.  Tolerances,
 as relative 2-norms: bf16 outputs 2^-8 (one rounding of the result and one of
 the edges); fp32 state sums and score-scale gradients 2e-6 and 1e-5 (fp32
-projections of K = D terms, three-term products, sums over N); weight gradients
+projections of K = D terms, fp32 products, sums over N); weight gradients
 2^-8 (the projection gradient is rounded to bf16); the bias gradient, a sum of
 N^2 terms of either sign, 2^-20 of the sum of their magnitudes.
 """
@@ -118,3 +118,42 @@ def test_edgeless_rule():
     assert ok(4096, 512, 64, 0) == 1
     for args in ((4096, 520, 64, 0), (4096, 640, 64, 0), (4096, 512, 65, 0), (4096, 512, 64, 1), (256, 512, 64, 0)):
         assert ok(*args) == 0
+
+
+def _library_step(B, N, D, r, causal, edges):
+    """Every output of one layer through the C entry points: over a kept edge matrix, or on scratch of its size."""
+    import jakal_net_native as jn
+
+    t = {k: v.detach() for k, v in _case(B, N, D, r, causal, True, True, seed=B + N + r).items()}
+    L, p, st = jn._LIB, jn._ptr, jn._stream(DEV)
+    ds, dv, proj = torch.empty(B, N, device=DEV), torch.empty_like(t["X"]), torch.empty(B * N, 2 * r, device=DEV)
+    E = torch.empty(B * N * N * 4 + 256, device=DEV, dtype=torch.uint8)
+    args = [p(t[k]) for k in ("X", "ps", "pv", "U", "V", "w", "b")]
+    sizes = [B, N, D, D, r, 0, causal]
+    out = [p(ds), p(dv), p(proj), p(E)]
+    if edges:
+        jn._check(L.jn_propagation_dense_forward_bf16(*args, *sizes, *out, st))
+        ws_bytes = L.jn_propagation_dense_workspace_bytes(B, N, D, D, r, 0, 1)
+    else:
+        jn._check(L.jn_propagation_dense_forward_chunked_bf16(*args, *sizes, B, *out, E.numel(), st))
+        ws_bytes = L.jn_propagation_dense_chunked_workspace_bytes(B, N, D, D, r, 0, B, 1)
+    ws = torch.empty(ws_bytes, device=DEV, dtype=torch.uint8)
+    grads = [torch.empty_like(t[k]) for k in ("X", "ps", "pv", "U", "V", "w", "b")]
+    back = [p(proj), p(E), p(t["gs"]), p(t["gv"]), *sizes, 0]
+    tail = [*map(p, grads), p(ws), ws_bytes, st]
+    if edges:
+        jn._check(L.jn_propagation_dense_backward_bf16(*args[:6], *back, 1, *tail))
+    else:
+        jn._check(L.jn_propagation_dense_backward_chunked_bf16(*args, *back, B, 0, *tail))
+    torch.cuda.synchronize()
+    return dict(zip(("delta_state", "delta_val", "X", "ps", "pv", "U", "V", "w", "b"), (ds, dv, *grads)))
+
+
+@pytest.mark.parametrize("B,N,D,r,causal", [
+    (32, 776, 128, 20, 0), (24, 1032, 256, 64, 1), (28, 904, 384, 48, 1), (26, 1000, 512, 32, 0), (24, 1024, 512, 64, 0),
+])
+def test_same_bits_as_over_an_edge_matrix(B, N, D, r, causal):
+    """Rebuilding the edges keeps every product and every sum of the GEMMs over a stored edge matrix."""
+    got, want = (_library_step(B, N, D, r, causal, edges) for edges in (False, True))
+    for k in want:
+        assert torch.equal(got[k], want[k]), k
