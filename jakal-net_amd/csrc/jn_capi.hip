@@ -2201,7 +2201,7 @@ int jn_propagation_dense_backward_bf16(
 }
 
 int32_t jn_propagation_dense_edgeless_bf16(int64_t nodes, int64_t out_dim, int64_t rank, int32_t compress_kind) {
-  return dense_fused_batch(1, nodes, out_dim, rank, compress_kind, (size_t)nodes * nodes * sizeof(float)) > 0 ? 1 : 0;
+  return dense_fused_serves(nodes, out_dim, rank, compress_kind) ? 1 : 0;
 }
 
 size_t jn_propagation_dense_chunked_workspace_bytes(int64_t batch, int64_t nodes, int64_t in_dim, int64_t out_dim,

@@ -563,14 +563,19 @@ static size_t df_element_bytes(int64_t N, int64_t D) {
          std::max(rows * ranks, rows * dense_epi_parts((int)N) * sizeof(float));
 }
 
-// Whole 128-column pieces of value rows (at most 512: a wave's accumulators),
-// up to 64 ranks, 32-bit offsets, at least 512 nodes (the smallest measured) and
-// scratch for a batch element at least.
+// The layers these kernels serve: whole 128-column pieces of value rows (at most
+// 512: a wave's accumulators), up to 64 ranks, 32-bit offsets, at least 512 nodes
+// (the smallest measured), and layouts no larger than the edge matrix, whose
+// buffer holds them.
+bool dense_fused_serves(int64_t N, int64_t D, int64_t r, int compress_kind) {
+  return compress_kind == 0 && r <= kDfRank && D % 128 == 0 && D <= 512 && N >= 512 && N * D * 2 < (1LL << 31) &&
+         (size_t)N * N * sizeof(float) >= df_element_bytes(N, D);
+}
+
 int64_t dense_fused_batch(int64_t batch, int64_t N, int64_t D, int64_t r, int compress_kind, size_t scratch_bytes) {
-  if (compress_kind != 0 || r > kDfRank || D % 128 != 0 || D > 512 || N < 512 || N * D * 2 >= (1LL << 31)) return 0;
+  if (!dense_fused_serves(N, D, r, compress_kind)) return 0;
   const int64_t fit = (int64_t)(scratch_bytes / df_element_bytes(N, D));
-  const int64_t nb = std::min(batch, fit);
-  return std::min<int64_t>(nb, 65535);
+  return std::min<int64_t>(std::min(batch, fit), 65535);
 }
 
 struct DenseLayouts {

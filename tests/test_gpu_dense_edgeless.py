@@ -157,3 +157,22 @@ def test_same_bits_as_over_an_edge_matrix(B, N, D, r, causal):
     got, want = (_library_step(B, N, D, r, causal, edges) for edges in (False, True))
     for k in want:
         assert torch.equal(got[k], want[k]), k
+
+
+@pytest.mark.parametrize("B,N,D,r", [(4, 520, 512, 33), (8, 256, 256, 17)])
+def test_second_backward_where_one_matrix_is_too_small(B, N, D, r):
+    """Layers whose operand layouts exceed one edge matrix but not the batch's: their edges are kept, and a second
+    backward rebuilds them as the forward did."""
+    import jakal_net_native as jn
+
+    assert jn._LIB.jn_propagation_dense_edgeless_bf16(N, D, r, 0) == 0
+    t = _case(B, N, D, r, False, True, True, seed=N)
+    ds, dv = _run(t, False)
+    grads = []
+    for keep in (True, False):
+        torch.autograd.backward([ds, dv], [t["gs"], t["gv"]], retain_graph=keep)
+        grads.append({k: v.grad for k, v in t.items() if v.requires_grad})
+        for v in t.values():
+            v.grad = None
+    for k in grads[0]:
+        assert torch.equal(grads[0][k], grads[1][k]), k
