@@ -39,7 +39,7 @@ typedef void* jn_stream_t;
 /* Message of the last failing call on this host thread ("" if none). */
 const char* jn_last_error(void);
 
-/* ABI revision of this header (bumped on any signature or accepted-range change); this is 16. */
+/* ABI revision of this header (bumped on any signature or accepted-range change); this is 17. */
 int jn_abi_version(void);
 
 /*
@@ -684,12 +684,25 @@ int jn_propagation_dense_backward_bf16(
     int32_t projected_val_is_layer_val, int32_t reuse_edges, uint16_t* grad_layer_val, float* grad_projected_state,
     uint16_t* grad_projected_val, float* grad_target_weight, float* grad_source_weight, float* grad_core_weight,
     float* grad_bias, void* workspace, size_t workspace_bytes, jn_stream_t stream);
-/* 1 when the chunked bf16 entry points run a layer of these sizes without an
- * edge matrix (softsign, out_dim a multiple of 128 up to 512, rank <= 64): the
- * forward's workspace and the backward's edge_chunk (chunk_batch * nodes * nodes
- * floats, both) are then scratch, hold no edges afterwards, and chunk_resident
- * is ignored.  No counterpart in the reference. */
+/* 1 when the chunked bf16 entry points can run a layer of these sizes without
+ * an edge matrix: softsign, out_dim a multiple of 128 up to 512, rank <= 64, at
+ * least 512 nodes and operand layouts no larger than the edge matrix (512 nodes
+ * or a few more).  They do so where a batch fills the chip: below.  No
+ * counterpart in the reference. */
 int32_t jn_propagation_dense_edgeless_bf16(int64_t nodes, int64_t out_dim, int64_t rank, int32_t compress_kind);
+/* The smallest chunk_batch, at most the given one, with which the chunked bf16
+ * entry points run this batch without an edge matrix in no more launches than
+ * with the given one (which works as well); 0 when they build one (the
+ * layer is not of the sizes above, or its launches have too few blocks of 128
+ * rows to be the faster path: fewer than 256; 192 for out_dim >= 256 or 2560
+ * nodes; 128 for 3000 nodes, not causal).
+ * Where it is not 0 the forward's workspace and the backward's edge_chunk
+ * (chunk_batch * nodes * nodes floats, both) are scratch, hold no edges
+ * afterwards, and chunk_resident is ignored.  Results are the same bits either
+ * way for ranks that are multiples of 4, apart from the summation order of the
+ * state sums and gradients.  No counterpart in the reference. */
+int64_t jn_propagation_dense_edgeless_chunk_bf16(int64_t batch, int64_t nodes, int64_t out_dim, int64_t rank,
+                                                 int32_t compress_kind, int32_t causal, int64_t chunk_batch);
 int jn_propagation_dense_forward_chunked_bf16(const uint16_t* layer_val, const float* projected_state,
                                               const uint16_t* projected_val, const float* target_weight,
                                               const float* source_weight, const float* core_weight, const float* bias,

@@ -538,8 +538,9 @@ int dense_backward(const float* layer_val, const float* projected_state, const f
   float* gpv = projected_val_is_layer_val ? grad_layer_val : grad_projected_val;
   int rc;
   // a bf16 softsign layer whose forward kept no edges: nothing is rebuilt
-  const int64_t edgeless =
-      bf16 && recompute ? dense_fused_batch(B, N, D, r, compress_kind, (size_t)chunk_batch * N * N * sizeof(float)) : 0;
+  const int64_t edgeless = bf16 && recompute ? dense_fused_batch(B, N, D, r, compress_kind, causal != 0,
+                                                                 (size_t)chunk_batch * N * N * sizeof(float))
+                                             : 0;
   for (int b0 = 0; edgeless > 0 && b0 < B; b0 += (int)edgeless) {
     const int nb = (int)std::min<int64_t>(edgeless, B - b0);
     const int64_t pr = (int64_t)b0 * N;
@@ -1261,7 +1262,7 @@ extern "C" {
 
 const char* jn_last_error(void) { return jakal::last_error(); }
 
-int jn_abi_version(void) { return 16; }
+int jn_abi_version(void) { return 17; }
 
 int jn_unit_scale_forward(const float* weight, int64_t rows, int64_t rank, float eps, float* weight_hat,
                           jn_stream_t stream) {
@@ -2204,6 +2205,15 @@ int32_t jn_propagation_dense_edgeless_bf16(int64_t nodes, int64_t out_dim, int64
   return dense_fused_serves(nodes, out_dim, rank, compress_kind) ? 1 : 0;
 }
 
+int64_t jn_propagation_dense_edgeless_chunk_bf16(int64_t batch, int64_t nodes, int64_t out_dim, int64_t rank,
+                                                 int32_t compress_kind, int32_t causal, int64_t chunk_batch) {
+  if (chunk_batch < 1) return 0;
+  const size_t one = (size_t)nodes * nodes * sizeof(float);
+  const int64_t nb = dense_fused_batch(batch, nodes, out_dim, rank, compress_kind, causal != 0,
+                                       std::min(batch, chunk_batch) * one);
+  return nb > 0 ? (int64_t)((nb * dense_fused_element_bytes(nodes, out_dim) + one - 1) / one) : 0;
+}
+
 size_t jn_propagation_dense_chunked_workspace_bytes(int64_t batch, int64_t nodes, int64_t in_dim, int64_t out_dim,
                                                     int64_t rank, int32_t compress_kind, int64_t chunk_batch,
                                                     int32_t backward) {
@@ -2237,7 +2247,7 @@ static int propagation_dense_forward_chunked_impl(
                     (int)in_dim, st, bf16);
   if (rc) return rc;
   if (bf16) {
-    const int64_t nb = dense_fused_batch(B, N, D, r, compress_kind, (size_t)cb * N * N * sizeof(float));
+    const int64_t nb = dense_fused_batch(B, N, D, r, compress_kind, causal != 0, (size_t)cb * N * N * sizeof(float));
     for (int b0 = 0; nb > 0 && b0 < B; b0 += (int)nb) {
       DenseFused f = dense_fused_range(projected_state, projected_val, core_weight, bias, projections, b0,
                                        (int)std::min<int64_t>(nb, B - b0), N, D, r, causal != 0, E);

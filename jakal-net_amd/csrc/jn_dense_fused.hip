@@ -557,7 +557,7 @@ static int64_t df_npad(int64_t N) { return (N + kDfRows - 1) / kDfRows * kDfRows
 // bytes of one batch element's layouts (a multiple of 256): the ranks of both
 // projections, the packed values, and the transposed projections (backward) or
 // the partial state sums (forward)
-static size_t df_element_bytes(int64_t N, int64_t D) {
+size_t dense_fused_element_bytes(int64_t N, int64_t D) {
   const size_t rows = (size_t)df_npad(N), ranks = 2 * kDfRank * sizeof(float);
   return rows * (ranks + (size_t)D * sizeof(bf16_t)) +
          std::max(rows * ranks, rows * dense_epi_parts((int)N) * sizeof(float));
@@ -569,13 +569,42 @@ static size_t df_element_bytes(int64_t N, int64_t D) {
 // buffer holds them.
 bool dense_fused_serves(int64_t N, int64_t D, int64_t r, int compress_kind) {
   return compress_kind == 0 && r <= kDfRank && D % 128 == 0 && D <= 512 && N >= 512 && N * D * 2 < (1LL << 31) &&
-         (size_t)N * N * sizeof(float) >= df_element_bytes(N, D);
+         (size_t)N * N * sizeof(float) >= dense_fused_element_bytes(N, D);
 }
 
-int64_t dense_fused_batch(int64_t batch, int64_t N, int64_t D, int64_t r, int compress_kind, size_t scratch_bytes) {
-  if (!dense_fused_serves(N, D, r, compress_kind)) return 0;
-  const int64_t fit = (int64_t)(scratch_bytes / df_element_bytes(N, D));
-  return std::min<int64_t>(std::min(batch, fit), 65535);
+// Whether a launch of that many aggregate workgroups (128 rows) is the faster
+// path.  A workgroup walks all columns by itself, so a small grid takes as long
+// as a full one, where the GEMMs over an edge matrix spread over the chip; they
+// gain a little more from causal ranges.  Forward / step in us, without and with
+// an edge matrix (rank 64; every width and rank measured on the line at 512 to
+// 4096 nodes is the faster or within 2 % of it, but for the forward of 4 x 4096
+// nodes with 256 values and rank 40, 302 against 278, whose step is 1102 against
+// 1321):
+//                          512 values                  128 values
+//    4 x 1024   (32)  112 /  384,  68 /  282     89 /  312,  57 /  263
+//   16 x 1024  (128)  125 /  422, 121 /  443     98 /  330,  81 /  336
+//   24 x 1024  (192)  124 /  533, 161 /  593     98 /  412, 102 /  423
+//     causal          126 /  558, 150 /  572    101 /  415,  95 /  411
+//   64 x 512   (256)  102 /  393, 125 /  438     74 /  285,  82 /  312
+//    1 x 4096   (32)  318 / 1196, 131 /  762    265 /  991, 130 /  726
+//    4 x 4096  (128)  331 / 1234, 357 / 1488    268 / 1014, 316 / 1232
+//     causal          339 / 1443, 300 / 1350    284 / 1046, 291 / 1157
+//    6 x 4096  (192)  346 / 1603, 524 / 2121    284 / 1301, 459 / 1751
+//     causal          346 / 1602, 406 / 1887    286 / 1188, 390 / 1607
+static bool df_fills(int64_t blocks, int64_t N, int64_t D, bool causal) {
+  if (blocks >= 256) return true;
+  if (blocks >= 192) return D >= 256 || N >= 2560;
+  return blocks >= 128 && N >= 3000 && !causal;
+}
+
+int64_t dense_fused_batch(int64_t batch, int64_t N, int64_t D, int64_t r, int compress_kind, bool causal,
+                          size_t scratch_bytes) {
+  if (batch < 1 || !dense_fused_serves(N, D, r, compress_kind)) return 0;
+  const int64_t fit = std::min<int64_t>((int64_t)(scratch_bytes / dense_fused_element_bytes(N, D)), 65535);
+  if (fit < 1) return 0;
+  const int64_t launches = (batch + fit - 1) / fit;
+  const int64_t nb = (batch + launches - 1) / launches;  // an even share each
+  return df_fills(nb * (df_npad(N) / kDfRows), N, D, causal) ? nb : 0;
 }
 
 struct DenseLayouts {

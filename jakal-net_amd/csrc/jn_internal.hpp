@@ -405,10 +405,13 @@ struct DenseFused {
   float* dP;                      // [nb][N] rows of 2 r: w_hat (G P_s), G^T P_t
   float* rowsum;                  // [nb][N][dense_epi_parts(N)] sums of G per 32 columns
 };
+size_t dense_fused_element_bytes(int64_t N, int64_t D);  // scratch of one batch element
 bool dense_fused_serves(int64_t N, int64_t D, int64_t r, int compress_kind);
 // Batch elements per launch of these kernels with that much scratch; 0 where
-// they do not serve the layer (the edge matrix is then built).
-int64_t dense_fused_batch(int64_t batch, int64_t N, int64_t D, int64_t r, int compress_kind, size_t scratch_bytes);
+// they do not serve the layer or are the slower path (the edge matrix is then
+// built).
+int64_t dense_fused_batch(int64_t batch, int64_t N, int64_t D, int64_t r, int compress_kind, bool causal,
+                          size_t scratch_bytes);
 int launch_dense_fused_forward(const DenseFused& f, hipStream_t stream);
 int launch_dense_fused_backward(const DenseFused& f, hipStream_t stream);
 

@@ -131,6 +131,7 @@ _declare(
 )
 
 _declare("jn_propagation_dense_edgeless_bf16", [_I64, _I64, _I64, _I32], _I32)
+_declare("jn_propagation_dense_edgeless_chunk_bf16", [_I64, _I64, _I64, _I64, _I32, _I32, _I64], _I64)
 _declare("jn_propagation_dense_multihead_chunk_bytes", [_I64] * 3, _SZ)
 _declare("jn_propagation_dense_multihead_workspace_bytes", [_I64] * 6 + [_I32, _I64], _SZ)
 _declare(
@@ -728,8 +729,9 @@ class _PropagationDense(torch.autograd.Function):
         dev = X.device
         edge_bytes = N * N * 4
         chunk = B if B * edge_bytes <= DENSE_EDGE_BYTES else max(1, DENSE_EDGE_BYTES // edge_bytes)
-        # a bf16 softsign layer builds no edges: the chunk buffer is scratch
-        edgeless = bf16 and _LIB.jn_propagation_dense_edgeless_bf16(N, Dout, r, compress) == 1
+        # bf16 softsign layers that fill the chip build no edges: the chunk buffer is scratch
+        edgeless = bf16 and _LIB.jn_propagation_dense_edgeless_chunk_bf16(B, N, Dout, r, compress, 1 if causal else 0,
+                                                                          chunk) > 0
         with _on(dev):
             ds = torch.empty(B, N, device=dev, dtype=torch.float32)
             dv = torch.empty(B, N, Dout, device=dev, dtype=torch.bfloat16 if bf16 else torch.float32)

@@ -150,7 +150,7 @@ def _library_step(B, N, D, r, causal, edges):
 
 
 @pytest.mark.parametrize("B,N,D,r,causal", [
-    (32, 776, 128, 20, 0), (24, 1032, 256, 64, 1), (28, 904, 384, 48, 1), (26, 1000, 512, 32, 0), (24, 1024, 512, 64, 0),
+    (37, 776, 128, 20, 0), (24, 1032, 256, 64, 1), (28, 904, 384, 48, 1), (26, 1000, 512, 32, 0), (24, 1024, 512, 64, 0),
 ])
 def test_same_bits_as_over_an_edge_matrix(B, N, D, r, causal):
     """Rebuilding the edges keeps every product and every sum of the GEMMs over a stored edge matrix."""
@@ -176,3 +176,45 @@ def test_second_backward_where_one_matrix_is_too_small(B, N, D, r):
             v.grad = None
     for k in grads[0]:
         assert torch.equal(grads[0][k], grads[1][k]), k
+
+
+@pytest.mark.parametrize("B,N,D,r,causal,separate,bias,per_launch", [
+    (43, 712, 128, 1, False, False, True, None),
+    (28, 776, 256, 32, False, True, False, None),
+    (24, 1000, 384, 33, True, False, True, None),
+    (24, 904, 512, 64, True, True, True, None),
+    (22, 1032, 512, 20, False, False, True, None),
+    (28, 776, 384, 64, False, True, False, None),
+    (32, 1024, 128, 63, True, True, False, None),
+    (63, 1024, 128, 40, False, True, True, 10),  # launches of 32 and 31
+    (49, 1016, 512, 64, True, False, True, 16),  # 25 and 24
+])
+def test_edgeless_dense_on_full_grids(B, N, D, r, causal, separate, bias, per_launch):
+    """The same at the batches from which the layer runs without an edge matrix."""
+    import jakal_net_native as jn
+
+    assert jn._LIB.jn_propagation_dense_edgeless_chunk_bf16(B, N, D, r, 0, int(causal), per_launch or B) > 0
+    test_edgeless_dense(B, N, D, r, causal, separate, bias, per_launch)
+
+
+@pytest.mark.parametrize("B,N,D,r,causal,edgeless", [
+    (31, 704, 512, 64, False, False), (32, 704, 512, 64, True, True), (63, 512, 128, 8, False, False),
+    (64, 512, 128, 8, True, True), (5, 3000, 512, 64, False, False), (6, 3000, 512, 64, False, True),
+    (1, 4096, 512, 64, False, False), (4, 4096, 512, 64, False, True), (5, 4096, 512, 64, True, False),
+    (6, 4096, 128, 64, True, True),
+])
+def test_kernels_of_a_batch(B, N, D, r, causal, edgeless):
+    """Which kernels a layer runs on either side of the line (small grids leave most of the chip idle without edges)."""
+    import jakal_net_native as jn
+
+    t = _case(B, N, D, r, causal, False, True, seed=5)
+    jn.profile_enable(True)
+    try:
+        ds, dv = _run(t, causal)
+        torch.autograd.backward([ds, dv], [t["gs"], t["gv"]])
+        torch.cuda.synchronize()
+        names = "".join(jn.profile_collect())
+    finally:
+        jn.profile_enable(False)
+    assert ("dense_score_grad_kernel" in names) == ("dense_aggregate_kernel<forward>" in names) == edgeless
+    assert ("gemm_bf16_kernel<dense_edge_grad_bf16>" in names) != edgeless
