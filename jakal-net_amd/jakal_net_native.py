@@ -712,7 +712,8 @@ class _PropagationDense(torch.autograd.Function):
     problems keep the edge matrix for the backward; larger ones run in batch
     chunks of at most DENSE_EDGE_BYTES of edges and rebuild them.  With bf16,
     X and pv are bf16 and delta_val comes back in bf16 (the *_bf16 entry
-    points); the edge matrix stays fp32."""
+    points); the edge matrix stays fp32, and softsign layers that fill the chip
+    build none (their edges are rebuilt tile by tile, in scratch of each call)."""
 
     @staticmethod
     def _entry(name: str, bf16: bool):
@@ -729,9 +730,13 @@ class _PropagationDense(torch.autograd.Function):
         dev = X.device
         edge_bytes = N * N * 4
         chunk = B if B * edge_bytes <= DENSE_EDGE_BYTES else max(1, DENSE_EDGE_BYTES // edge_bytes)
-        # bf16 softsign layers that fill the chip build no edges: the chunk buffer is scratch
-        edgeless = bf16 and _LIB.jn_propagation_dense_edgeless_chunk_bf16(B, N, Dout, r, compress, 1 if causal else 0,
-                                                                          chunk) > 0
+        # bf16 softsign layers that fill the chip build no edges: their chunk
+        # buffer is scratch of the call, in the forward as in the backward
+        scratch = bf16 and _LIB.jn_propagation_dense_edgeless_chunk_bf16(B, N, Dout, r, compress, 1 if causal else 0,
+                                                                         chunk)
+        edgeless = scratch > 0
+        if edgeless:
+            chunk = scratch
         with _on(dev):
             ds = torch.empty(B, N, device=dev, dtype=torch.float32)
             dv = torch.empty(B, N, Dout, device=dev, dtype=torch.bfloat16 if bf16 else torch.float32)
@@ -757,7 +762,7 @@ class _PropagationDense(torch.autograd.Function):
                         _ptr(edges), ws_bytes, _stream(dev),
                     )
                 )
-        ctx.save_for_backward(X, ps, pv_t, V, U, w_hat, proj, edges, bias)
+        ctx.save_for_backward(X, ps, pv_t, V, U, w_hat, proj, None if edgeless else edges, bias)
         ctx.meta = (compress, pv_is_x, bias is not None, bool(causal), chunk, bool(bf16))
         ctx.edges_consumed = edgeless
         ctx.set_materialize_grads(False)  # an unused delta_state arrives as None
@@ -818,6 +823,8 @@ class _PropagationDense(torch.autograd.Function):
         need = ctx.needs_input_grad
         ds_used = g_ds is not None  # projected_state reaches delta_state only
         with _on(dev):
+            if edge_chunk is None:  # no edges: the layouts' scratch
+                edge_chunk = torch.empty(chunk * N * N, device=dev, dtype=torch.float32)
             vdt = torch.bfloat16 if bf16 else torch.float32
             g_ds = torch.zeros(B, N, device=dev) if g_ds is None else g_ds.float().contiguous()
             g_dv = torch.zeros(B, N, Dout, device=dev, dtype=vdt) if g_dv is None else g_dv.to(vdt).contiguous()

@@ -218,3 +218,16 @@ def test_kernels_of_a_batch(B, N, D, r, causal, edgeless):
         jn.profile_enable(False)
     assert ("dense_score_grad_kernel" in names) == ("dense_aggregate_kernel<forward>" in names) == edgeless
     assert ("gemm_bf16_kernel<dense_edge_grad_bf16>" in names) != edgeless
+
+
+def test_edgeless_forward_keeps_no_scratch():
+    """Between forward and backward the layer holds its outputs and projections, not an edge matrix's worth of scratch."""
+    B, N, D, r = 24, 1024, 512, 64
+    t = _case(B, N, D, r, False, True, True, seed=9)
+    _run(t, False)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated(DEV)
+    ds, dv = _run(t, False)
+    held = torch.cuda.memory_allocated(DEV) - before
+    assert held <= B * N * (4 + 2 * D + 8 * r) + (1 << 20)
+    torch.autograd.backward([ds, dv], [t["gs"], t["gv"]])
