@@ -56,12 +56,16 @@ int jn_profile_collect(char* buffer, size_t size);
  * GEMM tiling control (no counterpart in the reference; for tests and tuning).
  * tile = 64 or 128 forces that square workgroup tile on every later dense
  * product (projections, their gradients, the dense-mode score, aggregation and
- * gradient products); 32 forces the 32 x 32 tile on the projection products
- * and their gradients (64 elsewhere); 0 (the default) picks per call: 128 when
- * both output extents are >= 128 and the grid still has >= 256 workgroups,
- * else 64, or 32 for the projection products when a 64 x 64 grid has fewer
- * than 256 workgroups.  Process-wide; results are the same up to fp32
- * summation order.
+ * gradient products), on bf16 MFMAs for the bf16 dense products and, at 128,
+ * for the projections of bf16 layers and their gradients, else on fp32 MFMAs;
+ * 32 forces the 32 x 32 tile on the projection products and their gradients (64
+ * elsewhere); 0 (the default) picks per call: 128 when both output extents are
+ * >= 128 and the grid still has >= 256 workgroups, else 64, or 32 for the
+ * projection products on fp32 MFMAs when a 64 x 64 grid has fewer than 256
+ * workgroups.  Only 0 runs the fp32 projections, their gradients and the fp32
+ * dense aggregation and value gradient as three-term bf16 products, and
+ * projections of few rows on a kernel of their own.  Process-wide; results are
+ * the same up to fp32 summation order.
  */
 int jn_set_gemm_tile(int32_t tile);
 

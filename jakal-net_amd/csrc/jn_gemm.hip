@@ -1656,9 +1656,10 @@ int launch_gemm(const GemmArgs& g, GemmUse use, int splits, hipStream_t stream) 
     RowsGemm r;
     if (rows_form(g, use, fast, r)) return launch_gemm_rows(&r, 1, stream);
   }
-  // the 128-wide MFMA tiles of this product, or 64-wide where those leave CUs idle
+  // the 128-wide MFMA tiles of this product, or 64-wide where those leave CUs
+  // idle (or as forced: 32 x 32 tiles are not among them)
   const int64_t tiles128 = (int64_t)((g.M + kBfT - 1) / kBfT) * ((g.N + kBfT - 1) / kBfT) * zdim;
-  const int tile = tiles128 < kTile64Below ? 64 : kBfT;
+  const int tile = forced ? (forced == kBfT ? kBfT : 64) : tiles128 < kTile64Below ? 64 : kBfT;
   const int tm = (g.M + tile - 1) / tile, tn = (g.N + tile - 1) / tile;
   const int64_t tiles = (int64_t)tm * tn * zdim;
   auto at_tile = [&](auto launch) {

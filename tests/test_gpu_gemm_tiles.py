@@ -142,3 +142,75 @@ def test_bf16_product_is_the_same_on_both_tiles(dev):
                                             None, "softmax", 1.0, rho, src[:n], dst[:n], ps[:n], pv[:n], Ns, Nd)[1]
 
     assert torch.equal(run(64)[:63], run(63))
+
+
+@pytest.mark.parametrize("compress,causal,separate_pv", [
+    ("softsign", True, True), ("softsign", False, True), ("signed_abs_softmax", True, False),
+    ("signed_entmax15", False, True),
+])
+def test_bf16_dense_products(dev, tile, compress, causal, separate_pv):
+    # the bf16 dense products on 64- and 128-wide MFMA tiles: softsign epilogue, causal K ranges, ragged extents
+    TB.test_bf16_dense_variants(dev, None, compress, causal, separate_pv, None)
+
+
+@pytest.mark.parametrize("compress", ["softmax", "signed_abs_softmax"])
+def test_bf16_route_products(dev, tile, compress):
+    TB.test_bf16_dense_transition(dev, compress)
+
+
+def _bf16_dense_step(dev, routes):
+    """Outputs and gradients of a causal bf16 dense layer, and of a bf16 dense transition."""
+    import jakal_net_native as jn
+
+    B, N, Nd, D, r = 2, 264, 136, 200, 18
+    g = torch.Generator().manual_seed(4700)
+    leaf = lambda *s, dt=torch.float32: torch.randn(*s, generator=g).to(dev, dt).requires_grad_(True)  # noqa: E731
+    X, dst = leaf(B, N, D, dt=torch.bfloat16), leaf(B, Nd, D, dt=torch.bfloat16)
+    ps, w, U, V = leaf(B, N), leaf(r), leaf(r, D), leaf(r, D)
+    out = jn.propagation_dense("low_rank_bilinear", w, None, V, None, U, None, "softsign", X, ps, X, None, N, N,
+                               _causal=True)
+    if routes:
+        out += jn.transition_pairwise_dense("low_rank_bilinear_route", U, None, V, None, w, None, None, None, None,
+                                            None, "softmax", 1.0, torch.nn.functional.softplus(ps), X, dst, ps, X, N,
+                                            Nd)
+    gs = [torch.randn(o.shape, generator=g).to(dev, o.dtype) for o in out]
+    return [*out, *torch.autograd.grad(out, [X, ps, w, U, V], gs)]
+
+
+@pytest.mark.parametrize("forced", [64, 128])
+def test_forced_tile_reaches_the_mfma_products(dev, forced):
+    """The bf16 MFMA kernels of the dense products run on the forced tile (their last template argument), whatever
+    the grid."""
+    import jakal_net_native as jn
+    from torch.profiler import ProfilerActivity, profile
+
+    try:
+        jn.set_gemm_tile(forced)
+        _bf16_dense_step(dev, True)
+        with profile(activities=[ProfilerActivity.CUDA]) as prof:
+            _bf16_dense_step(dev, True)
+            torch.cuda.synchronize()
+    finally:
+        jn.set_gemm_tile(0)
+    names = [e.key for e in prof.key_averages() if "gemm_bf16_kernel<" in e.key]
+    assert len(names) >= 6 and all(f", {forced}>" in n for n in names), names
+
+
+def test_bf16_dense_step_is_the_same_on_both_tiles(dev):
+    """Every element of the MFMA products keeps its chain over K on either tile, so everything but the weight
+    gradients, fp32 products that a forced tile moves as well, is the same bit for bit.  (Rank 18 keeps the other fp32
+    products on their 64 x 64 tiles.)"""
+    import jakal_net_native as jn
+
+    results = []
+    try:
+        for forced in (64, 128):
+            jn.set_gemm_tile(forced)
+            results.append(_bf16_dense_step(dev, False))
+    finally:
+        jn.set_gemm_tile(0)
+    for i, (a, b) in enumerate(zip(*results)):
+        if i < len(results[0]) - 2:
+            assert torch.equal(a, b), i
+        else:
+            assert (a - b).norm() <= 1e-5 * b.norm()
