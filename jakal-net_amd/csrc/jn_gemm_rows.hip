@@ -1,8 +1,8 @@
 // Projections of few rows (transitions, slot and query layers, one graph at a
 // time): C[M][N] = X[M][K] . [W0; W1]^T with N = the ranks (up to a few
-// hundred) and M up to some ten thousand, where tiles of 128 x 128 or 64 x 64
-// leave most of the 256 CUs idle and walk K behind two barriers per slice with
-// one slice's latency exposed each time.
+// hundred) and few enough rows (gemm_rows_fits) that tiles of 128 x 128 or 64 x
+// 64 leave many of the 256 CUs idle and walk K behind two barriers per slice
+// with one slice's latency exposed each time.
 //
 // Every wave is a worker of its own: it owns an output tile of MT x NT MFMA
 // tiles and walks all of K in 32-wide slices -- whole lines into registers,
@@ -22,11 +22,16 @@
 //
 // Bound: below some 4096 rows the chain of 16 slices (K = 512), each a load's
 // latency and a dependent run of MFMAs; above, the splits' VALU work and the
-// MFMAs.  Measured with the events' own 5 us, K = 512, N = 128, against the
-// kernels it replaces: fp32 36 -> 14 us at 1024 rows, 37 -> 18 at 4096,
-// 37 -> 24 at 8192, 39 -> 30 at 16,384 (44 -> 53 at 32,768: not taken); bf16
-// 18 -> 10, 20 -> 12, 20 -> 15, 21 -> 18 us; K = 384, N = 64 on fp32 MFMA
-// 11 -> 9 us at 1024 rows, 16 -> 14 at 8192, 32 -> 27 at 32,768.
+// MFMAs.  Measured with the events' own 5 us, K = 512, against the tile kernel
+// of the same arithmetic (its 64 x 64 tiles where the grid is small):
+//                      three-term           bf16              fp32 MFMA (N = 64)
+//   1024 x 128      19.8 -> 13.4 us    11.2 ->  9.1 us    12.8 -> 10.3 us
+//   4096 x 128      20.3 -> 17.8       11.3 -> 11.7       13.2 -> 10.5
+//   8192 x 128      21.0 -> 22.8       12.1 -> 14.2       17.0 -> 14.4
+//   1024 x 512      20.5 -> 18.1       12.0 -> 11.7       (32,768: 37.6 -> 33.1)
+//   1300 x 512      20.8 -> 22.2       11.7 -> 13.0
+//   4096 x 512      25.7 -> 30.0       14.2 -> 18.3
+//   16,384 x 512    56.5 -> 99         27   -> 43
 #include "jn_internal.hpp"
 
 namespace jakal {
@@ -227,15 +232,28 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(RowsGemmArgs args) {
       }
 }
 
+static int64_t rows_tiles(const RowsGemm& g) { return (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16); }
+
+// Whether this kernel is the faster one.  A wave loads (and splits) its rows of X
+// again for every column tile, so against the MFMA tile kernels the outputs
+// count: up to 2048 tiles of 16 x 16 on three-term products, fewer on bf16 ones
+// (level there, 11.7 against 11.3 us, and slower beyond).  Against
+// gemm_f32_kernel, at any number of columns, the rows: 32,768, or 16,384 from
+// 128 columns on (the largest measured).
+static bool rows_few(const RowsGemm& g) {
+  if (g.arith == kRowsX3) return rows_tiles(g) <= 2048;
+  if (g.arith == kRowsBf) return rows_tiles(g) < 2048;
+  return g.M <= (g.N >= 128 ? kRowsMaxM / 2 : kRowsMaxM);
+}
+
 // Whole 16-byte loads (K and the row strides in whole vectors, 16-byte aligned
-// operands), and the rows up to which this kernel is the faster one: 16,384
-// against the 128 x 128 kernels (N >= 128), 32,768 against gemm_f32_kernel.
+// operands), few rows.
 bool gemm_rows_fits(const RowsGemm& g) {
   const bool bf = g.arith == kRowsBf || g.arith == kRowsC4Bf;
   const int kv = bf ? 8 : 4;
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  return g.M >= 1 && g.N >= 1 && g.K >= 1 && g.M <= (g.N >= 128 ? kRowsMaxM / 2 : kRowsMaxM) && g.N <= kRowsMaxN && g.K % kv == 0 &&
-         g.ldx % kv == 0 && g.ldw % 4 == 0 && al16(g.X) && al16(g.W0) && al16(g.W1);
+  return g.M >= 1 && g.N >= 1 && g.K >= 1 && g.N <= kRowsMaxN && rows_few(g) && g.K % kv == 0 && g.ldx % kv == 0 &&
+         g.ldw % 4 == 0 && al16(g.X) && al16(g.W0) && al16(g.W1);
 }
 
 template <int ARITH, int MT, int NT, int DEPTH>
@@ -255,11 +273,14 @@ static void launch_rows(const RowsGemm* p, int n, hipStream_t stream) {
 template <int ARITH>
 static void launch_rows_tile(const RowsGemm* p, int n, hipStream_t stream) {
   int64_t tiles = 0;
-  for (int i = 0; i < n; ++i) tiles += (int64_t)((p[i].M + 15) / 16) * ((p[i].N + 15) / 16);
+  for (int i = 0; i < n; ++i) tiles += rows_tiles(p[i]);
   // the largest tile that still gives every SIMD (1024) two waves (K = 512,
-  // N = 128: 30 us at 16,384 rows on 32 x 32 tiles against 38 on 16 x 32)
-  if (tiles >= 8192) launch_rows<ARITH, 2, 2, 2>(p, n, stream);
-  else if (tiles >= 2048) launch_rows<ARITH, 1, 2, 3>(p, n, stream);
+  // N = 128: 30 us at 16,384 rows on 32 x 32 tiles against 38 on 16 x 32); the
+  // MFMA tile kernels take over before 32 x 32 ones would
+  if constexpr (ARITH == kRowsC4 || ARITH == kRowsC4Bf) {
+    if (tiles >= 8192) return launch_rows<ARITH, 2, 2, 2>(p, n, stream);
+  }
+  if (tiles >= 2048) launch_rows<ARITH, 1, 2, 3>(p, n, stream);
   else launch_rows<ARITH, 1, 1, 4>(p, n, stream);
 }
 

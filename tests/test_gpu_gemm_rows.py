@@ -72,3 +72,21 @@ def test_two_projections_in_one_launch(Ns, Nd, r, bf16):
         want = op.compute_delta(f(src), f(dst))
     tol = 2e-2 if bf16 else 1e-5
     assert (got.delta_val.double() - want.delta_val).norm() <= tol * want.delta_val.norm()
+
+
+@pytest.mark.parametrize("M,r,bf16,rows", [
+    (4096, 64, False, True), (4097, 64, False, False), (4080, 64, True, True), (4081, 64, True, False),
+    (1024, 256, False, True), (1025, 256, False, False), (1008, 256, True, True), (1009, 256, True, False),
+    (16384, 65, False, True), (16385, 65, False, False), (32768, 32, True, True), (32769, 32, True, False),
+])
+def test_rows_kernel_on_both_sides_of_its_line(M, r, bf16, rows):
+    """Three-term and bf16 products of at most 2048 and fewer than 2048 tiles of 16 x 16, others by their rows."""
+    import jakal_net_native as jn
+
+    jn.profile_enable(True)
+    try:
+        _project(torch.device("cuda:0"), M, r, 64, bf16)
+        names = [n for n in jn.profile_collect() if "project" in n]
+    finally:
+        jn.profile_enable(False)
+    assert len(names) == 1 and names[0].startswith("gemm_rows_kernel") == rows, names
