@@ -13,12 +13,14 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _project(dev, M, r, K, bf16):
-    """projections [M, 2r] of a window forward (one node per batch element) with its operands."""
+def _project(dev, M, r, K, bf16, of=None):
+    """projections [M, 2r] of a window forward (one node per batch element) with its operands: the first M rows of
+    `of` rows."""
     import jakal_net_native as jn
 
-    g = torch.Generator().manual_seed(M * 131 + r * 17 + K)
-    X = torch.randn(M, 1, K, generator=g).to(dev, torch.bfloat16 if bf16 else torch.float32)
+    of = of or M
+    g = torch.Generator().manual_seed(of * 131 + r * 17 + K)
+    X = torch.randn(of, 1, K, generator=g)[:M].to(dev, torch.bfloat16 if bf16 else torch.float32)
     U, V = (torch.randn(r, K, generator=g).to(dev) for _ in range(2))
     ps, w = torch.randn(M, 1, generator=g).to(dev), torch.ones(r, device=dev)
     ds, proj = torch.empty(M, 1, device=dev), torch.full((M, 2 * r), float("nan"), device=dev)
@@ -90,3 +92,40 @@ def test_rows_kernel_on_both_sides_of_its_line(M, r, bf16, rows):
     finally:
         jn.profile_enable(False)
     assert len(names) == 1 and names[0].startswith("gemm_rows_kernel") == rows, names
+
+
+@pytest.mark.parametrize("r,K,bf16,of", [
+    (64, 136, False, 4200),   # three-term: a call of one tile of rows more than the line, and of fewer
+    (80, 520, False, 3300),
+    (64, 136, True, 4200),    # bf16 MFMAs
+    (96, 264, True, 2900),
+    (40, 520, False, 32800),  # fp32 MFMAs, four chains
+    (64, 72, False, 40),      # (too few rows for the MFMA tile kernels)
+    (33, 136, True, 32800),   # the same on widened bf16 rows
+])
+def test_rows_kernel_has_the_bits_of_the_tile_kernel(r, K, bf16, of):
+    """The rows of a large call, on the kernel that the rows kernel stands for, and the same rows in calls that it
+    takes: top-k selections downstream must not depend on the number of rows."""
+    import jakal_net_native as jn
+
+    dev = torch.device("cuda:0")
+    fp32_mfma = 2 * r < 128 or of < 128
+
+    def run(M, forced=0):
+        jn.set_gemm_tile(forced)
+        jn.profile_enable(True)
+        try:
+            out = _project(dev, M, r, K, bf16, of)[3]
+            names = [n for n in jn.profile_collect() if "project" in n]
+        finally:
+            jn.profile_enable(False)
+            jn.set_gemm_tile(0)
+        return out, names[0].startswith("gemm_rows_kernel")
+
+    want, on_rows = run(of, 64 if fp32_mfma else 0)
+    assert not on_rows
+    for M in {1, 17, 40, 200, 1040, 2500, of - 1}:
+        got, on_rows = run(min(M, of))
+        if on_rows and (fp32_mfma or M >= 128):  # (below 128 rows every wide projection is one of fp32 MFMAs)
+            assert torch.equal(got, want[:M]), M
+        assert on_rows or M > 1040, M

@@ -214,3 +214,23 @@ def test_bf16_dense_step_is_the_same_on_both_tiles(dev):
             assert torch.equal(a, b), i
         else:
             assert (a - b).norm() <= 1e-5 * b.norm()
+
+
+def test_three_term_products_are_the_same_on_both_tiles(dev):
+    """A window layer's projections and input gradient on 256 tiles of 128 x 128 and on 255, which take 64 x 64: every
+    element keeps its chain over K, so the rows both calls have are the same bit for bit."""
+    import jakal_net_native as jn
+
+    B, N, D, r = 256, 128, 128, 64
+    g = torch.Generator().manual_seed(4800)
+    val, state, gs, gv = (torch.randn(B, N, *s, generator=g).to(dev) for s in ((D,), (), (), (D,)))
+    U, V = ((torch.randn(r, D, generator=g) / D**0.5).to(dev) for _ in range(2))
+    w = torch.full((r,), r**-0.5, device=dev)
+
+    def run(n):
+        X, ps = val[:n].clone().requires_grad_(True), state[:n].clone().requires_grad_(True)
+        out = jn.propagation_window("low_rank_bilinear", w, None, V, None, U, None, "softsign", X, ps, X, 16, N, N)
+        return [t[:B - 1] for t in (*out, *torch.autograd.grad(out, [X, ps], [gs[:n], gv[:n]]))]
+
+    for a, b in zip(run(B), run(B - 1)):
+        assert torch.equal(a, b)
