@@ -826,7 +826,7 @@ int propagation_edges_backward(const float* layer_val, const float* projected_st
       ca.gds = nullptr;
       ca.rec_eid = 1;
       ca.pos = s.pos;
-      const SideStream* side = side_stream_for(st, (int64_t)M * k);
+      const SideStream* side = csr_layout_empty(ca) ? nullptr : side_stream_for(st, (int64_t)M * k);
       if (side) {
         rc = fork_to(side, st);
         if (rc) return rc;
@@ -890,10 +890,11 @@ int propagation_edges_backward(const float* layer_val, const float* projected_st
   }
   if (!dot_slabs) {
     const SideStream* side = side_stream_for(st, (int64_t)M * k);
+    const SideStream* layout_side = !band && !csr_layout_empty(ca) ? side : nullptr;
     if (!band) {
-      hipStream_t cs = side ? side->stream : st;
-      if (side) {
-        rc = fork_to(side, st);
+      hipStream_t cs = layout_side ? layout_side->stream : st;
+      if (layout_side) {
+        rc = fork_to(layout_side, st);
         if (rc) return rc;
       }
       rc = launch_csr_layout(ca, cs);
@@ -927,8 +928,8 @@ int propagation_edges_backward(const float* layer_val, const float* projected_st
     // 2b. the edge records, grouped by key (deterministic transpose; a band's
     //     is closed form and needs none)
     if (!band) {
-      if (side) {
-        rc = join_from(side, st);
+      if (layout_side) {
+        rc = join_from(layout_side, st);
         if (rc) return rc;
       }
       rc = launch_csr_fill(ca, st);
@@ -1599,6 +1600,7 @@ static int transition_topk_forward_impl(const float* sender_strength, const floa
   ca.rec = s.rec;
   ca.coef = s.coef;
   ca.gds = projected_state;
+  if (csr_layout_empty(ca)) side = nullptr;
   if (side) {
     rc = fork_to(side, st);
     if (rc) return rc;
@@ -1708,16 +1710,17 @@ static int transition_topk_backward_impl(const float* sender_strength, const flo
   ca.g_score = s.g_logit;
   ca.ehead = mh ? route_head : nullptr;
   const SideStream* side = side_stream_for(st, (int64_t)B * Ns * k);
-  if (side) {
-    rc = fork_to(side, st);
+  const SideStream* layout_side = csr_layout_empty(ca) ? nullptr : side;
+  if (layout_side) {
+    rc = fork_to(layout_side, st);
     if (rc) return rc;
   }
-  rc = launch_csr_layout(ca, side ? side->stream : st);
+  rc = launch_csr_layout(ca, layout_side ? layout_side->stream : st);
   if (rc) return rc;
   rc = launch_route_rows_backward(rb, st);
   if (rc) return rc;
-  if (side) {
-    rc = join_from(side, st);
+  if (layout_side) {
+    rc = join_from(layout_side, st);
     if (rc) return rc;
   }
 

@@ -1046,6 +1046,8 @@ __global__ __launch_bounds__(64 * kCsrGroupWaves) void csr_group_kernel(CsrArgs 
 
 static bool csr_group_fits(const CsrArgs& a) { return (int64_t)a.Nq * a.k <= kCsrGroupEdges && a.B < 65536; }
 
+bool csr_layout_empty(const CsrArgs& a) { return csr_group_fits(a); }
+
 static int launch_csr_group(const CsrArgs& a, hipStream_t stream) {
   // about a workgroup per CU, 4 to 64 keys each
   const int kg = (int)std::min<int64_t>(kWave, std::max<int64_t>(4, ((int64_t)a.B * a.Nk + 255) / 256));

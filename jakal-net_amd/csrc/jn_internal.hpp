@@ -468,7 +468,9 @@ int launch_csr(const CsrArgs& a, hipStream_t stream);
 // The two halves of launch_csr: the layout (per-tile edge counts, segment
 // starts and per-tile slots; reads only the edge index) and the fill (the
 // records; reads the coefficients, score gradients and state gradients as
-// well).  Small edge lists are grouped by the fill alone.
+// well).  Small edge lists are grouped by the fill alone: the layout launches
+// nothing (csr_layout_empty), so there is nothing to run on another stream.
+bool csr_layout_empty(const CsrArgs& a);
 int launch_csr_layout(const CsrArgs& a, hipStream_t stream);
 int launch_csr_fill(const CsrArgs& a, hipStream_t stream);
 
