@@ -1170,6 +1170,8 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
   }
 
   // ---- sort each row's k winners and write them -----------------------------
+  // (a row of NaN scores keeps fewer than k: what its list lacks comes back as
+  // -inf with some index in range, as above)
   if constexpr (KEEP == 48) {
     // k <= 32: two rows per pass, row t + h on half-wave h
     const int h = lane >> 5, e = lane & 31;
@@ -1179,7 +1181,8 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
       const int slot = wave * kSelRowsPerWave + t + h;
       float vs = -INFINITY;
       int vi = 0x7fffffff;
-      if (e < k) {
+      const int n0 = readlane_i(kept, t), n1 = readlane_i(kept, t + 1);
+      if (e < min(k, h ? n1 : n0)) {
         vs = key_to_float(s_kept_k[slot * KST + e]);
         vi = s_kept_i[slot * KIST + e];
       }
@@ -1190,7 +1193,7 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
       }
       if (e < k && row < a.Nq) {
         const int64_t o = ((int64_t)b * a.Nq + row) * k + e;
-        a.out_idx[o] = vi;
+        a.out_idx[o] = vi < a.Nk ? vi : e;
         a.out_score[o] = vs;
       }
     }
@@ -1201,7 +1204,7 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
     const int slot = wave * kSelRowsPerWave + t;
     float vs = -INFINITY;
     int vi = 0x7fffffff;
-    if (lane < k) {
+    if (lane < min(k, readlane_i(kept, t))) {
       vs = key_to_float(s_kept_k[slot * KST + lane]);
       vi = s_kept_i[slot * KIST + lane];
     }
@@ -1209,7 +1212,7 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
     if (scaled_domain) vs = ldexpf(vs, -readlane_i(score_exp, t));
     if (lane < k) {
       const int64_t o = ((int64_t)b * a.Nq + row) * k + lane;
-      a.out_idx[o] = vi;
+      a.out_idx[o] = vi < a.Nk ? vi : lane;
       a.out_score[o] = vs;
     }
   }

@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void topk_rows_kernel(const float* S, int64_t 
   }
   const int64_t orow = out_row0 + blockIdx.x;
   for (int e = tid; e < k; e += 256) {
-    out_idx[orow * k + e] = ci[e];
+    out_idx[orow * k + e] = ci[e] < Nk ? ci[e] : e;  // (padding sorted before NaN scores: some index in range)
     out_score[orow * k + e] = cs[e];
   }
 }

@@ -302,3 +302,27 @@ def test_key_split_heads(dev, heads, head_rank, k, N):
         jn.set_select_mode(jn.SELECT_SPLIT_F16)
     a, b = out[jn.SELECT_SPLIT_F16_WAVE], out[jn.SELECT_SPLIT_F16_KEYSPLIT]
     assert torch.equal(a.delta_state, b.delta_state) and torch.equal(a.delta_val, b.delta_val)
+
+
+@pytest.mark.parametrize("mode", ["SELECT_SPLIT_F16", "SELECT_F32", "SELECT_SPLIT_F16_WAVE", "SELECT_SPLIT_F16_COOP4",
+                                  "SELECT_SPLIT_F16_REGISTER"])
+@pytest.mark.parametrize("k,Nk", [(12, 800), (32, 2100), (64, 2100), (80, 700)])
+def test_rows_without_comparable_scores(dev, mode, k, Nk):
+    """A row of NaN scores comes back with indices in range from every kernel (a gather or an edge grouping reads
+    through them), and the other rows come back as they do without it."""
+    import jakal_net_native as jn
+
+    g = torch.Generator().manual_seed(9300 + k)
+    q, key = torch.randn(2, 300, 24, generator=g).to(dev), torch.randn(2, Nk, 24, generator=g).to(dev)
+    scale = (torch.rand(24, generator=g) + 0.5).to(dev)
+    bad = q.clone()
+    bad[:, 5] = float("nan")
+    bad[1, 299] = float("nan")
+    try:
+        jn.set_select_mode(getattr(jn, mode))
+        (wi, ws), (gi, gs) = (jn.low_rank_topk_select(x, key, scale, None, False, 1.0, k) for x in (q, bad))
+    finally:
+        jn.set_select_mode(jn.SELECT_SPLIT_F16)
+    ok = ~bad.isnan().any(-1)
+    assert torch.equal(wi[ok], gi[ok]) and torch.equal(ws[ok], gs[ok])
+    assert int(gi.min()) >= 0 and int(gi.max()) < Nk
