@@ -51,13 +51,14 @@ constexpr int kSelectSplitF16 = 0;
 // Split fp16 on one kernel only (tests): the per-wave streaming kernel, or the
 // 4-wave cooperative (LDS-staged) kernel whenever the rank is at most 64.
 // kSelectSplitF16 picks the cooperative kernel for rank <= 64 on grids of at
-// least 512 workgroups (fp32 keys of rank > 32: 257), else the per-wave kernel.
+// least 512 workgroups (fp32 keys of rank > 32 with k <= 32 or >= 4096 keys:
+// 257), else the per-wave kernel.
 // (Mode 3 is retired.)
 constexpr int kSelectSplitF16Wave = 2;
 constexpr int kSelectSplitF16Coop4 = 4;
 // Split fp16 on the key-split per-wave kernel whenever k <= 32 (tests); mode 0
 // picks it with >= 192 keys on grids below 256 workgroups of the per-wave kernel
-// for k <= 16, below 129 for k <= 32.
+// for k <= 16; for k <= 32 below 129 with >= 2048 keys, below 65 with >= 384.
 constexpr int kSelectSplitF16KeySplit = 5;
 // Split fp16 on the register kernels only: mode 0 as it was before the
 // small-key select (tests and A/B timing).

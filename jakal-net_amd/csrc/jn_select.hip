@@ -1284,18 +1284,26 @@ constexpr int64_t kSelCoop4MinBlocks = 512;
 // fp32 keys of 33 to 64 ranks load twice the bytes per score: there the staging
 // wins from the first workgroup beyond one per CU (4096 keys, k = 32: 320
 // workgroups 177 us against 257 per wave, 256 workgroups 154 against 155; bf16
-// keys and ranks <= 32 are level, 152 against 156 and 155 against 155).
+// keys and ranks <= 32 are level, 152 against 156 and 155 against 155).  Longer
+// lists merge every wave more often: with fewer keys than kSelCoop4WideKeys they
+// are better off per wave (400 workgroups, k = 64: 1100 keys 145 against 134,
+// 2048 keys 189 against 186).
 constexpr int64_t kSelCoop4MinBlocksWide = 257;
+constexpr int kSelCoop4WideKeys = 4096;
 // Below one 64-row workgroup per CU, with k <= 16 and at least four key chunks,
 // the key-split per-wave form runs a quarter of the serial chunk chain.  Lists
 // of up to 32 take longer to merge: it serves them while its workgroups of 16
 // rows fit the chip at two per CU (4096 keys, k = 32: 64 workgroups of 64 rows
 // 77 us against 150 per wave, 128: 104 against 155, 192: 157 against 154; rank
 // 128: 103 against 254 and 200 against 260; two heads of rank 32: 105 against
-// 157 at 128).
+// 157 at 128).  With few keys a wave's quarter is soon scanned and the merges
+// are what is left: below kSelKspKeys32 keys up to 64 workgroups (1100 keys, rank
+// 100: 100 workgroups 121 against 105; 512 keys in bf16, 128: 78 against 72 of
+// the whole forward), none below kSelKspMinKeys32 (256 keys, 16: 56 against 53).
 constexpr int64_t kSelKspMaxBlocks = 256;
-constexpr int64_t kSelKspMaxBlocks32 = 129;
+constexpr int64_t kSelKspMaxBlocks32 = 129, kSelKspMaxBlocks32Few = 65;
 constexpr int kSelKspMinKeys = 4 * kSelChunk;
+constexpr int kSelKspMinKeys32 = 384, kSelKspKeys32 = 2048;
 
 namespace {
 std::atomic<int> g_select_mode{kSelectSplitF16};
@@ -1402,13 +1410,17 @@ int launch_topk_select(const SelectArgs& a_in, hipStream_t stream) {
     }
     a.split_key = s.split;
     a.split_exp = s.kexp;
-    const int64_t coop4_min = RP > 32 && !a.bf16 ? kSelCoop4MinBlocksWide : kSelCoop4MinBlocks;
-    const int64_t ksp_max = a.k <= 16 ? kSelKspMaxBlocks : kSelKspMaxBlocks32;
+    const bool coop4_wide = RP > 32 && !a.bf16 && (a.k <= 32 || a.Nk >= kSelCoop4WideKeys);
+    const int64_t coop4_min = coop4_wide ? kSelCoop4MinBlocksWide : kSelCoop4MinBlocks;
+    const int64_t ksp_max = a.k <= 16             ? kSelKspMaxBlocks
+                            : a.Nk >= kSelKspKeys32 ? kSelKspMaxBlocks32
+                                                    : kSelKspMaxBlocks32Few;
+    const int ksp_keys = a.k <= 16 ? kSelKspMinKeys : kSelKspMinKeys32;
     const bool coop4 = !mh && RP <= 64 &&
                        (mode == kSelectSplitF16Coop4 || (mode == kSelectSplitF16 && blocks >= coop4_min));
     const bool ksp = !coop4 && a.k <= 32 &&
                      (mode == kSelectSplitF16KeySplit ||
-                      (mode == kSelectSplitF16 && blocks < ksp_max && a.Nk >= kSelKspMinKeys));
+                      (mode == kSelectSplitF16 && blocks < ksp_max && a.Nk >= ksp_keys));
     const int64_t kblocks = (int64_t)((a.Nq + kSelRowsPerWave - 1) / kSelRowsPerWave) * a.B;
     JN_REQUIRE(!ksp || kblocks < (1LL << 31), kInvalidArgument, "bad grid size");
     const dim3 kgrid((unsigned)kblocks);

@@ -326,3 +326,28 @@ def test_rows_without_comparable_scores(dev, mode, k, Nk):
     ok = ~bad.isnan().any(-1)
     assert torch.equal(wi[ok], gi[ok]) and torch.equal(ws[ok], gs[ok])
     assert int(gi.min()) >= 0 and int(gi.max()) < Nk
+
+
+@pytest.mark.parametrize("blocks,Nk,r,k,form", [
+    (257, 1100, 64, 32, 4), (256, 1100, 64, 32, 0), (511, 2048, 64, 33, 0), (257, 4096, 64, 64, 4), (511, 4096, 32, 8, 0),
+    (512, 1100, 32, 64, 4),
+    (128, 2048, 64, 32, -1), (129, 2048, 64, 32, 0), (64, 1100, 100, 17, -1), (65, 1100, 100, 17, 0),
+    (255, 1100, 100, 16, -1), (256, 1100, 100, 16, 0), (1, 4096, 64, 33, 0),
+])
+def test_kernel_of_a_select(dev, blocks, Nk, r, k, form):
+    """Which form a select of split keys runs on either side of each line (4: cooperative, -1: key-split, 0: per wave;
+    the fifth template argument)."""
+    import re
+
+    import jakal_net_native as jn
+    from torch.profiler import ProfilerActivity, profile
+
+    q, key, scale = (torch.randn(*s, device=dev) for s in ((1, 64 * blocks, r), (1, Nk, r), (r,)))
+    call = lambda: jn.low_rank_topk_select(q, key, scale, None, False, 1.0, k)  # noqa: E731
+    call()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages() if "lowrank_topk_select_kernel<" in e.key]
+    forms = {int(re.search(r"<(.*?)>", n).group(1).split(",")[4]) for n in names}
+    assert forms == {form}, names
