@@ -932,9 +932,8 @@ __global__ __launch_bounds__(256) void csr_fill_kernel(CsrArgs a, int tile_rows,
 // own 5 us per launch 6.3 + 6.2 + 11.5 -> 7.2 us at 16 x 256 rows of 16 edges,
 // 7.7 + 6.4 + 12.6 -> 8.4 at 8 x 1024 (256) rows of 16.  The index is read
 // ceil(Nk / kg) times per element, from L2, and a workgroup with hubs (keys
-// that many rows choose) takes them in one wave's steps, so it serves lists of
-// up to kCsrGroupEdges edges per element (20,000 edges on 1531 keys: 21.6 us
-// against 27 in three launches, 17 against 12 without the events).  k_inv: ceil(2^32 / k), so that the high
+// that many rows choose) takes them in one wave's steps: csr_group_fits has
+// where that costs more than the launches.  k_inv: ceil(2^32 / k), so that the high
 // word of e * k_inv is e / k (exact while e k < 2^32; k > 1).
 constexpr int kCsrGroupWaves = 16;
 constexpr int kCsrGroupEdges = 16 * 64 * kCsrGroupWaves;  // 16 edges per lane at most
@@ -1044,7 +1043,22 @@ __global__ __launch_bounds__(64 * kCsrGroupWaves) void csr_group_kernel(CsrArgs 
   }
 }
 
-static bool csr_group_fits(const CsrArgs& a) { return (int64_t)a.Nq * a.k <= kCsrGroupEdges && a.B < 65536; }
+// Besides the edges of an element, what every key group reads of them counts:
+// B k Nk times the rows (1024 at most: the three launches walk more rows than
+// that at no better a rate).  Up to 16 elements one launch was never the slower
+// way (64 to 65,536 keys); beyond, from 2^30 on it is, first where the lists have
+// hubs (the whole calls around the grouping, B x rows of k on Nk keys, one launch
+// against three, on random / crowded keys: 64 x 1024 of 16 on 512 keys 122 / 173
+// us against 141 / 171, on 1024 138 / 175 against 152 / 172, on 4096 258 / 263
+// against 238 / 224; 32 x 512 of 32 on 4096 137 / 137 against 135 / 125, 128 x 512
+// of 32 on 2048 340 / 391 against 323 / 311; 32 x 4096 of 4 on 4096 145 / 170
+// against 168 / 181).
+constexpr int64_t kCsrGroupBatch = 16, kCsrGroupReads = 1LL << 30;
+
+static bool csr_group_fits(const CsrArgs& a) {
+  if ((int64_t)a.Nq * a.k > kCsrGroupEdges || a.B >= 65536) return false;
+  return a.B <= kCsrGroupBatch || (int64_t)a.B * a.k * min(a.Nq, 1024) * a.Nk < kCsrGroupReads;
+}
 
 bool csr_layout_empty(const CsrArgs& a) { return csr_group_fits(a); }
 

@@ -157,6 +157,8 @@ def test_edge_layout_is_the_stable_key_sort(dev, B, N, k):
     (1, 2, 1, 1), (2, 70, 7, 1), (17, 64, 4, 2), (3, 500, 32, 1), (1, 4000, 4, 1), (5, 129, 64, 1), (2, 5, 3, 1),
     (2, 1024, 16, 1),   # 16,384 edges per element: the largest grouped in one launch
     (2, 1025, 16, 1),   # above: count, prefix and fill
+    (63, 1024, 16, 1),  # the largest batch of such lists grouped in one launch
+    (64, 1024, 16, 1),  # above: count, prefix and fill
 ])
 def test_grouping_is_a_stable_sort(dev, B, N, k, heads):
     """Segments, records and record indices of the layout against a stable sort of each element's edges by key."""
@@ -200,3 +202,28 @@ def test_grouping_is_a_stable_sort(dev, B, N, k, heads):
         s = score[b][order]
         np.testing.assert_allclose(rec[b, :, 1].copy().view(np.float32), s / (1 + np.abs(s)), rtol=1e-6)
         np.testing.assert_array_equal(pos[b][order], b * N * k + np.arange(N * k))
+
+
+@pytest.mark.parametrize("B,Ns,k,Nd,launches", [
+    (8, 64, 16, 16384, 1), (16, 1024, 16, 4096, 1),  # up to 16 elements: in one launch whatever the keys
+    (32, 512, 16, 1024, 1), (32, 512, 16, 8192, 3),  # 2^28 and 2^31 in the rule's measure
+    (32, 1024, 16, 2040, 1), (32, 1024, 16, 2048, 3),
+])
+def test_grouping_rule_counts_keys(dev, B, Ns, k, Nd, launches):
+    """Every key group reads the whole list again, so many keys of many elements take three launches."""
+    import jakal_net as J
+    import jakal_net_native as jn
+
+    D = 8
+    op = J.SparseTransition(J.LowRankBilinearRoute(D, D, rank=8), topk=k, implementation="native").to(dev)
+    layer = lambda n: J.Layer(D, n, torch.randn(B, n, device=dev), torch.randn(B, n, D, device=dev))  # noqa: E731
+    src, dst = layer(Ns), layer(Nd)
+    jn.profile_enable(True)
+    try:
+        with torch.no_grad():
+            op.compute_delta(src, dst)
+        torch.cuda.synchronize()
+        names = [n for n in jn.profile_collect() if n.startswith("csr_")]
+    finally:
+        jn.profile_enable(False)
+    assert len(names) == launches and (launches == 3 or names[0].startswith("csr_group_kernel")), names
