@@ -367,7 +367,7 @@ struct DenseScoreGradArgs {
 // leaves its registers.  The rows' value fragments stay in registers; the
 // columns' values (pieces of a row exchanged by its row number, so that 16 rows'
 // pieces lie in distinct banks), ranks and transposed projections are staged in
-// LDS.  64 rows per workgroup and 48 KB of LDS at D = 512: two share a CU, and
+// LDS.  64 rows per workgroup and 66 KB of LDS at D = 512: two share a CU, and
 // one's barriers and LDS phases run beside the other's MFMAs.
 // Bound: MFMA (per 64 x 32 pairs and SIMD 1024 cycles of scores and 1024 of
 // G . P at rank 64, 512 of gdv . pv^T at D = 512) and LDS reads (1500 cycles).
