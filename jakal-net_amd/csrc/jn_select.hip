@@ -868,6 +868,15 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
   int kept = 0;  // valid kept entries of this lane's row (<= k)
   uint32_t* my_kept_k = s_kept_k + lrow * KST;
   uint16_t* my_kept_i = s_kept_i + lrow * KIST;
+  if constexpr (!KSP) {
+    // A row of NaN scores keeps fewer than k: what its list lacks comes back as
+    // -inf with some index in range.  (Set here once: a test or a fill at the
+    // end cost 3 us of 340 and 280 at 16 x 4096 rows.)
+    for (int e = lane / kSelRowsPerWave; e < k; e += kWave / kSelRowsPerWave) {
+      my_kept_k[e] = order_key(-INFINITY);
+      my_kept_i[e] = (uint16_t)e;
+    }
+  }
   float* wave_cand_s = s_cand_s + wave * CAP * kWave;
   uint16_t* wave_cand_i = s_cand_i + wave * CAP * kWave;
   float* my_cand_s = wave_cand_s + lane;
@@ -1170,8 +1179,6 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
   }
 
   // ---- sort each row's k winners and write them -----------------------------
-  // (a row of NaN scores keeps fewer than k: what its list lacks comes back as
-  // -inf with some index in range, as above)
   if constexpr (KEEP == 48) {
     // k <= 32: two rows per pass, row t + h on half-wave h
     const int h = lane >> 5, e = lane & 31;
@@ -1181,8 +1188,7 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
       const int slot = wave * kSelRowsPerWave + t + h;
       float vs = -INFINITY;
       int vi = 0x7fffffff;
-      const int n0 = readlane_i(kept, t), n1 = readlane_i(kept, t + 1);
-      if (e < min(k, h ? n1 : n0)) {
+      if (e < k) {
         vs = key_to_float(s_kept_k[slot * KST + e]);
         vi = s_kept_i[slot * KIST + e];
       }
@@ -1193,7 +1199,7 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
       }
       if (e < k && row < a.Nq) {
         const int64_t o = ((int64_t)b * a.Nq + row) * k + e;
-        a.out_idx[o] = vi < a.Nk ? vi : e;
+        a.out_idx[o] = vi;
         a.out_score[o] = vs;
       }
     }
@@ -1204,7 +1210,7 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
     const int slot = wave * kSelRowsPerWave + t;
     float vs = -INFINITY;
     int vi = 0x7fffffff;
-    if (lane < min(k, readlane_i(kept, t))) {
+    if (lane < k) {
       vs = key_to_float(s_kept_k[slot * KST + lane]);
       vi = s_kept_i[slot * KIST + lane];
     }
@@ -1212,7 +1218,7 @@ __global__ __launch_bounds__(CW > 0 ? CW * 64 : 256,
     if (scaled_domain) vs = ldexpf(vs, -readlane_i(score_exp, t));
     if (lane < k) {
       const int64_t o = ((int64_t)b * a.Nq + row) * k + lane;
-      a.out_idx[o] = vi < a.Nk ? vi : lane;
+      a.out_idx[o] = vi;
       a.out_score[o] = vs;
     }
   }
