@@ -957,7 +957,9 @@ def main() -> int:
         measured = json.loads(traffic_file.read_text()).get("kernels", {})
         # timing names whose kernel function has another name in the rocprofv3 summaries
         for name, func in (("route_gather_kernel", "cols_gather_kernel"),
-                           ("unit_scale_backward_kernel", "unit_scale_kernel")):
+                           ("unit_scale_backward_kernel", "unit_scale_kernel"),
+                           ("dense_colsum_kernel", "colsum_rows_kernel"),
+                           ("route_dense_colsum_kernel", "colsum_narrow_kernel")):
             if name not in measured and func in measured:
                 measured[name] = measured[func]
     for name, entry in kernels.items():
