@@ -239,10 +239,19 @@ static int64_t rows_tiles(const RowsGemm& g) { return (int64_t)((g.M + 15) / 16)
 // count: up to 2048 tiles of 16 x 16 on three-term products, fewer on bf16 ones
 // (level there, 11.7 against 11.3 us, and slower beyond).  Against
 // gemm_f32_kernel, at any number of columns, the rows: 32,768, or 16,384 from
-// 128 columns on (the largest measured).
+// 128 columns on (the largest measured), but for fp32 products that fill about
+// three of its 64 x 64 tiles per CU, which run at their best there (K = 512 /
+// 200: 16,384 x 130 47 / 27 us against 51 / 30 here, 12,288 x 194 49 / 27
+// against 54 / 31, 8192 x 322 49 / 27 against 54 / 31, 24,576 x 114 49 / 28
+// against 55 / 32; 24,576 x 82 only half fills them, 49 / 28 against 44 / 27;
+// at other counts 2 to 40 % faster here).
 static bool rows_few(const RowsGemm& g) {
   if (g.arith == kRowsX3) return rows_tiles(g) <= 2048;
   if (g.arith == kRowsBf) return rows_tiles(g) < 2048;
+  if (g.arith == kRowsC4) {
+    const int64_t t64 = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64);
+    if (t64 > 640 && t64 <= 768 && (int64_t)g.M * g.N * 3 > t64 * 64 * 64 * 2) return false;
+  }
   return g.M <= (g.N >= 128 ? kRowsMaxM / 2 : kRowsMaxM);
 }
 
@@ -272,13 +281,17 @@ static void launch_rows(const RowsGemm* p, int n, hipStream_t stream) {
 
 template <int ARITH>
 static void launch_rows_tile(const RowsGemm* p, int n, hipStream_t stream) {
-  int64_t tiles = 0;
-  for (int i = 0; i < n; ++i) tiles += rows_tiles(p[i]);
-  // the largest tile that still gives every SIMD (1024) two waves (K = 512,
-  // N = 128: 30 us at 16,384 rows on 32 x 32 tiles against 38 on 16 x 32); the
-  // MFMA tile kernels take over before 32 x 32 ones would
+  int64_t tiles = 0, waves = 0;  // of 16 x 16, and of 16 x 32
+  for (int i = 0; i < n; ++i) {
+    tiles += rows_tiles(p[i]);
+    waves += (int64_t)((p[i].M + 15) / 16) * ((p[i].N + 31) / 32);
+  }
+  // the largest tile that still gives every SIMD (1024) two waves, 32 x 32 also
+  // where 16 x 32 would make a fourth (K = 512: 30 us at 16,384 x 128 against 38
+  // on 16 x 32, 32 at 16,384 x 98 against 39; 24,576 x 66, of 4.5 waves of 16 x
+  // 32 each, 43 against 40).  The MFMA tile kernels take over before those.
   if constexpr (ARITH == kRowsC4 || ARITH == kRowsC4Bf) {
-    if (tiles >= 8192) return launch_rows<ARITH, 2, 2, 2>(p, n, stream);
+    if (tiles >= 8192 || (waves > 3 * 1024 && waves <= 4 * 1024)) return launch_rows<ARITH, 2, 2, 2>(p, n, stream);
   }
   if (tiles >= 2048) launch_rows<ARITH, 1, 2, 3>(p, n, stream);
   else launch_rows<ARITH, 1, 1, 4>(p, n, stream);

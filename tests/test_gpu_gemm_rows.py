@@ -79,10 +79,13 @@ def test_two_projections_in_one_launch(Ns, Nd, r, bf16):
 @pytest.mark.parametrize("M,r,bf16,rows", [
     (4096, 64, False, True), (4097, 64, False, False), (4080, 64, True, True), (4081, 64, True, False),
     (1024, 256, False, True), (1025, 256, False, False), (1008, 256, True, True), (1009, 256, True, False),
-    (16384, 65, False, True), (16385, 65, False, False), (32768, 32, True, True), (32769, 32, True, False),
+    (16384, 129, False, True), (16385, 129, False, False), (32768, 32, True, True), (32769, 32, True, False),
+    (13632, 65, False, True), (13633, 65, False, False), (16384, 65, False, False), (16384, 65, True, True),
+    (24576, 41, False, True), (24576, 57, False, False),  # three 64 x 64 tiles per CU, half and nearly filled
 ])
 def test_rows_kernel_on_both_sides_of_its_line(M, r, bf16, rows):
-    """Three-term and bf16 products of at most 2048 and fewer than 2048 tiles of 16 x 16, others by their rows."""
+    """Three-term and bf16 products of at most 2048 and fewer than 2048 tiles of 16 x 16, others by their rows, fp32
+    ones but for those that fill three 64 x 64 tiles per CU."""
     import jakal_net_native as jn
 
     jn.profile_enable(True)
