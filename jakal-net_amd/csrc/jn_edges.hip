@@ -1046,14 +1046,12 @@ __global__ __launch_bounds__(64 * kCsrGroupWaves) void csr_group_kernel(CsrArgs 
 // Besides the edges of an element, what every key group reads of them counts:
 // B k Nk times the rows (1024 at most: the three launches walk more rows than
 // that at no better a rate).  Up to 16 elements one launch was never the slower
-// way (64 to 65,536 keys); beyond, from 2^30 on it is, first where the lists have
-// hubs (the whole calls around the grouping, B x rows of k on Nk keys, one launch
-// against three, on random / crowded keys: 64 x 1024 of 16 on 512 keys 122 / 173
-// us against 141 / 171, on 1024 138 / 175 against 152 / 172, on 4096 258 / 263
-// against 238 / 224; 32 x 512 of 32 on 4096 137 / 137 against 135 / 125, 128 x 512
-// of 32 on 2048 340 / 391 against 323 / 311; 32 x 4096 of 4 on 4096 145 / 170
-// against 168 / 181).
-constexpr int64_t kCsrGroupBatch = 16, kCsrGroupReads = 1LL << 30;
+// way (64 to 65,536 keys); beyond, from about 2^31 on it is.  Whole training
+// steps, one launch against three: top-k 64 x 1024 rows of 16 716 against 728 us,
+// 128 x 1024 of 12 1177 against 1192; routes 32 x 1024 of 16 to 4096 (2^31) 1982
+// against 1987, 64 x (2^32) 3841 against 3812, 64 x 512 of 32 4070 against 4023,
+// 64 x 512 of 16 to 8192 6238 against 6191.
+constexpr int64_t kCsrGroupBatch = 16, kCsrGroupReads = 1LL << 31;
 
 static bool csr_group_fits(const CsrArgs& a) {
   if ((int64_t)a.Nq * a.k > kCsrGroupEdges || a.B >= 65536) return false;

@@ -157,8 +157,8 @@ def test_edge_layout_is_the_stable_key_sort(dev, B, N, k):
     (1, 2, 1, 1), (2, 70, 7, 1), (17, 64, 4, 2), (3, 500, 32, 1), (1, 4000, 4, 1), (5, 129, 64, 1), (2, 5, 3, 1),
     (2, 1024, 16, 1),   # 16,384 edges per element: the largest grouped in one launch
     (2, 1025, 16, 1),   # above: count, prefix and fill
-    (63, 1024, 16, 1),  # the largest batch of such lists grouped in one launch
-    (64, 1024, 16, 1),  # above: count, prefix and fill
+    (127, 1024, 16, 1),  # the largest batch of such lists grouped in one launch
+    (128, 1024, 16, 1),  # above: count, prefix and fill
 ])
 def test_grouping_is_a_stable_sort(dev, B, N, k, heads):
     """Segments, records and record indices of the layout against a stable sort of each element's edges by key."""
@@ -206,8 +206,8 @@ def test_grouping_is_a_stable_sort(dev, B, N, k, heads):
 
 @pytest.mark.parametrize("B,Ns,k,Nd,launches", [
     (8, 64, 16, 16384, 1), (16, 1024, 16, 4096, 1),  # up to 16 elements: in one launch whatever the keys
-    (32, 512, 16, 1024, 1), (32, 512, 16, 8192, 3),  # 2^28 and 2^31 in the rule's measure
-    (32, 1024, 16, 2040, 1), (32, 1024, 16, 2048, 3),
+    (32, 512, 16, 4096, 1), (32, 512, 16, 8192, 3),  # 2^30 and 2^31 in the rule's measure
+    (32, 1024, 16, 4092, 1), (32, 1024, 16, 4096, 3),
 ])
 def test_grouping_rule_counts_keys(dev, B, Ns, k, Nd, launches):
     """Every key group reads the whole list again, so many keys of many elements take three launches."""
