@@ -1021,7 +1021,7 @@ int propagation_edges_backward(const float* layer_val, const float* projected_st
   }
   if (grad_target_weight && grad_source_weight) {
     rc = gemm_grad_weight(s.dP, 2 * r, layer_val, in_dim, grad_target_weight, grad_source_weight, r, 2 * r,
-                          (int)in_dim, M, s.splitk, gside ? gside->stream : st, bf16);
+                          (int)in_dim, M, s.splitk, gside ? gside->stream : st, bf16, gside != nullptr);
     if (rc) return rc;
   }
 

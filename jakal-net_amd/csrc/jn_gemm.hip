@@ -952,6 +952,14 @@ constexpr int kBfT = 128;           // tile M and N
 // tiles 20 against 14.  From 256 tiles on the wide ones win where K is long
 // (route aggregate 79 against 86, weight gradient 20.1 against 22.7).
 constexpr int64_t kTile64Below = 256;
+// A weight gradient beside the input gradient on another stream leaves it more of
+// the chip on wide tiles, from 16,384 rows on and if they make half a tile per CU:
+// training steps of 40,960 x 256 (rank 64, 128 tiles) 446 against 472 us, 65,536 x
+// 384 852 against 889, 65,536 x 256 windows 413 against 437; 40,960 x 128 (64
+// tiles) 421 on 64-wide ones against 427, 16,384 x 192 233 against 235.  bf16
+// layers are within 1 % either way and keep the rule above.
+constexpr int64_t kTile64Beside = 128;
+constexpr int kBesideRows = 16384;
 constexpr int kBfK = 64;            // K per slice
 constexpr int kBfS = kBfK + 8;      // LDS row stride in bf16 elements (144 bytes)
 constexpr int bf_stage(int tile) { return tile / 2 + 4; }  // epilogue row stride in floats
@@ -1633,7 +1641,7 @@ static bool rows_form(const GemmArgs& g, int use, bool fast, RowsGemm& r) {
   return gemm_rows_fits(r);
 }
 
-int launch_gemm(const GemmArgs& g, GemmUse use, int splits, hipStream_t stream) {
+int launch_gemm(const GemmArgs& g, GemmUse use, int splits, hipStream_t stream, int64_t tile64_below = kTile64Below) {
   JN_REQUIRE(g.M >= 0 && g.N >= 0 && g.K >= 0, kInvalidArgument, "negative GEMM extent");
   if (g.M == 0 || g.N == 0) return kOk;
   JN_REQUIRE(g.batch <= 1 || splits == 1, kInvalidArgument, "batched GEMM has no split-K");
@@ -1659,7 +1667,7 @@ int launch_gemm(const GemmArgs& g, GemmUse use, int splits, hipStream_t stream) 
   // the 128-wide MFMA tiles of this product, or 64-wide where those leave CUs
   // idle (or as forced: 32 x 32 tiles are not among them)
   const int64_t tiles128 = (int64_t)((g.M + kBfT - 1) / kBfT) * ((g.N + kBfT - 1) / kBfT) * zdim;
-  const int tile = forced ? (forced == kBfT ? kBfT : 64) : tiles128 < kTile64Below ? 64 : kBfT;
+  const int tile = forced ? (forced == kBfT ? kBfT : 64) : tiles128 < tile64_below ? 64 : kBfT;
   const int tm = (g.M + tile - 1) / tile, tn = (g.N + tile - 1) / tile;
   const int64_t tiles = (int64_t)tm * tn * zdim;
   auto at_tile = [&](auto launch) {
@@ -1902,7 +1910,7 @@ size_t gemm_grad_weight_workspace(int M, int N, int K) {
 // Rows [0, m_split) of dW go to out0, the rest to out1.  Deterministic split-K.
 // x_bf16: X holds bf16 elements.
 int gemm_grad_weight(const float* dP, int64_t ldp, const float* X, int64_t ldx, float* out0, float* out1, int m_split,
-                     int M, int N, int K, float* partial, hipStream_t stream, bool x_bf16) {
+                     int M, int N, int K, float* partial, hipStream_t stream, bool x_bf16, bool beside) {
   int splits = grad_weight_splits(K);
   int k_chunk = (K + splits - 1) / splits;
   // chunks of whole K slices: 32 (the fp32 kernels' 16, gemm_x3_kernel's 32), 64 (the bf16 MFMA kernel)
@@ -1915,7 +1923,8 @@ int gemm_grad_weight(const float* dP, int64_t ldp, const float* X, int64_t ldx, 
   g.C = partial; g.ldc = N;
   g.M = M; g.N = N; g.K = K;
   g.k_chunk = k_chunk; g.c_split_stride = (int64_t)M * N;
-  int rc = launch_gemm(g, x_bf16 ? kGemmGradWeightBf16 : kGemmGradWeight, splits, stream);
+  int rc = launch_gemm(g, x_bf16 ? kGemmGradWeightBf16 : kGemmGradWeight, splits, stream,
+                       beside && !x_bf16 && K > kBesideRows ? kTile64Beside : kTile64Below);
   if (rc != kOk) return rc;
   const int64_t total = (int64_t)M * N;
   JN_REQUIRE((total + 63) / 64 < (1LL << 31), kUnsupported, "weight gradient too large");

@@ -234,3 +234,35 @@ def test_three_term_products_are_the_same_on_both_tiles(dev):
 
     for a, b in zip(run(B), run(B - 1)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("rows,D,tile", [(20480, 256, 128), (16384, 256, 64), (20480, 128, 64)])
+def test_weight_gradient_tile_beside_the_input_gradient(dev, rows, D, tile):
+    """The fp32 weight gradient takes 128-wide tiles beside the input gradient (on the second stream) of more than
+    16,384 rows where they make 128 workgroups, 64-wide ones by itself, and the same bits either way."""
+    import jakal_net_native as jn
+    from torch.profiler import ProfilerActivity, profile
+
+    g = torch.Generator().manual_seed(rows + D)
+    N, r = 2048, 64
+    X, ps = (torch.randn(*s, generator=g).to(dev).requires_grad_(True) for s in ((rows // N, N, D), (rows // N, N)))
+    U, V = (torch.randn(r, D, generator=g).to(dev).requires_grad_(True) for _ in range(2))
+    w, gv = torch.ones(r, device=dev), torch.randn(rows // N, N, D, generator=g).to(dev)
+
+    def step():
+        out = jn.propagation_window("low_rank_bilinear", w, None, V, None, U, None, "softsign", X, ps, X, 31, N, N)
+        return torch.autograd.grad(out[1], [X, U, V], gv)
+
+    grads = []
+    try:
+        for side, want in ((True, tile), (False, 64)):
+            jn.set_side_streams(side)
+            step()
+            with profile(activities=[ProfilerActivity.CUDA]) as prof:
+                grads.append(step())
+                torch.cuda.synchronize()
+            names = [e.key for e in prof.key_averages() if "gemm_x3_kernel<false, false, 2," in e.key]
+            assert len(names) == 1 and all(f", {want}>" in n for n in names), names
+    finally:
+        jn.set_side_streams(True)
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
