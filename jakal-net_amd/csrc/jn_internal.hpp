@@ -58,7 +58,8 @@ constexpr int kSelectSplitF16Wave = 2;
 constexpr int kSelectSplitF16Coop4 = 4;
 // Split fp16 on the key-split per-wave kernel whenever k <= 32 (tests); mode 0
 // picks it with >= 192 keys on grids below 256 workgroups of the per-wave kernel
-// for k <= 16; for k <= 32 below 129 with >= 2048 keys, below 65 with >= 384.
+// for k <= 16; for k <= 32 below 129 with >= 2048 keys, below 65 with >= 384 (several
+// heads: jn_select.hip's kSelKspHeadKeys).
 constexpr int kSelectSplitF16KeySplit = 5;
 // Split fp16 on the register kernels only: mode 0 as it was before the
 // small-key select (tests and A/B timing).

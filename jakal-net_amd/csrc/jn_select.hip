@@ -1310,6 +1310,15 @@ constexpr int64_t kSelKspMaxBlocks = 256;
 constexpr int64_t kSelKspMaxBlocks32 = 129, kSelKspMaxBlocks32Few = 65;
 constexpr int kSelKspMinKeys = 4 * kSelChunk;
 constexpr int kSelKspMinKeys32 = 384, kSelKspKeys32 = 2048;
+// Several heads fold each tile into a running maximum, a longer step per chunk:
+// up to 64 workgroups of 64 rows always (2 heads of 32, 1100 keys, k = 16: 43 us
+// against 71), up to 128 where the keys are enough for it (kSelKspHeadKeys, by
+// K-steps and list length: 2 K-steps, k = 16 126 workgroups 51 against 71, 160 99
+// against 98 over 2048 keys; 3 K-steps, k = 16 126 89 against 86 over 1100, 115
+// against 126 over 2048; 4, k = 20 128 150 against 153 over 2048, 212 against 265
+// over 4096; 3, k = 32 136 against 127 over 2048).
+constexpr int kSelKspHeadKeys[2][2] = {{0, 2048}, {2048, 4096}};  // [K-steps > 2][k > 16]
+constexpr int64_t kSelKspHeadBlocks = 64, kSelKspHeadMaxBlocks = 128;
 
 namespace {
 std::atomic<int> g_select_mode{kSelectSplitF16};
@@ -1418,9 +1427,10 @@ int launch_topk_select(const SelectArgs& a_in, hipStream_t stream) {
     a.split_exp = s.kexp;
     const bool coop4_wide = RP > 32 && !a.bf16 && (a.k <= 32 || a.Nk >= kSelCoop4WideKeys);
     const int64_t coop4_min = coop4_wide ? kSelCoop4MinBlocksWide : kSelCoop4MinBlocks;
-    const int64_t ksp_max = a.k <= 16             ? kSelKspMaxBlocks
-                            : a.Nk >= kSelKspKeys32 ? kSelKspMaxBlocks32
-                                                    : kSelKspMaxBlocks32Few;
+    int64_t ksp_max = a.k <= 16               ? kSelKspMaxBlocks
+                      : a.Nk >= kSelKspKeys32 ? kSelKspMaxBlocks32
+                                              : kSelKspMaxBlocks32Few;
+    if (mh) ksp_max = 1 + (a.Nk >= kSelKspHeadKeys[RP > 64][a.k > 16] ? kSelKspHeadMaxBlocks : kSelKspHeadBlocks);
     const int ksp_keys = a.k <= 16 ? kSelKspMinKeys : kSelKspMinKeys32;
     const bool coop4 = !mh && RP <= 64 &&
                        (mode == kSelectSplitF16Coop4 || (mode == kSelectSplitF16 && blocks >= coop4_min));

@@ -351,3 +351,34 @@ def test_kernel_of_a_select(dev, blocks, Nk, r, k, form):
     names = [e.key for e in prof.key_averages() if "lowrank_topk_select_kernel<" in e.key]
     forms = {int(re.search(r"<(.*?)>", n).group(1).split(",")[4]) for n in names}
     assert forms == {form}, names
+
+
+@pytest.mark.parametrize("blocks,N,heads,r,k,form", [
+    (64, 512, 4, 16, 32, -1), (72, 1536, 4, 16, 16, 0), (96, 1536, 2, 24, 16, -1), (128, 2048, 3, 24, 16, -1),
+    (160, 2048, 3, 24, 16, 0), (144, 1536, 2, 24, 8, 0), (128, 2048, 2, 24, 32, -1), (96, 1536, 2, 24, 17, 0),
+    (96, 2048, 3, 24, 20, 0), (128, 4096, 3, 24, 20, -1),
+])
+def test_kernel_of_a_multihead_select(dev, blocks, N, heads, r, k, form):
+    """The same for several heads, which leave the key-split form at fewer workgroups."""
+    import re
+
+    import jakal_net_native as jn
+    from torch.profiler import ProfilerActivity, profile
+
+    B, D = blocks * 64 // N, 16
+    X, ps = torch.randn(B, N, D, device=dev), torch.randn(B, N, device=dev)
+    U, V = (torch.randn(heads, r, D, device=dev) for _ in range(2))
+    w = torch.ones(heads, r, device=dev)
+
+    def call():
+        with torch.no_grad():
+            jn.propagation_topk("multihead_max_low_rank_bilinear", w, None, V, None, U, None, "softsign", X, ps, X, k,
+                                N, N)
+        torch.cuda.synchronize()
+
+    call()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        call()
+    names = [e.key for e in prof.key_averages() if "lowrank_topk_select_kernel<" in e.key]
+    forms = {int(re.search(r"<(.*?)>", n).group(1).split(",")[4]) for n in names}
+    assert forms == {form}, names
