@@ -943,15 +943,33 @@ __global__ __launch_bounds__(256, 4) void gemm_f32_fast_kernel(GemmArgs g, int t
 // buffer resources: a vector outside its operand reads as zeros.
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
 constexpr int kBfT = 128;           // tile M and N
-// Grids of fewer 128-wide tiles than CUs take 64-wide ones (2 x 2 waves of 32 x
-// 32, also for gemm_x3_kernel): four times the workgroups, every element's K
-// chain as before, so the same results bit for bit.  Measured on both tiles,
-// 128 and 64 wide: bf16 route aggregates of 64 and 256 tiles 29.5 against 19.7
-// us (mean), of 32 tiles over K = 4096 147 against 71; fp32 dense aggregate and
-// value gradient of 32 tiles 75 and 87 against 39 and 50; input gradients of 128
-// tiles 20 against 14.  From 256 tiles on the wide ones win where K is long
-// (route aggregate 79 against 86, weight gradient 20.1 against 22.7).
+// Grids of few 128-wide tiles take 64-wide ones (2 x 2 waves of 32 x 32, also for
+// gemm_x3_kernel): four times the workgroups, every element's K chain as before,
+// so the same results bit for bit.  The line is one tile per CU, lower where the
+// wide tiles' longer runs of MFMAs count for more before that (tile64_line, by
+// use).  Measured on both tiles, 64 and 128 wide:
+//   fp32 value gradient, K = 1024: 64 tiles 53 / 88 us, 128 69 / 89, 160 96 / 90,
+//     240 124 / 92 (K = 3648: 116 tiles 229 / 294, 145 310 / 295, 232 407 / 303)
+//   fp32 aggregate, K = 1024: 64 tiles 41 / 76, 192 75 / 79, 224 94 / 81
+//   fp32 input gradient, K = 128: 128 tiles 14 / 18, 192 17 / 19, 208 29 / 28 (K =
+//     256), 240 21 / 19.5
+//   fp32 weight gradient: 128 tiles over 40,960 rows 44 / 58, 192 over 131,072
+//     184 / 171
+//   bf16 value gradient, K = 3648: 116 tiles 78 / 129, 174 110 / 129, 232 144 / 131;
+//     bf16 aggregate 232 tiles 107 / 114; route aggregate, K = 4096: 128 tiles 80 /
+//     110, 240 145 / 138
 constexpr int64_t kTile64Below = 256;
+static int64_t tile64_line(int use) {
+  switch (use) {
+    case kGemmDenseValueGrad: return 129;
+    case kGemmGradWeight: return 192;
+    case kGemmDenseAggregate:
+    case kGemmGradInput:
+    case kGemmDenseValueGradBf16:
+    case kGemmRouteAggregateBf16: return 193;
+    default: return kTile64Below;
+  }
+}
 // A weight gradient beside the input gradient on another stream leaves it more of
 // the chip on wide tiles, from 16,384 rows on and if they make half a tile per CU:
 // training steps of 40,960 x 256 (rank 64, 128 tiles) 446 against 472 us, 65,536 x
@@ -1641,7 +1659,7 @@ static bool rows_form(const GemmArgs& g, int use, bool fast, RowsGemm& r) {
   return gemm_rows_fits(r);
 }
 
-int launch_gemm(const GemmArgs& g, GemmUse use, int splits, hipStream_t stream, int64_t tile64_below = kTile64Below) {
+int launch_gemm(const GemmArgs& g, GemmUse use, int splits, hipStream_t stream, int64_t tile64_max = kTile64Below) {
   JN_REQUIRE(g.M >= 0 && g.N >= 0 && g.K >= 0, kInvalidArgument, "negative GEMM extent");
   if (g.M == 0 || g.N == 0) return kOk;
   JN_REQUIRE(g.batch <= 1 || splits == 1, kInvalidArgument, "batched GEMM has no split-K");
@@ -1667,7 +1685,7 @@ int launch_gemm(const GemmArgs& g, GemmUse use, int splits, hipStream_t stream, 
   // the 128-wide MFMA tiles of this product, or 64-wide where those leave CUs
   // idle (or as forced: 32 x 32 tiles are not among them)
   const int64_t tiles128 = (int64_t)((g.M + kBfT - 1) / kBfT) * ((g.N + kBfT - 1) / kBfT) * zdim;
-  const int tile = forced ? (forced == kBfT ? kBfT : 64) : tiles128 < tile64_below ? 64 : kBfT;
+  const int tile = forced ? (forced == kBfT ? kBfT : 64) : tiles128 < std::min(tile64_line(use), tile64_max) ? 64 : kBfT;
   const int tm = (g.M + tile - 1) / tile, tn = (g.N + tile - 1) / tile;
   const int64_t tiles = (int64_t)tm * tn * zdim;
   auto at_tile = [&](auto launch) {

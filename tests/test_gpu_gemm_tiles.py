@@ -266,3 +266,39 @@ def test_weight_gradient_tile_beside_the_input_gradient(dev, rows, D, tile):
     finally:
         jn.set_side_streams(True)
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+@pytest.mark.parametrize("bf16,B,aggregate,value_grad", [
+    (False, 16, 64, 64), (False, 17, 64, 128), (False, 24, 64, 128), (False, 25, 128, 128),  # 8 wide tiles each
+    (True, 24, 64, 64), (True, 25, 64, 128), (True, 31, 64, 128), (True, 32, 128, 128),
+])
+def test_tile_of_a_dense_product(dev, bf16, B, aggregate, value_grad):
+    """Which tile the N x N products of a layer take on either side of their lines, by use."""
+    import re
+
+    import jakal_net_native as jn
+    from torch.profiler import ProfilerActivity, profile
+
+    N, D, r = 1024, 128, 8
+    dt = torch.bfloat16 if bf16 else torch.float32
+    X = torch.randn(B, N, D, device=dev).to(dt).requires_grad_(True)
+    ps, w = torch.randn(B, N, device=dev), torch.ones(r, device=dev)
+    U, V = (torch.randn(r, D, device=dev) for _ in range(2))
+
+    def step():
+        out = jn.propagation_dense("low_rank_bilinear", w, None, V, None, U, None, "signed_abs_softmax", X, ps, X, None,
+                                   N, N)
+        out[1].backward(torch.ones_like(out[1]))
+        torch.cuda.synchronize()
+
+    step()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        step()
+    tile = {}
+    for e in prof.key_averages():
+        m = re.search(r"gemm_(x3|bf16)_kernel<(.*?)>", e.key)
+        if m:
+            *_, use, t = m.group(2).split(",")
+            tile[int(use)] = int(t)
+    uses = (19, 20) if bf16 else (4, 6)
+    assert tuple(tile[u] for u in uses) == (aggregate, value_grad), tile
