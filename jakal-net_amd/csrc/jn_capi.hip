@@ -1727,7 +1727,11 @@ static int transition_topk_backward_impl(const float* sender_strength, const flo
   // 2. destination columns: grad of the destination projection and w partials
   rc = launch_csr_fill(ca, st);
   if (rc) return rc;
-  // the source side's projection grads (ready after the row pass) run beside them
+  // the source side's projection grads (ready after the row pass) run beside them;
+  // of many rows each side's weight gradient keeps wide tiles, which leave the
+  // other more of the chip (rank 128: 39 x 3300 rows of 256 to 1934 4372 -> 4216
+  // us a step, 64 x 1024 2459 -> 2347; 32 x 1024 of 192 1289 against 1310)
+  constexpr int kRouteBesideRows = 32768;
   hipStream_t ss = side ? side->stream : st;
   if (side) {
     rc = fork_to(side, st);
@@ -1735,7 +1739,7 @@ static int transition_topk_backward_impl(const float* sender_strength, const flo
   }
   if (grad_source_weight) {
     rc = gemm_grad_weight(s.dPs, r, src_val, src_dim, grad_source_weight, grad_source_weight, r, r, (int)src_dim,
-                          B * Ns, s.splitk2, ss, bf16);
+                          B * Ns, s.splitk2, ss, bf16, side && B * Ns > kRouteBesideRows);
     if (rc) return rc;
   }
   if (grad_src_val) {
@@ -1770,7 +1774,7 @@ static int transition_topk_backward_impl(const float* sender_strength, const flo
   // 3. destination-side projection weight and input grads
   if (grad_target_weight) {
     rc = gemm_grad_weight(s.dPt, r, dst_val, dst_dim, grad_target_weight, grad_target_weight, r, r, (int)dst_dim,
-                          B * Nd, s.splitk, st, bf16);
+                          B * Nd, s.splitk, st, bf16, side && B * Nd > kRouteBesideRows);
     if (rc) return rc;
   }
   if (grad_dst_val) {

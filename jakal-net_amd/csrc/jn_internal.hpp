@@ -186,7 +186,7 @@ enum GemmUse {
 int gemm_batched(const BatchedGemm& m, GemmUse use, hipStream_t stream);
 // Workgroup tile of every later GEMM launch: 0 = chosen per call, 64 or 128 = forced.
 void set_gemm_tile(int tile);
-// beside: the input gradient runs on another stream meanwhile.
+// beside: the input gradient (or a transition's other side) runs on another stream meanwhile.
 int gemm_grad_weight(const float* dP, int64_t ldp, const float* X, int64_t ldx, float* out0, float* out1, int m_split,
                      int M, int N, int K, float* partial, hipStream_t stream, bool x_bf16 = false, bool beside = false);
 

@@ -302,3 +302,36 @@ def test_tile_of_a_dense_product(dev, bf16, B, aggregate, value_grad):
             tile[int(use)] = int(t)
     uses = (19, 20) if bf16 else (4, 6)
     assert tuple(tile[u] for u in uses) == (aggregate, value_grad), tile
+
+
+@pytest.mark.parametrize("B,tile", [(32, 64), (33, 128)])
+def test_weight_gradient_tile_of_a_transition(dev, B, tile):
+    """A transition's weight gradients, of two sides on two streams, from 32,768 rows on; the same bits on one stream."""
+    import jakal_net_native as jn
+    from torch.profiler import ProfilerActivity, profile
+
+    g = torch.Generator().manual_seed(B)
+    N, D, r = 1024, 256, 128
+    rand = lambda *s: torch.randn(*s, generator=g).to(dev)  # noqa: E731
+    src, dst, rho, ps = rand(B, N, D), rand(B, N, D), rand(B, N), rand(B, N)
+    U, V = (rand(r, D).requires_grad_(True) for _ in range(2))
+    w, gv = torch.ones(r, device=dev) / r, rand(B, N, D)
+
+    def step():
+        out = jn.transition_pairwise_topk("low_rank_bilinear_route", U, None, V, None, w, None, None, None, None, None,
+                                          1.0, rho, src, dst, ps, src, 8, N, N)
+        return torch.autograd.grad(out[1], [U, V], gv)
+
+    grads = []
+    try:
+        for side, want in ((True, tile), (False, 64)):
+            jn.set_side_streams(side)
+            step()
+            with profile(activities=[ProfilerActivity.CUDA]) as prof:
+                grads.append(step())
+                torch.cuda.synchronize()
+            names = [e.key for e in prof.key_averages() if "gemm_x3_kernel<false, false, 2," in e.key]
+            assert len(names) == 1 and f", {want}>" in names[0], names
+    finally:
+        jn.set_side_streams(True)
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
